@@ -12,7 +12,12 @@
 // KS = 7 terms, so the truncation (< RHO^7/8! = 1.9e-7 relative to the chunk
 // displacement; 1e-9 at the typical |M|_F h ~ 0.25) is at FP32 resolution; no
 // eigenvalue case analysis (real / complex / repeated) and no transcendental
-// calls are needed in 2D/3D.
+// calls are needed in 2D/3D.  Cayley-Hamilton reduces the series to D scalars
+// (flow_at): q(s) = q0 + sum_{i<D} al_i(s) M^i v0 and exp(s M) =
+// sum_{i<D} e_i(s) M^i, with al and e from one Horner recurrence in the
+// invariants of s M.  The position, the Jacobian, every facet's G and G' and
+// the gradient integral share those scalars, so a chunk keeps D vectors
+// instead of KS and a facet D + 1 coefficients instead of KS + 1.
 // 1D uses the closed form q(s) = q0 + s*phi1(a s)*v0 and the analytic hit time
 // s = (qb-q0)/v0 * log1p(r)/r, r = a (qb-q0)/v0.
 //
@@ -119,40 +124,126 @@ CPAB_HD __forceinline__ void affine_apply(const float (&M)[D][D], const float (&
     }
 }
 
-// G(s) and G'(s) of sum_k cf[k] s^k by simultaneous Horner.
-CPAB_HD __forceinline__ void horner2(const float (&cf)[KS + 1], float s, float& g, float& d) {
-    float gg = cf[KS], dd = 0.f;
-#pragma unroll
-    for (int k = KS - 1; k >= 0; --k) {
-        dd = fmaf(dd, s, gg);
-        gg = fmaf(gg, s, cf[k]);
+// Invariants of a cell's M: trace, (3D) second invariant, determinant.
+template <int D>
+struct Invariants {
+    float t, sg, d;
+};
+template <int D>
+CPAB_HD __forceinline__ Invariants<D> invariants(const float (&M)[D][D]) {
+    Invariants<D> v;
+    if constexpr (D == 2) {
+        v.t = M[0][0] + M[1][1];
+        v.sg = 0.f;
+        v.d = fmaf(M[0][0], M[1][1], -(M[0][1] * M[1][0]));
+    } else {
+        v.t = M[0][0] + M[1][1] + M[2][2];
+        const float c0 = fmaf(M[1][1], M[2][2], -(M[1][2] * M[2][1]));
+        const float c1 = fmaf(M[1][0], M[2][2], -(M[1][2] * M[2][0]));
+        const float c2 = fmaf(M[1][0], M[2][1], -(M[1][1] * M[2][0]));
+        v.sg = c0 + fmaf(M[0][0], M[2][2], -(M[0][2] * M[2][0])) + fmaf(M[0][0], M[1][1], -(M[0][1] * M[1][0]));
+        v.d = fmaf(M[0][0], c0, fmaf(-M[0][1], c1, M[0][2] * c2));
     }
-    g = gg;
-    d = dd;
+    return v;
 }
 
-CPAB_HD __forceinline__ float horner1(const float (&cf)[KS + 1], float s) {
-    float gg = cf[KS];
+// The flow's scalars at time s: displacement sum_i al[i] M^i v0 and
+// exp(s M) = sum_i e[i] M^i.  With N = s M, phi1(N) = sum_{k<KS} N^k/(k+1)! is
+// evaluated by Horner's rule in the powers of N below D, each product by N
+// reduced by the characteristic polynomial (2D: N^2 = t N - d; 3D: N^3 =
+// t N^2 - sg N + d); then al_i M^i = s phi1 and exp(N) = I + N phi1.
+template <int D>
+struct FlowAt {
+    float al[D], e[D];
+};
+template <int D>
+CPAB_HD __forceinline__ FlowAt<D> flow_at(const Invariants<D>& iv, float s) {
+    static_assert(KS == 7, "the Horner constants below are 1/(k+1)! for k < 7");
+    constexpr float C[KS] = {1.f, 1.f / 2, 1.f / 6, 1.f / 24, 1.f / 120, 1.f / 720, 1.f / 5040};
+    FlowAt<D> f;
+    const float tt = s * iv.t, s2 = s * s;
+    if constexpr (D == 2) {
+        const float dd = s2 * iv.d;
+        float a = C[6], b = C[5];  // a N + b
 #pragma unroll
-    for (int k = KS - 1; k >= 0; --k) gg = fmaf(gg, s, cf[k]);
-    return gg;
+        for (int k = 4; k >= 0; --k) {
+            const float an = fmaf(tt, a, b);
+            b = fmaf(-dd, a, C[k]);
+            a = an;
+        }
+        f.al[0] = s * b;
+        f.al[1] = s2 * a;
+        f.e[0] = fmaf(-dd, a, 1.f);
+        f.e[1] = s * fmaf(tt, a, b);
+    } else {
+        const float s3 = s2 * s;
+        const float ss = s2 * iv.sg, dd = s3 * iv.d;
+        float a = C[6], b = C[5], c = C[4];  // a N^2 + b N + c
+#pragma unroll
+        for (int k = 3; k >= 0; --k) {
+            const float an = fmaf(tt, a, b);
+            b = fmaf(-ss, a, c);
+            c = fmaf(dd, a, C[k]);
+            a = an;
+        }
+        f.al[0] = s * c;
+        f.al[1] = s2 * b;
+        f.al[2] = s3 * a;
+        f.e[0] = fmaf(dd, a, 1.f);
+        f.e[1] = s * fmaf(-ss, a, c);
+        f.e[2] = s2 * fmaf(tt, a, b);
+    }
+    return f;
 }
 
-// Root of G in [lo, hi] with G(lo) <= 0 < G(hi): Newton steps from the
-// regula-falsi point, safeguarded by bisection.  A lane stops after a Newton
+// G(s) = n.q(s) + e along one facet: g[0] = G(0), g[i + 1] = n.M^i v0.
+template <int D>
+struct FacetG {
+    float g[D + 1];
+};
+template <int D>
+CPAB_HD __forceinline__ float facet_g(const FacetG<D>& F, const FlowAt<D>& f) {
+    float r = F.g[0];
+#pragma unroll
+    for (int i = 0; i < D; ++i) r = fmaf(f.al[i], F.g[i + 1], r);
+    return r;
+}
+template <int D>
+CPAB_HD __forceinline__ float facet_dg(const FacetG<D>& F, const FlowAt<D>& f) {
+    float r = f.e[0] * F.g[1];
+#pragma unroll
+    for (int i = 1; i < D; ++i) r = fmaf(f.e[i], F.g[i + 1], r);
+    return r;
+}
+// G(s) and G'(s)
+template <int D>
+CPAB_HD __forceinline__ void facet_at(const FacetG<D>& F, const Invariants<D>& iv, float s, float& g, float& d) {
+    const FlowAt<D> f = flow_at<D>(iv, s);
+    g = facet_g<D>(F, f);
+    d = facet_dg<D>(F, f);
+}
+
+// Root of G in [lo, hi] with G(lo) <= 0 < G(hi): Newton steps from the root of
+// the quadratic model, safeguarded by bisection.  A lane stops after a Newton
 // step below 1e-5 of its bracket (quadratic convergence: the error is then
 // ~1e-10) or after 6 steps; its result depends on its own iterates only, not
 // on the other lanes of the wave.
-CPAB_HD __forceinline__ float solve_bracket(const float (&cf)[KS + 1], float lo, float hi, float glo, float ghi) {
-    float s = lo + (hi - lo) * (glo * fast_rcp(glo - ghi));
+template <int D>
+CPAB_HD __forceinline__ float solve_bracket(const FacetG<D>& F, const Invariants<D>& iv, float lo, float hi, float glo,
+                                            float ghi) {
+    // the root of G's quadratic model at 0 (relative error ~ (|M| h)^2 / 6; two
+    // evaluations then usually end the iteration, four from the regula-falsi
+    // point), where it falls inside the bracket
+    float s = -2.f * F.g[0] * fast_rcp(F.g[1] + fast_sqrt(fmaf(F.g[1], F.g[1], -2.f * (F.g[2] * F.g[0]))));
+    if (!(s >= lo && s <= hi)) s = lo + (hi - lo) * (glo * fast_rcp(glo - ghi));
     if (!(s >= lo && s <= hi)) s = 0.5f * (lo + hi);
     const float tol = 1e-5f * (hi - lo);
     bool fin = false;
-#pragma unroll
+#pragma unroll 1
     for (int it = 0; it < 6; ++it) {
         if (!fin) {
             float g, d;
-            horner2(cf, s, g, d);
+            facet_at<D>(F, iv, s, g, d);
             if (g > 0.f) hi = s; else lo = s;
             float sn = s - g * fast_rcp(d);
             const bool newton = sn >= lo && sn <= hi;
@@ -172,14 +263,16 @@ CPAB_HD __forceinline__ float solve_bracket(const float (&cf)[KS + 1], float lo,
 // Zero of G' in [lo, hi] given G'(lo) and G'(hi) of opposite signs:
 // Illinois-modified secant steps inside the shrinking bracket; returns the
 // bracket end with the smaller |G'|.
-CPAB_HD __forceinline__ float crit_point(const float (&cf)[KS + 1], float lo, float hi, float dlo, float dhi) {
+template <int D>
+CPAB_HD __forceinline__ float crit_point(const FacetG<D>& F, const Invariants<D>& iv, float lo, float hi, float dlo,
+                                         float dhi) {
     int side = 0;
 #pragma unroll 1
     for (int it = 0; it < 4; ++it) {
         const float m = (lo * dhi - hi * dlo) * fast_rcp(dhi - dlo);
         if (!(m > lo && m < hi)) break;
         float gm, dm;
-        horner2(cf, m, gm, dm);
+        facet_at<D>(F, iv, m, gm, dm);
         if ((dm > 0.f) == (dlo > 0.f)) {
             lo = m;
             dlo = dm;
@@ -202,7 +295,7 @@ struct Bracket {
 };
 
 // Isolates the first time in [0, h] at which the trajectory leaves through the
-// facet with coefficients cf (G(s) = sum_k cf[k] s^k, G <= 0 inside).
+// facet F (G <= 0 inside).
 //  * A start on the facet (G(0) >= -tol0, taken as G(0) = 0) moving out
 //    exits at 0 when allow_start: G'(0) > tol1, or 0 <= G'(0) <= tol1 (an
 //    outward speed within the rounding of the field) with G''(0) > 0.
@@ -215,23 +308,24 @@ struct Bracket {
 //  * Any other start on the facet (G'(0) >= 0 with the start exit
 //    disallowed) is ignored until G has gone negative.
 //  * Between two negative samples a local maximum above 0 is a crossing.
-CPAB_HD __forceinline__ void first_bracket(const float (&cf)[KS + 1], float h, float tol0, float tol1, bool allow_start,
-                                           Bracket& br) {
+template <int D>
+CPAB_HD __forceinline__ void first_bracket(const FacetG<D>& F, const Invariants<D>& iv, float h, float tol0, float tol1,
+                                           bool allow_start, Bracket& br) {
     br.idx = NSAMP + 1;
-    const bool on = cf[0] >= -tol0;
-    if (on && allow_start && (cf[1] > tol1 || (cf[1] >= 0.f && cf[2] > 0.f))) {
+    const bool on = F.g[0] >= -tol0;
+    if (on && allow_start && (F.g[1] > tol1 || (F.g[1] >= 0.f && F.g[2] > 0.f))) {
         br.idx = 0;
         br.lo = br.hi = 0.f;
         return;
     }
-    bool skip = on && !(cf[1] < 0.f);
+    bool skip = on && !(F.g[1] < 0.f);
     bool dip = on && !skip;
-    float ps = 0.f, pg = cf[0], pd = cf[1];
+    float ps = 0.f, pg = F.g[0], pd = F.g[1];
 #pragma unroll 1
     for (int i = 1; i <= NSAMP; ++i) {
         const float s = h * ((float)i * (1.0f / NSAMP));
         float g, d;
-        horner2(cf, s, g, d);
+        facet_at<D>(F, iv, s, g, d);
         // 0: nothing, 1: dip minimum (G comes back above 0), 2: graze maximum
         int crit = 0;
         if (skip) {
@@ -247,8 +341,8 @@ CPAB_HD __forceinline__ void first_bracket(const float (&cf)[KS + 1], float h, f
             if (pd > 0.f && d < 0.f) crit = 2;
         }
         if (crit) {
-            const float m = crit_point(cf, ps, s, pd, d);
-            const float gm = horner1(cf, m);
+            const float m = crit_point<D>(F, iv, ps, s, pd, d);
+            const float gm = facet_g<D>(F, flow_at<D>(iv, m));
             if (crit == 1 && gm < 0.f) {
                 br.idx = i; br.lo = m; br.hi = s; br.glo = gm; br.ghi = g;
                 return;
@@ -268,122 +362,44 @@ CPAB_HD __forceinline__ void first_bracket(const float (&cf)[KS + 1], float h, f
     }
 }
 
-// Series vectors W[k] = M^k v0 / (k+1)!, so q(s) = q0 + sum_k s^(k+1) W[k].
+// The chunk's vectors v[i] = M^i v0, i < D.
 template <int D>
-CPAB_HD __forceinline__ void series(const float (&M)[D][D], const float (&v0)[D], float (&W)[KS][D]) {
+CPAB_HD __forceinline__ void powers(const float (&M)[D][D], const float (&v0)[D], float (&v)[D][D]) {
 #pragma unroll
-    for (int a = 0; a < D; ++a) W[0][a] = v0[a];
+    for (int a = 0; a < D; ++a) v[0][a] = v0[a];
 #pragma unroll
-    for (int k = 1; k < KS; ++k) {
-        const float inv = 1.0f / (float)(k + 1);
+    for (int k = 1; k < D; ++k)
 #pragma unroll
         for (int r = 0; r < D; ++r) {
-            float acc = 0.f;
+            float acc = M[r][0] * v[k - 1][0];
 #pragma unroll
-            for (int a = 0; a < D; ++a) acc = fmaf(M[r][a], W[k - 1][a], acc);
-            W[k][r] = acc * inv;
+            for (int a = 1; a < D; ++a) acc = fmaf(M[r][a], v[k - 1][a], acc);
+            v[k][r] = acc;
         }
-    }
 }
 
+// Coefficients of facet f of cell c.  A start within tol0 of the facet is a
+// start on it: G(0) = 0 exactly, so the sign of G just after the start is that
+// of G'(0) (and, for a shallow dip into the cell, of the dip) rather than that
+// of the rounding in n.q + e.
 template <int D>
-CPAB_HD __forceinline__ void series_eval(const float (&q0)[D], const float (&W)[KS][D], float s, float (&q)[D]) {
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        float acc = W[KS - 1][a];
-#pragma unroll
-        for (int k = KS - 2; k >= 0; --k) acc = fmaf(acc, s, W[k][a]);
-        q[a] = fmaf(acc, s, q0[a]);
-    }
-}
-
-// E = exp(N), N = s M, by the Taylor series to N^KS with every power reduced
-// by Cayley-Hamilton to the span of {I, N} (2D: N^2 = tr N - det I) or
-// {I, N, N^2} (3D: N^3 = tr N^2 - sigma N + det I): scalar recurrences for the
-// coordinates of N^k, then one combination.
-template <int D>
-CPAB_HD __forceinline__ void exp_mat(const float (&M)[D][D], float s, float (&E)[D][D]) {
-    float N[D][D];
-#pragma unroll
-    for (int r = 0; r < D; ++r)
-#pragma unroll
-        for (int c = 0; c < D; ++c) N[r][c] = s * M[r][c];
-    if constexpr (D == 2) {
-        const float tr = N[0][0] + N[1][1];
-        const float det = fmaf(N[0][0], N[1][1], -N[0][1] * N[1][0]);
-        // N^k = a N + b I;  exp(N) = al N + be I
-        float a = 1.f, b = 0.f, al = 1.f, be = 1.f, fac = 1.f;
-#pragma unroll
-        for (int k = 2; k <= KS; ++k) {
-            const float an = fmaf(tr, a, b);
-            b = -det * a;
-            a = an;
-            fac *= 1.0f / (float)k;
-            al = fmaf(a, fac, al);
-            be = fmaf(b, fac, be);
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) E[r][c] = fmaf(al, N[r][c], (r == c) ? be : 0.f);
-    } else {
-        float N2[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                float acc = 0.f;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) acc = fmaf(N[r][k], N[k][c], acc);
-                N2[r][c] = acc;
-            }
-        const float tr = N[0][0] + N[1][1] + N[2][2];
-        const float sg = fmaf(N[0][0], N[1][1], -N[0][1] * N[1][0]) + fmaf(N[0][0], N[2][2], -N[0][2] * N[2][0]) +
-                         fmaf(N[1][1], N[2][2], -N[1][2] * N[2][1]);
-        const float det = N[0][0] * fmaf(N[1][1], N[2][2], -N[1][2] * N[2][1]) -
-                          N[0][1] * fmaf(N[1][0], N[2][2], -N[1][2] * N[2][0]) +
-                          N[0][2] * fmaf(N[1][0], N[2][1], -N[1][1] * N[2][0]);
-        // N^k = a N^2 + b N + c I, from k = 2;  exp(N) = ga N^2 + be N + al I
-        float a = 1.f, b = 0.f, c = 0.f, ga = 0.5f, be = 1.f, al = 1.f, fac = 0.5f;
-#pragma unroll
-        for (int k = 3; k <= KS; ++k) {
-            const float an = fmaf(tr, a, b);
-            const float bn = fmaf(-sg, a, c);
-            c = det * a;
-            a = an;
-            b = bn;
-            fac *= 1.0f / (float)k;
-            ga = fmaf(a, fac, ga);
-            be = fmaf(b, fac, be);
-            al = fmaf(c, fac, al);
-        }
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int cc = 0; cc < 3; ++cc) E[r][cc] = fmaf(ga, N2[r][cc], fmaf(be, N[r][cc], (r == cc) ? al : 0.f));
-    }
-}
-
-// Series coefficients of G(s) = n.q(s) + e for facet f of cell c.  A start
-// within tol0 of the facet is a start on it: G(0) = 0 exactly, so the sign of
-// G just after the start is that of G'(0) (and, for a shallow dip into the
-// cell, of the dip) rather than that of the rounding in n.q + e.
-template <int D>
-CPAB_HD __forceinline__ void facet_coeffs(const CellTable<D>& tab, int c, int f, const float (&q)[D],
-                                          const float (&W)[KS][D], float tol0, float (&cf)[KS + 1]) {
+CPAB_HD __forceinline__ FacetG<D> facet_coeffs(const CellTable<D>& tab, int c, int f, const float (&q)[D],
+                                               const float (&v)[D][D], float tol0) {
     const float4 P = tab.pl[c * NF + f];
     const float n[3] = {P.x, P.y, P.z};
+    FacetG<D> F;
     float g0 = P.w;
 #pragma unroll
     for (int a = 0; a < D; ++a) g0 = fmaf(n[a], q[a], g0);
-    cf[0] = (g0 >= -tol0) ? 0.f : g0;
+    F.g[0] = (g0 >= -tol0) ? 0.f : g0;
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-        float acc = 0.f;
+    for (int k = 0; k < D; ++k) {
+        float acc = n[0] * v[k][0];
 #pragma unroll
-        for (int a = 0; a < D; ++a) acc = fmaf(n[a], W[k][a], acc);
-        cf[k + 1] = acc;
+        for (int a = 1; a < D; ++a) acc = fmaf(n[a], v[k][a], acc);
+        F.g[k + 1] = acc;
     }
+    return F;
 }
 
 // What one chunk did; handed to the pass callbacks.
@@ -392,23 +408,31 @@ struct Chunk {
     float M[D][D];
     float b[D];
     float q0[D];
-    float W[KS][D];  // W[0] = v0
-    float h;         // time advanced
+    float v[D][D];     // v[i] = M^i v0
+    Invariants<D> iv;
+    FlowAt<D> f;       // the flow's scalars at h
+    float h;           // time advanced
     int cell;
-    int facet;       // crossed facet (-1: none)
-    int next;        // cell entered (== cell if no crossing)
-    float q1[D];     // end point
+    int facet;         // crossed facet (-1: none)
+    int next;          // cell entered (== cell if no crossing)
+    float q1[D];       // end point
 };
 
 // End of a chunk of duration step that crosses facet bf (-1: none): end point,
-// chunk record and the point's state (ch.M, ch.b and ch.W are set).
+// chunk record and the point's state (ch.M, ch.b, ch.v and ch.f are set).
 template <int D>
 CPAB_HD __forceinline__ void finish_chunk(PointState<D>& st, const CellTable<D>& tab, float step, int bf,
                                           Chunk<D>& ch) {
     const int c = st.c;
 #pragma unroll
     for (int a = 0; a < D; ++a) ch.q0[a] = st.q[a];
-    series_eval<D>(ch.q0, ch.W, step, ch.q1);
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        float acc = ch.f.al[D - 1] * ch.v[D - 1][a];
+#pragma unroll
+        for (int k = D - 2; k >= 0; --k) acc = fmaf(ch.f.al[k], ch.v[k][a], acc);
+        ch.q1[a] = ch.q0[a] + acc;
+    }
     ch.h = step;
     ch.cell = c;
     ch.facet = bf;
@@ -491,6 +515,20 @@ CPAB_HD __forceinline__ void logged_chunk(const ChunkLog& lg, int k, float& h, i
 
 // ---------------------------------------------------------------------------
 // one chunk of integration, D = 2, 3
+//
+// VALU issue bounds it (89% of the nominal rate in the plain 2D grid
+// transform), so what counts is instructions per wave and chunk, and a branch
+// costs its whole body whenever one of 64 lanes takes it.  Hence the shared
+// scalars of flow_at instead of a series vector and a polynomial per facet, one
+// straight cull for all facets, then a loop over each lane's own remaining
+// facet (0.5 trips per chunk on [4, 4] images) instead of four branches, and a
+// root search that starts from the quadratic model (1.0 Newton steps per chunk
+// and wave instead of 2-3) and samples only where neither G'' nor G' has a
+// certified sign (2% of a wave's chunks).  [4, 4], 64 x 256^2 points,
+// us per launch before / after: grid transform 88 / 67, its recomputing
+// backward 208 / 152; fused with 3 channels and 256 thetas: forward 491 / 459,
+// backward 790 / 732; [3, 3, 3], 16 x 64^3: forward 192 / 167, backward
+// 293 / 260.
 // ---------------------------------------------------------------------------
 template <int D>
 CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab, float tol0, Chunk<D>& ch) {
@@ -498,12 +536,49 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
     load_affine<D>(tab, c, ch.M, ch.b);
     float v0[D];
     affine_apply<D>(ch.M, ch.b, st.q, v0);
-    float h = fminf(st.T, RHO * tab.inv_n[c]);
-    series<D>(ch.M, v0, ch.W);
+    const float h = fminf(st.T, RHO * tab.inv_n[c]);
+    powers<D>(ch.M, v0, ch.v);
+    ch.iv = invariants<D>(ch.M);
+    ch.f = flow_at<D>(ch.iv, h);
     float vn2 = 0.f;
 #pragma unroll
     for (int a = 0; a < D; ++a) vn2 = fmaf(v0[a], v0[a], vn2);
     const float vn = fast_sqrt(vn2);
+    // Bounds on the chunk (|n| = 1, |M| <= |M|_F, |M|_F h <= RHO, |cf_k| <=
+    // |M|^(k-1) |v0| / k!):  the terms of G from s^3 on sum to at most
+    // K3 s^3, K3 = |M|_F^2 |v0| e^RHO / 6, their derivative to 3 K3 s^2, and
+    // |G''(s) - 2 cf2 - 6 cf3 s| <= K4 = |M|_F^3 |v0| h^2 e^RHO / 2.
+    const float nrm = fast_rcp(tab.inv_n[c]);  // |M|_F (the bounds below carry margin for its last bit)
+    const float mh = h * nrm;
+    const float K = GROW * vn * nrm;
+    const float K4 = 0.5f * K * mh * mh;
+    const float K3 = K * nrm * (1.0f / 6.0f);
+
+    // phase 1: cull, the same straight code for every facet slot (a wave runs
+    // it once; a branch per facet would run nearly every body of a wave with
+    // most lanes off)
+    const float hK3 = h * h * K3, hh = 0.5f * h;
+    unsigned live = 0u;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        const float4 P = tab.pl[c * NF + f];
+        const float n[3] = {P.x, P.y, P.z};
+        float g0 = P.w, g1 = n[0] * v0[0], g2 = n[0] * ch.v[1][0];
+#pragma unroll
+        for (int a = 0; a < D; ++a) g0 = fmaf(n[a], st.q[a], g0);
+#pragma unroll
+        for (int a = 1; a < D; ++a) {
+            g1 = fmaf(n[a], v0[a], g1);
+            g2 = fmaf(n[a], ch.v[1][a], g2);
+        }
+        // G(s) <= g0 + g1 s + max(cf2, 0) s^2 + K3 s^3 on [0, h] (cf2 = g2 / 2),
+        // a convex bound (its s^2 and s^3 coefficients are >= 0), so no
+        // crossing when it is below 0 at h; a start on the facet counts as
+        // G(0) = 0, and a convex bound that is 0 at 0 and below 0 at h is
+        // below 0 in between
+        const bool culled = fmaf(h, fmaf(hh, fmaxf(g2, 0.f), hK3) + g1, g0 >= -tol0 ? 0.f : g0) < 0.f;
+        live |= culled || tab.nb[c * NF + f] < 0 ? 0u : 1u << f;
+    }
     // Tangential band for an outward normal speed G'(0): the neighbouring
     // cells' FP32 fields agree on a shared facet only up to the rounding of
     // M q + b, whose terms can be much larger than |v0| where they cancel, so
@@ -525,86 +600,63 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
     // crosses no facet in this chunk (otherwise the noise could carry it
     // back and forth across a facet through the fixed point, a hop per
     // chunk, until the chunk budget ran out).
-    const bool still = vn <= tol1;
-    // Bounds on the chunk (|n| = 1, |M| <= |M|_F, |M|_F h <= RHO, |cf_k| <=
-    // |M|^(k-1) |v0| / k!):  the terms of G from s^3 on sum to at most
-    // K3 s^3, K3 = |M|_F^2 |v0| e^RHO / 6, their derivative to 3 K3 s^2, and
-    // |G''(s) - 2 cf2 - 6 cf3 s| <= K4 = |M|_F^3 |v0| h^2 e^RHO / 2.
-    const float nrm = fast_rcp(tab.inv_n[c]);  // |M|_F (the bounds below carry margin for its last bit)
-    const float mh = h * nrm;
-    const float K = GROW * vn * nrm;
-    const float K4 = 0.5f * K * mh * mh;
-    const float K3 = K * nrm * (1.0f / 6.0f);
-
-    // phase 1: classify every facet.  A facet whose first crossing lies in a
-    // bracket with a unique root becomes a candidate; starts on a facet, and
-    // facets whose curvature sign is not certified, take the sampling path.
-    int start_f = -1;
-    unsigned cand = 0u, slow = 0u;
-    // bracket of each candidate facet (set only where cand has its bit)
-    float clo[NF], chi[NF], cglo[NF], cghi[NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const int nbf = tab.nb[c * NF + f];
-        if (nbf < 0 || still) continue;
-        const float4 P = tab.pl[c * NF + f];
-        const float n[3] = {P.x, P.y, P.z};
-        float g0 = P.w, g1 = 0.f, g2 = 0.f;
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            g0 = fmaf(n[a], st.q[a], g0);
-            g1 = fmaf(n[a], v0[a], g1);
-        }
-#pragma unroll
-        for (int a = 0; a < D; ++a) g2 = fmaf(n[a], ch.W[1][a], g2);
-        const bool on = g0 >= -tol0;
-        // G(s) <= g0 + g1 s + max(cf2, 0) s^2 + K3 s^3 on [0, h], a convex bound
-        // (its s^2 and s^3 coefficients are >= 0), so no crossing when it is
-        // below 0 at h
-        const float c2p = fmaxf(g2, 0.f);
-        if (!on && fmaf(h, fmaf(h, fmaf(h, K3, c2p), g1), g0) < 0.f) continue;
-        // start on the facet moving inwards with G' <= g1 + 2 max(cf2, 0) s +
-        // 3 K3 s^2 < 0 on all of [0, h]: no return
-        if (on && g1 < -tol1 && fmaf(h, fmaf(h, 3.f * K3, 2.f * c2p), g1) < 0.f) continue;
+    if (vn <= tol1) live = 0u;
+    // phase 2: classify the facets left, one of each lane at a time.  A facet
+    // whose first crossing lies in [0, h] with a unique root becomes a
+    // candidate (cand); the best so far is the one with the earliest
+    // regula-falsi estimate.  Starts on a facet, and facets whose curvature
+    // sign is not certified, take the sampling path (slow).
+    int start_f = -1, bf = -1;
+    unsigned cand = 0u, slow = 0u, sampled = 0u;
+    float est = INFINITY, lo = 0.f, hi = 0.f, glo = 0.f, ghi = 0.f;
+#pragma unroll 1
+    while (live) {
+        const int f = __builtin_ctz(live);
+        live &= live - 1u;
+        const FacetG<D> F = facet_coeffs<D>(tab, c, f, st.q, ch.v, tol0);
+        const bool on = F.g[0] >= -tol0;
+        // G''(s) = 2 cf2 + 6 cf3 s + R(s), |R| <= K4, 6 cf3 = n.M^2 v0: the sign
+        // of G'' is certified when the linear part keeps one sign with margin K4
+        float g3;
+        if constexpr (D == 2) g3 = fmaf(ch.iv.t, F.g[2], -(ch.iv.d * F.g[1]));
+        else g3 = F.g[3];
+        const float l0 = F.g[2], l1 = fmaf(g3, h, l0);
+        const bool bent = fminf(l0, l1) > K4 || fmaxf(l0, l1) < -K4;
+        const float gh = facet_g<D>(F, ch.f);
         if (on) {
-            const bool allow_start = !(st.zero_hops > 0 && nbf == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
-            if (allow_start && (g1 > tol1 || (g1 >= 0.f && g2 > 0.f))) {
+            const bool allow_start =
+                !(st.zero_hops > 0 && tab.nb[c * NF + f] == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
+            if (allow_start && (F.g[1] > tol1 || (F.g[1] >= 0.f && F.g[2] > 0.f))) {
                 if (start_f < 0) start_f = f;
-            } else {
+            } else if (!(F.g[1] < -tol1 && bent && gh <= 0.f)) {
+                // (a clear start inwards that ends inside has no crossing in
+                // between when G is convex or concave on the chunk)
                 slow |= 1u << f;
             }
             continue;
         }
-        float cf[KS + 1];
-        cf[0] = g0;
-        cf[1] = g1;
-        cf[2] = g2;
-#pragma unroll
-        for (int k = 2; k < KS; ++k) {
-            float acc = 0.f;
-#pragma unroll
-            for (int a = 0; a < D; ++a) acc = fmaf(n[a], ch.W[k][a], acc);
-            cf[k + 1] = acc;
-        }
-        // G''(s) = 2 cf2 + 6 cf3 s + R(s), |R| <= K4: the sign of G'' is
-        // certified when the linear part keeps one sign with margin K4
-        const float l0 = 2.f * g2, l1 = fmaf(6.f * cf[3], h, l0);
-        if (!((l0 > K4 && l1 > K4) || (l0 < -K4 && l1 < -K4))) {
+        // Likewise G' = g1 + g2 s + R, |R| <= 3 K3 s^2, for a G that is too
+        // straight for its curvature to have a certified sign.
+        const float e1 = fmaf(l0, h, F.g[1]), r1 = 3.f * hK3;
+        const bool rising = fminf(F.g[1], e1) > r1, falling = fmaxf(F.g[1], e1) < -r1;
+        if (!(bent || rising || falling)) {
             slow |= 1u << f;
             continue;
         }
-        // G convex (g2 > 0) or concave (g2 < 0) on [0, h], G(0) < 0: a positive
-        // G(h) means exactly one crossing; otherwise only a concave G rising
-        // and falling inside the chunk can cross (sampling path).
-        float gh, dh;
-        horner2(cf, h, gh, dh);
+        // G convex (g2 > 0), concave (g2 < 0) or monotonic on [0, h], G(0) < 0: a
+        // positive G(h) means exactly one crossing; otherwise only a concave G
+        // rising and falling inside the chunk can cross (sampling path).
         if (gh > 0.f) {
             cand |= 1u << f;
-            clo[f] = 0.f;
-            chi[f] = h;
-            cglo[f] = g0;
-            cghi[f] = gh;
-        } else if (g2 < 0.f && g1 > 0.f && dh < 0.f) {
+            const float e = h * (F.g[0] * fast_rcp(F.g[0] - gh));
+            if (e < est) {
+                est = e;
+                bf = f;
+                hi = h;
+                glo = F.g[0];
+                ghi = gh;
+            }
+        } else if (l0 < 0.f && F.g[1] > 0.f && !rising && facet_dg<D>(F, ch.f) < 0.f) {
             slow |= 1u << f;
         }
     }
@@ -614,71 +666,59 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
         while (slow) {
             const int f = __builtin_ctz(slow);
             slow &= slow - 1u;
-            float cf[KS + 1];
-            facet_coeffs<D>(tab, c, f, st.q, ch.W, tol0, cf);
+            const FacetG<D> F = facet_coeffs<D>(tab, c, f, st.q, ch.v, tol0);
             const int nbf = tab.nb[c * NF + f];
             const bool allow_start = !(st.zero_hops > 0 && nbf == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
             Bracket br;
-            first_bracket(cf, h, tol0, tol1, allow_start, br);
+            first_bracket<D>(F, ch.iv, h, tol0, tol1, allow_start, br);
             if (br.idx >= 1 && br.idx <= NSAMP) {
                 cand |= 1u << f;
-#pragma unroll
-                for (int k = 0; k < NF; ++k)
-                    if (k == f) {
-                        clo[k] = br.lo;
-                        chi[k] = br.hi;
-                        cglo[k] = br.glo;
-                        cghi[k] = br.ghi;
-                    }
+                sampled |= 1u << f;
+                const float e = fmaf(br.hi - br.lo, br.glo * fast_rcp(br.glo - br.ghi), br.lo);
+                if (e < est) {
+                    est = e;
+                    bf = f;
+                    lo = br.lo;
+                    hi = br.hi;
+                    glo = br.glo;
+                    ghi = br.ghi;
+                }
             }
         }
     }
-    // phase 2: solve the candidate with the earliest regula-falsi estimate, then
-    // any other candidate that is still positive at (or ends before) that root
+    // phase 3: solve the candidate with the earliest estimate, then any other
+    // candidate that is still positive at (or ends before) that root
     float best = h;
-    int bf = -1;
     if (start_f >= 0) {
         best = 0.f;
         bf = start_f;
-    } else if (cand) {
-        float est = INFINITY, lo = 0.f, hi = 0.f, glo = 0.f, ghi = 0.f;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            if (!((cand >> f) & 1u)) continue;
-            const float e = fmaf(chi[f] - clo[f], cglo[f] * fast_rcp(cglo[f] - cghi[f]), clo[f]);
-            if (e < est) {
-                est = e;
-                bf = f;
-                lo = clo[f];
-                hi = chi[f];
-                glo = cglo[f];
-                ghi = cghi[f];
-            }
-        }
-        float cf[KS + 1];
-        facet_coeffs<D>(tab, c, bf, st.q, ch.W, tol0, cf);
-        best = solve_bracket(cf, lo, hi, glo, ghi);
+    } else if (bf >= 0) {
+        best = solve_bracket<D>(facet_coeffs<D>(tab, c, bf, st.q, ch.v, tol0), ch.iv, lo, hi, glo, ghi);
         unsigned others = cand & ~(1u << bf);
 #pragma unroll 1
         while (others) {
             const int f = __builtin_ctz(others);
             others &= others - 1u;
-#pragma unroll
-            for (int k = 0; k < NF; ++k)
-                if (k == f) {
-                    lo = clo[k];
-                    hi = chi[k];
-                    glo = cglo[k];
-                    ghi = cghi[k];
-                }
-            if (!(lo < best)) continue;
-            facet_coeffs<D>(tab, c, f, st.q, ch.W, tol0, cf);
-            if (best < hi) {
-                hi = best;
-                ghi = horner1(cf, best);
+            const FacetG<D> F = facet_coeffs<D>(tab, c, f, st.q, ch.v, tol0);
+            // a certified candidate's bracket is [0, h]; a sampled one's is
+            // found again
+            lo = 0.f;
+            hi = h;
+            glo = F.g[0];
+            if ((sampled >> f) & 1u) {
+                const int nbf = tab.nb[c * NF + f];
+                const bool allow_start = !(st.zero_hops > 0 && nbf == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
+                Bracket br;
+                first_bracket<D>(F, ch.iv, h, tol0, tol1, allow_start, br);
+                lo = br.lo;
+                hi = br.hi;
+                glo = br.glo;
             }
+            if (!(lo < best)) continue;
+            if (best < hi) hi = best;
+            ghi = facet_g<D>(F, flow_at<D>(ch.iv, hi));
             if (ghi > 0.f) {
-                const float s2 = solve_bracket(cf, lo, hi, glo, ghi);
+                const float s2 = solve_bracket<D>(F, ch.iv, lo, hi, glo, ghi);
                 if (s2 < best) {
                     best = s2;
                     bf = f;
@@ -686,6 +726,7 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
             }
         }
     }
+    if (bf >= 0) ch.f = flow_at<D>(ch.iv, best);
     finish_chunk<D>(st, tab, best, bf, ch);
 }
 
@@ -698,7 +739,9 @@ CPAB_HD __forceinline__ void replay(PointState<D>& st, const CellTable<D>& tab, 
     load_affine<D>(tab, st.c, ch.M, ch.b);
     float v0[D];
     affine_apply<D>(ch.M, ch.b, st.q, v0);
-    series<D>(ch.M, v0, ch.W);
+    powers<D>(ch.M, v0, ch.v);
+    ch.iv = invariants<D>(ch.M);
+    ch.f = flow_at<D>(ch.iv, h);
     finish_chunk<D>(st, tab, h, bf, ch);
 }
 
@@ -910,6 +953,38 @@ CPAB_HD __forceinline__ void saltation_adj(const CellTable<D>& tab, const Chunk<
     for (int a = 0; a < D; ++a) mu[a] = fmaf(-n[a], f, mu[a]);
 }
 
+// J <- exp(h M) J = sum_i e_i M^i J
+template <int D>
+CPAB_HD __forceinline__ void carry_jacobian(const Chunk<D>& ch, float (&J)[D][D]) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+        float w[D], acc[D];
+#pragma unroll
+        for (int r = 0; r < D; ++r) {
+            w[r] = J[r][j];
+            acc[r] = ch.f.e[0] * w[r];
+        }
+#pragma unroll
+        for (int k = 1; k < D; ++k) {
+            float m[D];
+#pragma unroll
+            for (int r = 0; r < D; ++r) {
+                float t = ch.M[r][0] * w[0];
+#pragma unroll
+                for (int a = 1; a < D; ++a) t = fmaf(ch.M[r][a], w[a], t);
+                m[r] = t;
+            }
+#pragma unroll
+            for (int r = 0; r < D; ++r) {
+                w[r] = m[r];
+                acc[r] = fmaf(ch.f.e[k], m[r], acc[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < D; ++r) J[r][j] = acc[r];
+    }
+}
+
 template <int D>
 CPAB_HD __forceinline__ void init_point(PointState<D>& st, const float (&q)[D], int c0, float T) {
 #pragma unroll
@@ -946,21 +1021,7 @@ CPAB_HD __forceinline__ void step_point(PointState<D>& st, const CellTable<D>& t
         Chunk<D> ch;
         advance<D>(st, tab, tol0, ch);
         if constexpr (WITHJ) {
-            float E[D][D], Jn[D][D];
-            exp_mat<D>(ch.M, ch.h, E);
-#pragma unroll
-            for (int r = 0; r < D; ++r)
-#pragma unroll
-                for (int j = 0; j < D; ++j) {
-                    float acc = 0.f;
-#pragma unroll
-                    for (int a = 0; a < D; ++a) acc = fmaf(E[r][a], J[a][j], acc);
-                    Jn[r][j] = acc;
-                }
-#pragma unroll
-            for (int r = 0; r < D; ++r)
-#pragma unroll
-                for (int j = 0; j < D; ++j) J[r][j] = Jn[r][j];
+            carry_jacobian<D>(ch, J);
             if (ch.facet >= 0) saltation_fwd<D>(tab, ch, J);
         }
         // logged last, when the chunk's temporaries are dead
@@ -1033,56 +1094,111 @@ CPAB_HD __forceinline__ void integrate(float (&q)[D], int c0, float T, const Cel
 // ---------------------------------------------------------------------------
 // pass 2: gradient contribution of one chunk
 // ---------------------------------------------------------------------------
+// K[i][j] = int_0^h e_i(-s) al_j(s) ds: with mu(s) = exp(-s M^T) mu0 =
+// sum_i e_i(-s) (M^T)^i mu0 and q(s) = q0 + sum_j al_j(s) M^j v0, the integral
+// of mu(s) (q(s) - q0)^T over the chunk is sum_ij K[i][j] (M^T)^i mu0 (M^j v0)^T.
+// Each K is h^(2+i+j) times a polynomial in the invariants of h M, the terms of
+// total degree below KS in h M of the double series sum_{j,m} (-1)^j N^j (x) N^m
+// / (j! (m+1)! (j+m+2)) with every power reduced by Cayley-Hamilton (exact
+// rational coefficients, rounded to FP32).
+template <int D>
+CPAB_HD __forceinline__ void chunk_moments(const Invariants<D>& iv, float h, float (&K)[D][D]) {
+    const float h2 = h * h, h3 = h2 * h, h4 = h2 * h2, tt = h * iv.t;
+    if constexpr (D == 2) {
+        const float dd = h2 * iv.d;
+        K[0][0] = h2 * fmaf(dd, fmaf(dd, fmaf(dd, -0.00158730159f, fmaf(tt, fmaf(tt, 0.00111607143f,
+                  -0.00297619048f), 0.0222222222f)), fmaf(tt, fmaf(tt, fmaf(tt, fmaf(tt, -0.000198412698f,
+                  0.000992063492f), -0.00833333333f), 0.025f), -0.166666667f)), 0.5f);
+        K[0][1] = h3 * fmaf(dd, fmaf(dd, fmaf(tt, 7.44047619e-05f, 0.00615079365f), fmaf(tt, fmaf(tt, fmaf(tt,
+                  -9.92063492e-05f, -0.00257936508f), -0.00277777778f), -0.0583333333f)), fmaf(tt, fmaf(tt, fmaf(tt,
+                  fmaf(tt, fmaf(tt, 2.48015873e-05f, 0.000198412698f), 0.00138888889f), 0.00833333333f),
+                  0.0416666667f), 0.166666667f));
+        K[1][0] = h3 * fmaf(dd, fmaf(dd, fmaf(tt, 0.0015625f, -0.00634920635f), fmaf(tt, fmaf(tt, fmaf(tt,
+                  -0.00104166667f, 0.00575396825f), -0.0208333333f), 0.0666666667f)), fmaf(tt, fmaf(tt, fmaf(tt,
+                  fmaf(tt, fmaf(tt, 0.000173611111f, -0.00119047619f), 0.00694444444f), -0.0333333333f), 0.125f),
+                  -0.333333333f));
+        K[1][1] = h4 * fmaf(dd, fmaf(dd, -0.0015625f, fmaf(tt, fmaf(tt, 0.00104166667f, -0.00257936508f),
+                  0.0208333333f)), fmaf(tt, fmaf(tt, fmaf(tt, fmaf(tt, -0.000173611111f, 0.000793650794f),
+                  -0.00694444444f), 0.0166666667f), -0.125f));
+    } else {
+        const float h5 = h4 * h, h6 = h3 * h3, ss = h2 * iv.sg, dd = h3 * iv.d;
+        K[0][0] = h2 * fmaf(dd, fmaf(dd, -0.000669642857f, fmaf(ss, fmaf(tt, -0.000396825397f, 0.000992063492f),
+                  fmaf(tt, fmaf(tt, fmaf(tt, 0.000198412698f, -0.000992063492f), 0.00833333333f), -0.025f))), 0.5f);
+        K[0][1] = h3 * fmaf(dd, fmaf(ss, 0.00133928571f, fmaf(tt, fmaf(tt, -0.000496031746f, 0.00317460317f),
+                  -0.0125f)), fmaf(ss, fmaf(ss, fmaf(tt, 4.96031746e-05f, 0.000198412698f), fmaf(tt, fmaf(tt,
+                  fmaf(tt, -2.48015873e-05f, -0.000198412698f), -0.00138888889f), -0.00833333333f)), 0.166666667f));
+        K[0][2] = h4 * fmaf(dd, fmaf(tt, 4.96031746e-05f, -0.00376984127f), fmaf(ss, fmaf(ss, 2.48015873e-05f,
+                  fmaf(tt, fmaf(tt, -7.44047619e-05f, -0.000396825397f), -0.00138888889f)), fmaf(tt, fmaf(tt,
+                  fmaf(tt, fmaf(tt, 2.48015873e-05f, 0.000198412698f), 0.00138888889f), 0.00833333333f),
+                  0.0416666667f)));
+        K[1][0] = h3 * fmaf(dd, fmaf(ss, 0.000694444444f, (tt * -0.00238095238f)), fmaf(ss, fmaf(ss, fmaf(tt,
+                  0.000347222222f, -0.00119047619f), fmaf(tt, fmaf(tt, fmaf(tt, -0.000173611111f, 0.00119047619f),
+                  -0.00694444444f), 0.0333333333f)), -0.333333333f));
+        K[1][1] = h4 * fmaf(dd, fmaf(tt, -0.000694444444f, 0.00178571429f), fmaf(ss, fmaf(ss, -0.0015625f, fmaf(tt,
+                  fmaf(tt, 0.000694444444f, -0.00178571429f), 0.0208333333f)), -0.125f));
+        K[1][2] = h5 * fmaf(dd, 0.000694444444f, fmaf(ss, fmaf(tt, 0.000347222222f, 0.00515873016f), fmaf(tt,
+                  fmaf(tt, fmaf(tt, -0.000173611111f, -0.00119047619f), -0.00694444444f), -0.0333333333f)));
+        K[2][0] = h4 * fmaf(dd, 0.00178571429f, fmaf(ss, fmaf(ss, 0.000173611111f, fmaf(tt, fmaf(tt,
+                  -0.000520833333f, 0.00238095238f), -0.00694444444f)), fmaf(tt, fmaf(tt, fmaf(tt, fmaf(tt,
+                  0.000173611111f, -0.00119047619f), 0.00694444444f), -0.0333333333f), 0.125f)));
+        K[2][1] = h5 * fmaf(ss, fmaf(tt, 0.00138888889f, -0.00595238095f), fmaf(tt, fmaf(tt, fmaf(tt,
+                  -0.000520833333f, 0.00297619048f), -0.0138888889f), 0.05f));
+        K[2][2] = h6 * fmaf(ss, -0.00138888889f, fmaf(tt, fmaf(tt, 0.000520833333f, -0.000992063492f),
+                  0.0138888889f));
+    }
+}
+
+// A chunk's dL/dA_q in G; carries mu to the chunk's end.
 template <int D>
 CPAB_HD __forceinline__ void chunk_grad(const Chunk<D>& ch, float (&mu)[D], float (&G)[D * (D + 1)]) {
-    const float h = ch.h;
-    float hp[KS + 2];
-    hp[0] = 1.f;
-#pragma unroll
-    for (int r = 1; r < KS + 2; ++r) hp[r] = hp[r - 1] * h;
-    float m[D], mend[D];
+    const FlowAt<D> fb = flow_at<D>(ch.iv, -ch.h);  // exp(-h M) and -int_0^h exp(-s M) ds
+    float K[D][D];
+    chunk_moments<D>(ch.iv, ch.h, K);
+    float m[D], gbar[D], mend[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) {
         m[a] = mu[a];
-        mend[a] = 0.f;
+        gbar[a] = -fb.al[0] * mu[a];
+        mend[a] = fb.e[0] * mu[a];
     }
 #pragma unroll
-    for (int p = 0; p < D * (D + 1); ++p) G[p] = 0.f;
+    for (int i = 0; i < D; ++i) {
+        // m = (M^T)^i mu0, u = sum_j K[i][j] M^j v0
+        float u[D];
 #pragma unroll
-    for (int j = 0; j <= KS; ++j) {
-        // Y_j = sum_{k=0}^{KS-j} h^(j+k+1)/(j+k+1) X_k,  X_0 = [q0;1], X_k = [W[k-1];0]
-        const float w0 = hp[j + 1] * (1.0f / (float)(j + 1));
-        float y[D];
+        for (int a = 0; a < D; ++a) {
+            float acc = K[i][0] * ch.v[0][a];
 #pragma unroll
-        for (int a = 0; a < D; ++a) y[a] = w0 * ch.q0[a];
-#pragma unroll
-        for (int k = 1; k <= KS - j; ++k) {
-            const float wk = hp[j + k + 1] * (1.0f / (float)(j + k + 1));
-#pragma unroll
-            for (int a = 0; a < D; ++a) y[a] = fmaf(wk, ch.W[k - 1][a], y[a]);
+            for (int k = 1; k < D; ++k) acc = fmaf(K[i][k], ch.v[k][a], acc);
+            u[a] = acc;
         }
-        const float sg = (j & 1) ? -1.f : 1.f;
 #pragma unroll
-        for (int r = 0; r < D; ++r) {
-            const float mr = sg * m[r];
+        for (int r = 0; r < D; ++r)
 #pragma unroll
-            for (int a = 0; a < D; ++a) G[r * (D + 1) + a] = fmaf(mr, y[a], G[r * (D + 1) + a]);
-            G[r * (D + 1) + D] = fmaf(mr, w0, G[r * (D + 1) + D]);
-            mend[r] = fmaf(sg * hp[j], m[r], mend[r]);
-        }
-        if (j < KS) {
-            const float inv = 1.0f / (float)(j + 1);
+            for (int a = 0; a < D; ++a)
+                G[r * (D + 1) + a] = (i == 0) ? m[r] * u[a] : fmaf(m[r], u[a], G[r * (D + 1) + a]);
+        if (i + 1 < D) {
             float t[D];
 #pragma unroll
             for (int r = 0; r < D; ++r) {
-                float acc = 0.f;
+                float acc = ch.M[0][r] * m[0];
 #pragma unroll
-                for (int a = 0; a < D; ++a) acc = fmaf(ch.M[a][r], m[a], acc);
-                t[r] = acc * inv;
+                for (int a = 1; a < D; ++a) acc = fmaf(ch.M[a][r], m[a], acc);
+                t[r] = acc;
             }
 #pragma unroll
-            for (int r = 0; r < D; ++r) m[r] = t[r];
+            for (int r = 0; r < D; ++r) {
+                m[r] = t[r];
+                gbar[r] = fmaf(-fb.al[i + 1], t[r], gbar[r]);
+                mend[r] = fmaf(fb.e[i + 1], t[r], mend[r]);
+            }
         }
+    }
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) G[r * (D + 1) + a] = fmaf(gbar[r], ch.q0[a], G[r * (D + 1) + a]);
+        G[r * (D + 1) + D] = gbar[r];
     }
 #pragma unroll
     for (int a = 0; a < D; ++a) mu[a] = mend[a];
