@@ -1214,28 +1214,9 @@ CPAB_HD __forceinline__ void chunk_grad1(const Chunk1& ch, float& mu, float (&G)
 // ---------------------------------------------------------------------------
 // wave-level deterministic accumulation of per-lane cell contributions
 // ---------------------------------------------------------------------------
-// One DPP step: every lane receives v of the lane CTRL selects (0 where there
-// is none or where ROWS masks the row out).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_take(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, true));
-}
-
-// Sum over the 64 lanes in a fixed order: inclusive scans inside each row of
-// 16 (row_shr 1, 2, 4, 8), then the row totals carried by row_bcast:15 and
-// row_bcast:31; lane 63 ends with the total, read into a scalar.
-__device__ __forceinline__ float wave_total(float v) {
-    v += dpp_take<0x111, 0xF>(v);
-    v += dpp_take<0x112, 0xF>(v);
-    v += dpp_take<0x114, 0xF>(v);
-    v += dpp_take<0x118, 0xF>(v);
-    v += dpp_take<0x142, 0xA>(v);
-    v += dpp_take<0x143, 0xC>(v);
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
-// Inclusive prefix sum over the 64 lanes (lane i gets lanes 0..i), same DPP
-// pattern as wave_total.
+// Inclusive prefix sum over the 64 lanes (lane i gets lanes 0..i): scans
+// inside each row of 16 (row_shr 1, 2, 4, 8), then the row totals carried by
+// row_bcast:15 and row_bcast:31.
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_take_int(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, true);
@@ -1275,55 +1256,106 @@ __device__ __forceinline__ int wave_max(int v) {
     return __builtin_amdgcn_readlane(v, 63);
 }
 
-// One DPP step on every row: adds the value of the lane CTRL selects (0
-// where there is none), a single add with a DPP operand.
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+// ---------------------------------------------------------------------------
+// Sums of P values over the 64 lanes, P = 2, 6 or 12 (D (D + 1)).
+//
+// Values are folded pairwise instead of one by one: a half-wave swap of two
+// registers (v_permlane32_swap) and one add leave the first value's partial
+// sums in lanes 0-31 and the second's in 32-63, a row swap (v_permlane16_swap)
+// does the same between neighbouring rows of 16, and inside the rows two
+// registers share one by a select on a lane bit.  12 instructions for P = 6
+// and 27 for P = 12 instead of 36 and 72 DPP adds, and the totals end in
+// different lanes, so one LDS add stores them all.  Every step is a fixed
+// order of additions.  us per launch, DPP adds / this: backward of [3, 3, 3] on
+// 16 x 64^3 points (5.5 cells per wave and round) 260 / 237, of [2, 2, 2] on
+// 16 clouds of 25001 points (every lane its own cell) 71 / 51; 2D (2.7 cells)
+// 732 / 730.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ float fold_halves(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+__device__ __forceinline__ float fold_rows(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// v plus w of the lane CTRL pairs this one with
+template <int CTRL>
+__device__ __forceinline__ float pair_add(float v, float w) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(w), CTRL, 0xF, 0xF, true));
+}
+constexpr int PAIR_8 = 0x128;  // row_ror:8          lane ^ 8
+constexpr int PAIR_7 = 0x141;  // row_half_mirror    lane ^ 7
+constexpr int PAIR_2 = 0x4E;   // quad_perm 2,3,0,1  lane ^ 2
+constexpr int PAIR_1 = 0xB1;   // quad_perm 1,0,3,2  lane ^ 1
 
-// wave_total of P values at once, left in lane 63: every step is taken for
-// all P before the next, so the steps of one value do not wait on each
-// other.  The two row broadcasts run on all rows; the rows wave_total masks
-// out (0 and 2, then 0 and 1) end with other sums, but lane 63 -- which
-// reads only the rows those steps keep -- gets wave_total's sum bit for bit.
+// The value index whose total fold_values leaves in this lane, if the lane is
+// the one that stores it, else -1.
 template <int P>
-__device__ __forceinline__ void wave_totals(float (&v)[P]) {
+__device__ __forceinline__ int fold_id() {
+    const int lane = __lane_id(), row = lane >> 4, in = lane & 15;
+    if constexpr (P == 2) {
+        return (in == 0 && !(row & 1)) ? row >> 1 : -1;
+    } else if constexpr (P == 6) {
+        if (in == 0) return 2 * (row & 1) + (row >> 1);
+        return (in == 8 && !(row & 1)) ? 4 + (row >> 1) : -1;
+    } else {
+        static_assert(P == 12, "P = D (D + 1)");
+        const int k = 2 * (row & 1) + (row >> 1);
+        return in == 0 ? k : (in == 8 ? 4 + k : (in == 4 ? 8 + k : -1));
+    }
+}
+template <int P>
+__device__ __forceinline__ float fold_values(const float (&v)[P]) {
+    float w[P / 2];
 #pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = dpp_add<0x111>(v[p]);
-#pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = dpp_add<0x112>(v[p]);
-#pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = dpp_add<0x114>(v[p]);
-#pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = dpp_add<0x118>(v[p]);
-#pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = dpp_add<0x142>(v[p]);
-#pragma unroll
-    for (int p = 0; p < P; ++p) v[p] = dpp_add<0x143>(v[p]);
+    for (int i = 0; i < P / 2; ++i) w[i] = fold_halves(v[2 * i], v[2 * i + 1]);
+    float y;
+    if constexpr (P == 2) {
+        y = fold_rows(w[0], w[0]);
+        y = pair_add<PAIR_8>(y, y);
+        y = pair_add<PAIR_7>(y, y);
+    } else {
+        const int lane = __lane_id();
+        const float x0 = fold_rows(w[0], w[1]);
+        const float x1 = P == 6 ? fold_rows(w[2], w[2]) : fold_rows(w[2], w[3 % (P / 2)]);
+        y = pair_add<PAIR_8>((lane & 8) ? x1 : x0, (lane & 8) ? x0 : x1);
+        if constexpr (P == 6) {
+            y = pair_add<PAIR_7>(y, y);
+        } else {
+            float x2 = fold_rows(w[4 % (P / 2)], w[5 % (P / 2)]);
+            x2 = pair_add<PAIR_8>(x2, x2);
+            y = pair_add<PAIR_7>((lane & 4) ? x2 : y, (lane & 4) ? y : x2);
+        }
+    }
+    y = pair_add<PAIR_2>(y, y);
+    return pair_add<PAIR_1>(y, y);
 }
 
 // Adds g (P values) of every lane with cell >= 0 into acc[cell*P + p] of this
 // wave's LDS region; the lanes sharing a cell are summed across the wave in a
-// fixed order and lane 63 adds the sums (LDS float adds, issued in program
-// order by the one lane).  Must be reached by all lanes of the wave.
+// fixed order, and each total is added by the lane that holds it (LDS float
+// adds, one lane per address, in program order).  Must be reached by all
+// lanes of the wave.
 template <int P>
 __device__ __forceinline__ void wave_accumulate(float* acc, int cell, const float (&g)[P]) {
-    const int lane = __lane_id();
+    const int id = fold_id<P>();
+    float* mine_acc = acc + id;
     uint64_t pending = __ballot(cell >= 0);
     while (pending) {
         const int leader = __ffsll((unsigned long long)pending) - 1;
         const int c0 = __builtin_amdgcn_readlane(cell, leader);
         const bool mine = (cell == c0);
         pending &= ~__ballot(mine);
-        float tot[P];
+        float v[P];
 #pragma unroll
-        for (int p = 0; p < P; ++p) tot[p] = mine ? g[p] : 0.f;
-        wave_totals<P>(tot);
-        if (lane == 63) {
-#pragma unroll
-            for (int p = 0; p < P; ++p) atomicAdd(&acc[c0 * P + p], tot[p]);
-        }
+        for (int p = 0; p < P; ++p) v[p] = mine ? g[p] : 0.f;
+        const float tot = fold_values<P>(v);
+        int off = c0 * P;
+        // the product stays scalar: folded into the lane address it would be a
+        // 64-bit multiply-add in every lane
+        asm volatile("" : "+s"(off));
+        if (id >= 0) atomicAdd(mine_acc + off, tot);
     }
 }
 
