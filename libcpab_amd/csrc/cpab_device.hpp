@@ -22,15 +22,14 @@
 // s = (qb-q0)/v0 * log1p(r)/r, r = a (qb-q0)/v0.
 //
 // Boundary hits.  For each facet G(s) = n.q(s) + e is the same series.  A
-// facet is skipped when a quadratic bound on G over the chunk stays negative
-// (for a start on the facet moving inwards: when G' stays negative).  Where a
-// bound on the series tail certifies the sign of G'' over the chunk, G(h)
-// decides the crossing and [0, h] brackets a unique root.  Starts on a facet,
+// facet is skipped when a convex cubic bound on G is negative at the chunk's
+// end.  Where a bound on the series tail certifies the sign of G'' or of G'
+// over the chunk, G(h) decides the crossing and [0, h] brackets a unique root.  Starts on a facet,
 // uncertified curvature and interior maxima are bracketed by sampling G and G'
 // at NSAMP points (a local maximum with G > 0 inside a sample interval
-// counts).  The candidate with the earliest regula-falsi estimate is solved
-// by Newton steps safeguarded by its bracket; another candidate is solved
-// only when it is positive at (or its bracket ends before) that root.
+// counts).  A bracket is solved by Newton steps safeguarded by it; a second
+// facet is solved only when it is positive at (or its bracket ends before) the
+// first one's root.
 //
 // Gradients.  The field is continuous across facets, so the sensitivity of the
 // final point obeys the variational equation with the saltation matrix
@@ -102,9 +101,15 @@ CPAB_HD __forceinline__ float fast_sqrt(float x) {
     return sqrtf(x);
 #endif
 }
+// a * b of non-negative integers below 2^24 (cell numbers and table strides): a
+// full-rate product; the compiler's own choice for a table address is a 64-bit
+// multiply-add at a quarter of the rate
+CPAB_HD __forceinline__ int mul_small(int a, int b) {
+    return (int)(((unsigned)a & 0xFFFFFFu) * ((unsigned)b & 0xFFFFFFu));
+}
 template <int D>
 CPAB_HD __forceinline__ void load_affine(const CellTable<D>& t, int c, float (&M)[D][D], float (&b)[D]) {
-    const float* a = t.A + c * (D * (D + 1));
+    const float* a = t.A + mul_small(c, D * (D + 1));
 #pragma unroll
     for (int r = 0; r < D; ++r) {
 #pragma unroll
@@ -378,6 +383,21 @@ CPAB_HD __forceinline__ void powers(const float (&M)[D][D], const float (&v0)[D]
         }
 }
 
+// The cells across the facets of cell c (one 16-byte load on the device, where
+// the staged table is aligned)
+template <int D>
+CPAB_HD __forceinline__ void cell_neighbours(const CellTable<D>& tab, int c, int (&nb)[NF]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int4 v = reinterpret_cast<const int4*>(tab.nb)[c];
+    nb[0] = v.x;
+    nb[1] = v.y;
+    nb[2] = v.z;
+    nb[3] = v.w;
+#else
+    for (int f = 0; f < NF; ++f) nb[f] = tab.nb[c * NF + f];
+#endif
+}
+
 // Coefficients of facet f of cell c.  A start within tol0 of the facet is a
 // start on it: G(0) = 0 exactly, so the sign of G just after the start is that
 // of G'(0) (and, for a shallow dip into the cell, of the dip) rather than that
@@ -516,19 +536,20 @@ CPAB_HD __forceinline__ void logged_chunk(const ChunkLog& lg, int k, float& h, i
 // ---------------------------------------------------------------------------
 // one chunk of integration, D = 2, 3
 //
-// VALU issue bounds it (89% of the nominal rate in the plain 2D grid
-// transform), so what counts is instructions per wave and chunk, and a branch
-// costs its whole body whenever one of 64 lanes takes it.  Hence the shared
-// scalars of flow_at instead of a series vector and a polynomial per facet, one
-// straight cull for all facets, then a loop over each lane's own remaining
-// facet (0.5 trips per chunk on [4, 4] images) instead of four branches, and a
-// root search that starts from the quadratic model (1.0 Newton steps per chunk
-// and wave instead of 2-3) and samples only where neither G'' nor G' has a
-// certified sign (2% of a wave's chunks).  [4, 4], 64 x 256^2 points,
-// us per launch before / after: grid transform 88 / 67, its recomputing
-// backward 208 / 152; fused with 3 channels and 256 thetas: forward 491 / 459,
-// backward 790 / 732; [3, 3, 3], 16 x 64^3: forward 192 / 167, backward
-// 293 / 260.
+// VALU issue bounds it (85-90% of the nominal rate in the plain 2D grid
+// transform, transcendentals counted once), so what counts is instructions per
+// wave and chunk, and a branch costs its whole body whenever one of 64 lanes
+// takes it.  Hence the shared scalars of flow_at instead of a series vector and
+// a polynomial per facet, one straight cull for all facets, then a loop over
+// each lane's own remaining facet (0.5 trips per chunk on [4, 4] images) instead
+// of four branches, and a root search that starts from the quadratic model (1.0
+// Newton steps per chunk and wave instead of 2-3) and samples only where neither
+// G'' nor G' has a certified sign (2% of a wave's chunks).  VALU instructions
+// per wave of the 2D grid transform (4 points a lane): 2600 with the scalars
+// alone, 2030 now.  [4, 4], 64 x 256^2 points, us per launch before / after:
+// grid transform 88 / 63, its recomputing backward 208 / 144; fused with 3
+// channels and 256 thetas: forward 491 / 448, backward 790 / 730-740;
+// [3, 3, 3], 16 x 64^3: forward 192 / 162, backward 293 / 234.
 // ---------------------------------------------------------------------------
 template <int D>
 CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab, float tol0, Chunk<D>& ch) {
@@ -551,7 +572,6 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
     const float nrm = fast_rcp(tab.inv_n[c]);  // |M|_F (the bounds below carry margin for its last bit)
     const float mh = h * nrm;
     const float K = GROW * vn * nrm;
-    const float K4 = 0.5f * K * mh * mh;
     const float K3 = K * nrm * (1.0f / 6.0f);
 
     // phase 1: cull, the same straight code for every facet slot (a wave runs
@@ -559,8 +579,14 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
     // most lanes off)
     const float hK3 = h * h * K3, hh = 0.5f * h;
     unsigned live = 0u;
+    int nbs[NF];
+    cell_neighbours(tab, c, nbs);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        // a 2D cell has a fourth facet only at the domain's boundary
+        if (D == 2 && f == 3 && __ballot(nbs[3] >= 0) == 0) break;
+#endif
         const float4 P = tab.pl[c * NF + f];
         const float n[3] = {P.x, P.y, P.z};
         float g0 = P.w, g1 = n[0] * v0[0], g2 = n[0] * ch.v[1][0];
@@ -576,45 +602,50 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
         // crossing when it is below 0 at h; a start on the facet counts as
         // G(0) = 0, and a convex bound that is 0 at 0 and below 0 at h is
         // below 0 in between
-        const bool culled = fmaf(h, fmaf(hh, fmaxf(g2, 0.f), hK3) + g1, g0 >= -tol0 ? 0.f : g0) < 0.f;
-        live |= culled || tab.nb[c * NF + f] < 0 ? 0u : 1u << f;
+        const float bound = fmaf(h, fmaf(hh, fmaxf(g2, 0.f), hK3) + g1, g0 >= -tol0 ? 0.f : g0);
+        live |= (!(bound < 0.f) & (nbs[f] >= 0)) ? 1u << f : 0u;
     }
-    // Tangential band for an outward normal speed G'(0): the neighbouring
-    // cells' FP32 fields agree on a shared facet only up to the rounding of
-    // M q + b, whose terms can be much larger than |v0| where they cancel, so
-    // both may round a vanishing normal speed to a small exit.  Inside the
-    // band a start exit also needs G'' > 0 (the same side from both cells for
-    // a tangent velocity); an inward G'(0) always follows the dip.
-    float vabs = 0.f;
+    float tol1 = 0.f;
+    if (live) {
+        // Tangential band for an outward normal speed G'(0): the neighbouring
+        // cells' FP32 fields agree on a shared facet only up to the rounding of
+        // M q + b, whose terms can be much larger than |v0| where they cancel,
+        // so both may round a vanishing normal speed to a small exit.  Inside
+        // the band a start exit also needs G'' > 0 (the same side from both
+        // cells for a tangent velocity); an inward G'(0) always follows the dip.
+        float vabs = 0.f;
 #pragma unroll
-    for (int r = 0; r < D; ++r) {
-        float t = fabsf(ch.b[r]);
+        for (int r = 0; r < D; ++r) {
+            float t = fabsf(ch.b[r]);
 #pragma unroll
-        for (int a = 0; a < D; ++a) t = fmaf(fabsf(ch.M[r][a]), fabsf(st.q[a]), t);
-        vabs += t;
+            for (int a = 0; a < D; ++a) t = fmaf(fabsf(ch.M[r][a]), fabsf(st.q[a]), t);
+            vabs += t;
+        }
+        tol1 = 1e-6f * vabs;
+        // A velocity inside that band is rounding noise: the point sits on a
+        // fixed point of the field at FP32 resolution (e.g. a domain corner
+        // under zero_boundary) and moves by at most e^RHO |v0| h over the
+        // chunk.  It crosses no facet in this chunk (otherwise the noise could
+        // carry it back and forth across a facet through the fixed point, a
+        // hop per chunk, until the chunk budget ran out).
+        if (vn <= tol1) live = 0u;
     }
-    const float tol1 = 1e-6f * vabs;
-    // A velocity inside that band is rounding noise: the point sits on a
-    // fixed point of the field at FP32 resolution (e.g. a domain corner under
-    // zero_boundary) and moves by at most e^RHO |v0| h over the chunk.  It
-    // crosses no facet in this chunk (otherwise the noise could carry it
-    // back and forth across a facet through the fixed point, a hop per
-    // chunk, until the chunk budget ran out).
-    if (vn <= tol1) live = 0u;
-    // phase 2: classify the facets left, one of each lane at a time.  A facet
-    // whose first crossing lies in [0, h] with a unique root becomes a
-    // candidate (cand); the best so far is the one with the earliest
-    // regula-falsi estimate.  Starts on a facet, and facets whose curvature
-    // sign is not certified, take the sampling path (slow).
-    int start_f = -1, bf = -1;
-    unsigned cand = 0u, slow = 0u, sampled = 0u;
-    float est = INFINITY, lo = 0.f, hi = 0.f, glo = 0.f, ghi = 0.f;
+    // phase 2: the facets left, one of each lane at a time, keep the earliest
+    // crossing (best, bf).  A facet whose first crossing lies in [0, h] with a
+    // certified unique root has that bracket; starts on a facet, and facets
+    // whose curvature and slope have no certified sign, are sampled for theirs.
+    // A later facet is solved only where it is outside at the best root so far.
+    // (One site each for the sampling and the root search: a second copy of
+    // either costs scalar registers for its nested lane masks, which then
+    // spill into vector lanes.)
+    const float K4 = 0.5f * K * mh * mh;
+    float best = h;
+    int bf = -1;
 #pragma unroll 1
     while (live) {
         const int f = __builtin_ctz(live);
         live &= live - 1u;
         const FacetG<D> F = facet_coeffs<D>(tab, c, f, st.q, ch.v, tol0);
-        const bool on = F.g[0] >= -tol0;
         // G''(s) = 2 cf2 + 6 cf3 s + R(s), |R| <= K4, 6 cf3 = n.M^2 v0: the sign
         // of G'' is certified when the linear part keeps one sign with margin K4
         float g3;
@@ -622,107 +653,51 @@ CPAB_HD __forceinline__ void advance(PointState<D>& st, const CellTable<D>& tab,
         else g3 = F.g[3];
         const float l0 = F.g[2], l1 = fmaf(g3, h, l0);
         const bool bent = fminf(l0, l1) > K4 || fmaxf(l0, l1) < -K4;
-        const float gh = facet_g<D>(F, ch.f);
-        if (on) {
-            const bool allow_start =
-                !(st.zero_hops > 0 && tab.nb[c * NF + f] == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
-            if (allow_start && (F.g[1] > tol1 || (F.g[1] >= 0.f && F.g[2] > 0.f))) {
-                if (start_f < 0) start_f = f;
-            } else if (!(F.g[1] < -tol1 && bent && gh <= 0.f)) {
-                // (a clear start inwards that ends inside has no crossing in
-                // between when G is convex or concave on the chunk)
-                slow |= 1u << f;
-            }
-            continue;
-        }
-        // Likewise G' = g1 + g2 s + R, |R| <= 3 K3 s^2, for a G that is too
-        // straight for its curvature to have a certified sign.
+        // likewise G' = g1 + g2 s + R, |R| <= 3 K3 s^2, for a G that is too
+        // straight for its curvature to have a certified sign
         const float e1 = fmaf(l0, h, F.g[1]), r1 = 3.f * hK3;
         const bool rising = fminf(F.g[1], e1) > r1, falling = fmaxf(F.g[1], e1) < -r1;
-        if (!(bent || rising || falling)) {
-            slow |= 1u << f;
-            continue;
-        }
-        // G convex (g2 > 0), concave (g2 < 0) or monotonic on [0, h], G(0) < 0: a
-        // positive G(h) means exactly one crossing; otherwise only a concave G
-        // rising and falling inside the chunk can cross (sampling path).
-        if (gh > 0.f) {
-            cand |= 1u << f;
-            const float e = h * (F.g[0] * fast_rcp(F.g[0] - gh));
-            if (e < est) {
-                est = e;
-                bf = f;
-                hi = h;
-                glo = F.g[0];
-                ghi = gh;
+        float lo = 0.f, hi = h, glo = F.g[0], ghi = facet_g<D>(F, ch.f);
+        const bool allow_start =
+            !(st.zero_hops > 0 && tab.nb[c * NF + f] == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
+        bool take = ghi > 0.f, sample;
+        if (F.g[0] >= -tol0) {
+            if (allow_start && (F.g[1] > tol1 || (F.g[1] >= 0.f && F.g[2] > 0.f))) {
+                if (best > 0.f) {
+                    best = 0.f;
+                    bf = f;
+                }
+                continue;
             }
-        } else if (l0 < 0.f && F.g[1] > 0.f && !rising && facet_dg<D>(F, ch.f) < 0.f) {
-            slow |= 1u << f;
+            // a clear start inwards that ends inside has no crossing in between
+            // when G is convex or concave on the chunk
+            sample = !(F.g[1] < -tol1 && bent && !take);
+        } else {
+            // G convex, concave or monotonic on [0, h], G(0) < 0: a positive G(h)
+            // means exactly one crossing; otherwise only a concave G rising and
+            // falling inside the chunk can cross
+            sample = !(bent || rising || falling) ||
+                     (!take && l0 < 0.f && F.g[1] > 0.f && !rising && facet_dg<D>(F, ch.f) < 0.f);
         }
-    }
-    // sampling path (starts on a facet, uncertified curvature, interior maxima)
-    if (start_f < 0) {
-#pragma unroll 1
-        while (slow) {
-            const int f = __builtin_ctz(slow);
-            slow &= slow - 1u;
-            const FacetG<D> F = facet_coeffs<D>(tab, c, f, st.q, ch.v, tol0);
-            const int nbf = tab.nb[c * NF + f];
-            const bool allow_start = !(st.zero_hops > 0 && nbf == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
+        if (sample) {
             Bracket br;
             first_bracket<D>(F, ch.iv, h, tol0, tol1, allow_start, br);
-            if (br.idx >= 1 && br.idx <= NSAMP) {
-                cand |= 1u << f;
-                sampled |= 1u << f;
-                const float e = fmaf(br.hi - br.lo, br.glo * fast_rcp(br.glo - br.ghi), br.lo);
-                if (e < est) {
-                    est = e;
-                    bf = f;
-                    lo = br.lo;
-                    hi = br.hi;
-                    glo = br.glo;
-                    ghi = br.ghi;
-                }
-            }
+            take = br.idx >= 1 && br.idx <= NSAMP;
+            lo = br.lo;
+            hi = br.hi;
+            glo = br.glo;
+            ghi = br.ghi;
         }
-    }
-    // phase 3: solve the candidate with the earliest estimate, then any other
-    // candidate that is still positive at (or ends before) that root
-    float best = h;
-    if (start_f >= 0) {
-        best = 0.f;
-        bf = start_f;
-    } else if (bf >= 0) {
-        best = solve_bracket<D>(facet_coeffs<D>(tab, c, bf, st.q, ch.v, tol0), ch.iv, lo, hi, glo, ghi);
-        unsigned others = cand & ~(1u << bf);
-#pragma unroll 1
-        while (others) {
-            const int f = __builtin_ctz(others);
-            others &= others - 1u;
-            const FacetG<D> F = facet_coeffs<D>(tab, c, f, st.q, ch.v, tol0);
-            // a certified candidate's bracket is [0, h]; a sampled one's is
-            // found again
-            lo = 0.f;
-            hi = h;
-            glo = F.g[0];
-            if ((sampled >> f) & 1u) {
-                const int nbf = tab.nb[c * NF + f];
-                const bool allow_start = !(st.zero_hops > 0 && nbf == st.came_from) && st.zero_hops < MAX_ZERO_HOPS;
-                Bracket br;
-                first_bracket<D>(F, ch.iv, h, tol0, tol1, allow_start, br);
-                lo = br.lo;
-                hi = br.hi;
-                glo = br.glo;
-            }
-            if (!(lo < best)) continue;
-            if (best < hi) hi = best;
+        if (!take || !(lo < best)) continue;
+        if (best < hi) {
+            hi = best;
             ghi = facet_g<D>(F, flow_at<D>(ch.iv, hi));
-            if (ghi > 0.f) {
-                const float s2 = solve_bracket<D>(F, ch.iv, lo, hi, glo, ghi);
-                if (s2 < best) {
-                    best = s2;
-                    bf = f;
-                }
+        }
+        if (ghi > 0.f) {
+            const float s = solve_bracket<D>(F, ch.iv, lo, hi, glo, ghi);
+            if (s < best || bf < 0) {
+                best = s;
+                bf = f;
             }
         }
     }
