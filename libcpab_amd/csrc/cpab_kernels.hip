@@ -448,7 +448,7 @@ __device__ __forceinline__ float interp_value(const float* __restrict__ dp, cons
 template <int D>
 constexpr int chan_group() { return 1; }
 template <int D>
-constexpr int chan_group_bwd() { return 2; }
+constexpr int chan_group_bwd() { return D == 2 ? 2 : 1; }
 
 // out[c * ostride] = channel c (data + c * dstride) at the corners, for every
 // channel.  The loads of a group of channels are all issued before the first
@@ -475,80 +475,155 @@ __device__ __forceinline__ void interp_channels(const float* __restrict__ data, 
     }
 }
 
-// backward of blend for upstream g at corner values v: adds d value / d fd[a]
-// into dfd and, with gp (nullable), scatters g times each corner's weight
-template <int D>
-__device__ __forceinline__ void blend_backward(const float (&v)[1 << D], const int (&off)[1 << D], float* gp,
-                                               const float (&fd)[3], float g, float (&dfd)[3]) {
-    if constexpr (D == 1) {
-        if (gp) {
-            atomicAdd(gp + off[0], g * (1.f - fd[0]));
-            atomicAdd(gp + off[1], g * fd[0]);
+// ---------------------------------------------------------------------------
+// scatter into dL/ddata
+// ---------------------------------------------------------------------------
+// A point adds its upstream value, weighted, to the 2^D samples around it.  A
+// wave's lanes are neighbouring points, and the samples above one point are
+// mostly the samples below the next: lane + 1 (next along the last axis) and
+// lane + w (next along the axis before, w lanes per row of the wave's tile).
+// So a lane hands the weights of its upper samples to the lane whose lower
+// samples they are, where there is one (its lower corner lies exactly one
+// sample further), and only what is left goes to memory: about 2 atomics per
+// point and channel instead of 4 in 2D, nearly all of them to addresses of
+// their own and in runs of the data's rows.  us per backward, an atomic per
+// corner / merged: [2, 2, 2], 6 x 2 x 49x40x35 volumes 115 / 85; [50], 2048
+// signals of 1024 112 / 101.
+struct MergePlan {
+    bool h, v;  // lane + 1 / lane + w takes the upper samples
+    bool valid;
+    int up;     // byte address (ds_bpermute) of lane - w
+};
+
+// inner: the lane is valid and its upper samples differ from its lower ones on
+// every axis (a point beyond the last sample has both on it; such a lane
+// neither gives nor takes, so equal lower corners mean equal upper ones).
+// INST: neighbouring lanes may belong to different instances inst.
+template <int D, bool INST>
+__device__ __forceinline__ MergePlan merge_plan(bool valid, bool inner, int lower, int row_stride, int w, int inst) {
+    MergePlan m;
+    const int lane = __lane_id();
+    const int code = inner ? lower : -2;  // the lower corner's offset; -2 + 1 is no offset
+    // row_shl:1 (lanes without a source in their row of 16 keep -2)
+    m.h = __builtin_amdgcn_update_dpp(-2, code, 0x101, 0xF, 0xF, false) == code + 1;
+    if constexpr (INST) m.h = m.h && __builtin_amdgcn_update_dpp(-2, inst, 0x101, 0xF, 0xF, false) == inst;
+    m.valid = valid;
+    m.v = false;
+    m.up = 0;
+    if constexpr (D > 1) {
+        if (w > 0) {
+            const int next = __builtin_amdgcn_ds_bpermute(((lane + w) & 63) << 2, code);
+            m.v = inner && lane + w < 64 && next == code + row_stride;
+            m.up = ((lane - w) & 63) << 2;
         }
+    }
+    return m;
+}
+
+// Adds the corner values x (corner_offsets order, already weighted; 0 where
+// the lane is not valid) into gp.  Reached by all lanes of the wave.
+template <int D>
+__device__ __forceinline__ void merged_scatter(float* __restrict__ gp, const int (&off)[1 << D], float (&x)[1 << D],
+                                               const MergePlan& m) {
+    constexpr int NK = 1 << D;
+    if (__ballot(m.h)) {
+#pragma unroll
+        for (int j = 1; j < NK; j += 2) {
+            const float s = m.h ? x[j] : 0.f;
+            // row_shr:1, 0 into the first lane of a row of 16
+            x[j - 1] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x111, 0xF, 0xF, true));
+        }
+    }
+    if (m.valid && !m.h) {
+#pragma unroll
+        for (int j = 1; j < NK; j += 2)
+            if (x[j] != 0.f) atomicAdd(gp + (unsigned)off[j], x[j]);
+    }
+    if constexpr (D > 1) {
+        if (__ballot(m.v)) {
+#pragma unroll
+            for (int j = 2; j < NK; j += 4) {
+                const float s = m.v ? x[j] : 0.f;
+                x[j - 2] += __int_as_float(__builtin_amdgcn_ds_bpermute(m.up, __float_as_int(s)));
+            }
+        }
+        if (m.valid && !m.v) {
+#pragma unroll
+            for (int j = 2; j < NK; j += 4)
+                if (x[j] != 0.f) atomicAdd(gp + (unsigned)off[j], x[j]);
+        }
+    }
+    if (m.valid) {
+#pragma unroll
+        for (int j = 0; j < NK; j += 4) atomicAdd(gp + (unsigned)off[j], x[j]);
+    }
+}
+
+// The 2^D corner weights from the fractions, each axis's whole weight on the
+// lower corner where the upper one is clamped onto it; inner: none is
+template <int D>
+__device__ __forceinline__ void corner_weights(const int (&i0)[3], const int (&i1)[3], const float (&fd)[3],
+                                               float (&wt)[1 << D], bool& inner) {
+    float f[D];
+    inner = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        f[a] = i1[a] != i0[a] ? fd[a] : 0.f;
+        inner = inner && i1[a] != i0[a];
+    }
+#pragma unroll
+    for (int j = 0; j < (1 << D); ++j) {
+        float p = 1.f;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            const float q = ((j >> (D - 1 - a)) & 1) ? f[a] : 1.f - f[a];
+            p = a ? p * q : q;
+        }
+        wt[j] = p;
+    }
+}
+
+// backward of blend for upstream g at corner values v: adds d value / d fd[a]
+// into dfd
+template <int D>
+__device__ __forceinline__ void blend_backward(const float (&v)[1 << D], const float (&fd)[3], float g,
+                                               float (&dfd)[3]) {
+    if constexpr (D == 1) {
         dfd[0] = fmaf(g, v[1] - v[0], dfd[0]);
     } else if constexpr (D == 2) {
         const float c00 = v[0], c01 = v[1], c10 = v[2], c11 = v[3];
         const float wx0 = 1.f - fd[0], wx1 = fd[0], wy0 = 1.f - fd[1], wy1 = fd[1];
-        if (gp) {
-            atomicAdd(gp + off[0], g * wx0 * wy0);
-            atomicAdd(gp + off[2], g * wx1 * wy0);
-            atomicAdd(gp + off[1], g * wx0 * wy1);
-            atomicAdd(gp + off[3], g * wx1 * wy1);
-        }
         const float c0 = c00 * wx0 + c10 * wx1;
         const float c1 = c01 * wx0 + c11 * wx1;
         dfd[0] = fmaf(g, (c10 - c00) * wy0 + (c11 - c01) * wy1, dfd[0]);
         dfd[1] = fmaf(g, c1 - c0, dfd[1]);
     } else {
         const float w[3][2] = {{1.f - fd[0], fd[0]}, {1.f - fd[1], fd[1]}, {1.f - fd[2], fd[2]}};
-        float cv[2][2][2];
-#pragma unroll
-        for (int bx = 0; bx < 2; ++bx)
-#pragma unroll
-            for (int by = 0; by < 2; ++by)
-#pragma unroll
-                for (int bz = 0; bz < 2; ++bz) {
-                    const int j = bx * 4 + by * 2 + bz;
-                    cv[bx][by][bz] = v[j];
-                    if (gp) atomicAdd(gp + off[j], g * w[0][bx] * w[1][by] * w[2][bz]);
-                }
-        // derivative of the trilinear blend w.r.t. fd[a]
+        // derivative of the trilinear blend w.r.t. fd[a]; v[bx * 4 + by * 2 + bz]
         float dx = 0.f, dy = 0.f, dz = 0.f;
 #pragma unroll
         for (int by = 0; by < 2; ++by)
 #pragma unroll
-            for (int bz = 0; bz < 2; ++bz) dx += (cv[1][by][bz] - cv[0][by][bz]) * w[1][by] * w[2][bz];
+            for (int bz = 0; bz < 2; ++bz) dx += (v[4 + by * 2 + bz] - v[by * 2 + bz]) * w[1][by] * w[2][bz];
 #pragma unroll
         for (int bx = 0; bx < 2; ++bx)
 #pragma unroll
-            for (int bz = 0; bz < 2; ++bz) dy += (cv[bx][1][bz] - cv[bx][0][bz]) * w[0][bx] * w[2][bz];
+            for (int bz = 0; bz < 2; ++bz) dy += (v[bx * 4 + 2 + bz] - v[bx * 4 + bz]) * w[0][bx] * w[2][bz];
 #pragma unroll
         for (int bx = 0; bx < 2; ++bx)
 #pragma unroll
-            for (int by = 0; by < 2; ++by) dz += (cv[bx][by][1] - cv[bx][by][0]) * w[0][bx] * w[1][by];
+            for (int by = 0; by < 2; ++by) dz += (v[bx * 4 + by * 2 + 1] - v[bx * 4 + by * 2]) * w[0][bx] * w[1][by];
         dfd[0] = fmaf(g, dx, dfd[0]);
         dfd[1] = fmaf(g, dy, dfd[1]);
         dfd[2] = fmaf(g, dz, dfd[2]);
     }
 }
 
-// backward of interp_value for channel data dp with upstream g: scatters into
-// gp (nullable) and returns d value / d fd[a] accumulated into dfd
-template <int D>
-__device__ __forceinline__ void interp_backward(const float* __restrict__ dp, float* gp, const Img& im, const int (&i0)[3],
-                                                const int (&i1)[3], const float (&fd)[3], float g, float (&dfd)[3]) {
-    int off[1 << D];
-    corner_offsets<D>(im, i0, i1, off);
-    float v[1 << D];
-#pragma unroll
-    for (int j = 0; j < (1 << D); ++j) v[j] = dp[off[j]];
-    blend_backward<D>(v, off, gp, fd, g, dfd);
-}
-
-// interp_backward over every channel c, upstream gout[c * gstride] (the first
-// four also returned in gk): the loads of a group of channels' upstream values
-// and corners are issued before any of them is used; dfd accumulates in
-// channel order.  gdata (nullable) receives the scatter.
+// Backward of interp_channels with upstream gout[c * gstride] (the first four
+// channels' values also returned in gk): dfd receives d value / d fd summed
+// over the channels, in channel order, and gdata (nullable) one atomic per
+// corner.  The loads of a group of channels are issued before any of them is
+// used.
 template <int D>
 __device__ __forceinline__ void interp_backward_channels(const float* __restrict__ data, float* gdata, size_t dstride,
                                                          const Img& im, const int (&i0)[3], const int (&i1)[3],
@@ -570,13 +645,58 @@ __device__ __forceinline__ void interp_backward_channels(const float* __restrict
 #pragma unroll
         for (int k = 0; k < CG; ++k)
             if (c0 + k < im.C) {
-                blend_backward<D>(v[k], off, gdata ? gdata + (size_t)(c0 + k) * dstride : nullptr, fd, gv[k], dfd);
+                blend_backward<D>(v[k], fd, gv[k], dfd);
+                if (gdata) {
+                    float* gp = gdata + (size_t)(c0 + k) * dstride;
+#pragma unroll
+                    for (int j = 0; j < NK; ++j) {
+                        float p = gv[k];
+#pragma unroll
+                        for (int a = 0; a < D; ++a) p *= ((j >> (D - 1 - a)) & 1) ? fd[a] : 1.f - fd[a];
+                        atomicAdd(gp + off[j], p);
+                    }
+                }
                 if (c0 + k < 4) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         if (j == c0 + k) gk[j] = gv[k];
                 }
             }
+    }
+}
+
+// The same with the merged scatter into gdata (nullable for the whole wave).
+// Reached by all lanes of the wave; a lane that is not valid has in-bounds
+// corners and pointers and adds nothing.  w: lanes per row of the wave's tile
+// (0: no second axis to merge along); INST, inst: as in merge_plan.
+template <int D, bool INST = false>
+__device__ __forceinline__ void interp_backward_merged(bool valid, const float* __restrict__ data, float* gdata,
+                                                       size_t dstride, const Img& im, const int (&i0)[3],
+                                                       const int (&i1)[3], const float (&fd)[3],
+                                                       const float* __restrict__ gout, size_t gstride, int w,
+                                                       float (&dfd)[3], int inst = 0) {
+    constexpr int NK = 1 << D;
+    int off[NK];
+    corner_offsets<D>(im, i0, i1, off);
+    float wt[NK];
+    MergePlan m;
+    if (gdata) {
+        bool inner;
+        corner_weights<D>(i0, i1, fd, wt, inner);
+        m = merge_plan<D, INST>(valid, valid && inner, off[0], D == 3 ? im.s2 : im.s1, w, inst);
+    }
+    for (int c = 0; c < im.C; ++c) {
+        const float* dp = data + (size_t)c * dstride;
+        const float g = gout[(size_t)c * gstride];
+        float v[NK];
+#pragma unroll
+        for (int j = 0; j < NK; ++j) v[j] = dp[off[j]];
+        blend_backward<D>(v, fd, g, dfd);
+        if (gdata) {
+#pragma unroll
+            for (int j = 0; j < NK; ++j) v[j] = valid ? g * wt[j] : 0.f;
+            merged_scatter<D>(gdata + (size_t)c * dstride, off, v, m);
+        }
     }
 }
 
@@ -866,9 +986,6 @@ __global__ __launch_bounds__(BLOCK) void k_transform_bwd(Launch L, Geo g, Src s,
     write_partials<D>(acc, part + ((size_t)th * L.tiles + tile) * nC * P, nC * P);
 }
 
-// adjoint of k_transform_data.  gout [n_theta, C, outsize] in output order;
-// saved (nullable) from the forward.  im.gdata (nullable, zero-filled by the
-// caller) receives dL/ddata by atomic scatter.
 // One tile of one instance's fused backward; adds dL/dA_q of the tile's points
 // into this wave's LDS accumulator wacc (all lanes of the block take part).
 //
@@ -880,8 +997,12 @@ __global__ __launch_bounds__(BLOCK) void k_transform_bwd(Launch L, Geo g, Src s,
 // straight to its slot in bin order, and every cell of the footprint's
 // bounding box gathers the weighted grad_out of the points in the four bins
 // that touch it and adds it to dL/ddata with one global atomic per channel --
-// instead of four atomics per point and channel.
-template <int D, bool HAVES>
+// instead of four atomics per point and channel.  (Merging lanes and adding what
+// is left to global memory directly took the image workload's backward from
+// 740 to 1506 us: the lanes that do not line up are scattered atomics.)
+//
+// MERGE: dL/ddata by merged_scatter, for the calls without the box.
+template <int D, bool HAVES, bool MERGE>
 __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, const Src& s, const Img& im,
                                                const CellTable<D>& tab, int tile, const float* __restrict__ data,
                                                float* __restrict__ gdata, const float* __restrict__ gout,
@@ -962,9 +1083,10 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
         }
     }
     for (int r = 0; r < L.ppt; ++r) {
-        const int t = tile_t<D>(L, s, tile, r);
+        int t = tile_t<D>(L, s, tile, r);
         const bool valid = t >= 0;
-        float q0[D], mu[D];
+        float q0[D], mu[D], J[D][D], y[D];
+        float dfd[3] = {0.f, 0.f, 0.f};
         int c0 = 0;
         ChunkLog lg;
         lg.code = 0;
@@ -972,6 +1094,9 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
         for (int a = 0; a < D; ++a) {
             q0[a] = 0.f;
             mu[a] = 0.f;
+            y[a] = 0.f;
+#pragma unroll
+            for (int k = 0; k < D; ++k) J[a][k] = 0.f;
         }
         if (valid) {
             int ix[3];
@@ -983,7 +1108,6 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                 q0[a] = x[a] * (float)nc[a];
             }
             c0 = start_cell<D>(x, nc, tab, g);
-            float J[D][D], y[D];
             if constexpr (HAVES) {
 #pragma unroll
                 for (int a = 0; a < D; ++a) y[a] = sv[(size_t)a * L.nP + t];
@@ -1004,31 +1128,31 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
 #pragma unroll
                 for (int a = 0; a < D; ++a) y[a] = q[a] * rnc[a];
             }
+            if constexpr (!MERGE) {
+                int i0[3], i1[3];
+                float fd[3], gk[4] = {0.f, 0.f, 0.f, 0.f};
+                corners<D>(y, im, i0, i1, fd);
+                interp_backward_channels<D>(data, (D != 2 || use_box) ? nullptr : gdata, dstride, im, i0, i1, fd, gout + t,
+                                            L.nP, gk, dfd);
+                if constexpr (D == 2) {
+                    if (use_box) {
+                        const int cd = code[r * BLOCK + threadIdx.x];
+                        const int pos = bins[cd & 2047] + (cd >> 11);
+                        // a clamped corner pair (i1 == i0) puts its whole weight on i0
+                        fd2[pos] = make_float2(i1[0] != i0[0] ? fd[0] : 0.f, i1[1] != i0[1] ? fd[1] : 0.f);
+                        gv4[pos] = make_float4(gk[0], gk[1], gk[2], gk[3]);
+                    }
+                }
+            }
+        }
+        if constexpr (MERGE) {
+            if (__ballot(valid) == 0) continue;
             int i0[3], i1[3];
-            float fd[3], dfd[3] = {0.f, 0.f, 0.f};
+            float fd[3];
             corners<D>(y, im, i0, i1, fd);
-            const int slot = r * BLOCK + threadIdx.x;
-            float gk[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (D == 2) {
-                interp_backward_channels<D>(data, (gdata && !use_box) ? gdata : nullptr, dstride, im, i0, i1, fd,
-                                            gout + t, L.nP, gk, dfd);
-            } else {
-                for (int c = 0; c < im.C; ++c) {
-                    const size_t base = (size_t)c * dstride;
-                    const float gv = gout[(size_t)c * L.nP + t];
-                    interp_backward<D>(data + base, gdata ? gdata + base : nullptr, im, i0, i1, fd, gv, dfd);
-                    if (c < 4) gk[c] = gv;
-                }
-            }
-            if constexpr (D == 2) {
-                if (use_box) {
-                    const int cd = code[slot];
-                    const int pos = bins[cd & 2047] + (cd >> 11);
-                    // a clamped corner pair (i1 == i0) puts its whole weight on i0
-                    fd2[pos] = make_float2(i1[0] != i0[0] ? fd[0] : 0.f, i1[1] != i0[1] ? fd[1] : 0.f);
-                    gv4[pos] = make_float4(gk[0], gk[1], gk[2], gk[3]);
-                }
-            }
+            interp_backward_merged<D>(valid, data, gdata, dstride, im, i0, i1, fd, gout + (valid ? t : 0), L.nP, L.ty, dfd);
+        }
+        if (valid) {
             float w[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) w[a] = dfd[a] * (float)(sz[a] - 1) * rnc[a];
@@ -1102,7 +1226,7 @@ __host__ __device__ inline int bwd_blocks_per_theta(int tiles, int g1, int ty, i
 // caller) receives dL/ddata by atomic scatter.  Each block runs tpb tiles of
 // one theta (bwd_blocks_per_theta) into one row of partials, so the tables
 // are staged and the partials written once per tpb tiles.
-template <int D, bool HAVES>
+template <int D, bool HAVES, bool MERGE>
 __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_data_bwd(Launch L, Geo g, Src s, Img im, const float* __restrict__ Aq,
                                                               const float* __restrict__ gout,
                                                               const float* __restrict__ saved, float* __restrict__ part,
@@ -1124,7 +1248,7 @@ __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_
         const int trow = (bt / tiles_y) * tpb + k;
         if (tpb > 1 && trow >= tiles_x) break;
         const int tile = tpb > 1 ? trow * tiles_y + bt % tiles_y : bt;
-        fused_bwd_tile<D, HAVES>(L, g, s, im, tab, tile, im.data + (size_t)th * im.C * dstride,
+        fused_bwd_tile<D, HAVES, MERGE>(L, g, s, im, tab, tile, im.data + (size_t)th * im.C * dstride,
                                  im.gdata ? im.gdata + (size_t)th * im.C * dstride : nullptr,
                                  gout + (size_t)th * im.C * L.nP,
                                  HAVES ? saved + (size_t)th * saved_rows(D) * L.nP : nullptr,
@@ -1182,8 +1306,10 @@ __global__ __launch_bounds__(BLOCK) void k_interp_fwd(int N, int nP, Src s, Img 
 template <int D>
 __global__ __launch_bounds__(BLOCK) void k_interp_bwd(int N, int nP, Src s, Img im, const float* __restrict__ gout,
                                                       float* __restrict__ ggrid) {
-    int n, t, p;
-    if (!interp_item<D>(s, N, nP, n, t, p)) return;
+    int n = 0, t = 0, p = 0;
+    const bool valid = interp_item<D>(s, N, nP, n, t, p);
+    if (__ballot(valid) == 0) return;
+    if (!valid) n = t = p = 0;
     float y[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) y[a] = s.pts[((size_t)n * D + a) * nP + p];
@@ -1191,12 +1317,11 @@ __global__ __launch_bounds__(BLOCK) void k_interp_bwd(int N, int nP, Src s, Img 
     float fd[3], dfd[3] = {0.f, 0.f, 0.f};
     corners<D>(y, im, i0, i1, fd);
     const size_t dstride = (size_t)im.s0 * (D > 1 ? im.s1 : 1) * (D > 2 ? im.s2 : 1);
-    for (int c = 0; c < im.C; ++c) {
-        const size_t base = ((size_t)n * im.C + c) * dstride;
-        interp_backward<D>(im.data + base, im.gdata ? im.gdata + base : nullptr, im, i0, i1, fd,
-                           gout[((size_t)n * im.C + c) * nP + t], dfd);
-    }
-    if (ggrid) {
+    const size_t base = (size_t)n * im.C * dstride;
+    // 2D waves are 8 x 8 tiles of one instance; others runs that may span two
+    interp_backward_merged<D, D != 2>(valid, im.data + base, im.gdata ? im.gdata + base : nullptr, dstride, im, i0, i1,
+                                        fd, gout + (size_t)n * im.C * nP + t, nP, D == 2 ? 8 : 0, dfd, n);
+    if (ggrid && valid) {
         const int sz[3] = {im.s0, im.s1, im.s2};
 #pragma unroll
         for (int a = 0; a < D; ++a) ggrid[((size_t)n * D + a) * nP + p] = dfd[a] * (float)(sz[a] - 1);
@@ -1533,7 +1658,7 @@ __device__ __forceinline__ void batch_bwd_item(float* smem, float* acc_base, flo
         for (int i = threadIdx.x; i < WAVES * nCP; i += BLOCK) acc[i] = 0.f;
     const CellTable<D> tab = restage ? stage_tables<D>(smem, static_cast<const float*>(I->ws), g) : table_view<D>(smem, g.nC + g.nV);
     if (!restage) __syncthreads();
-    fused_bwd_tile<D, HAVES>(L, g, s, im, tab, tile, im.data, im.gdata, I->grad_out, I->saved,
+    fused_bwd_tile<D, HAVES, D != 2>(L, g, s, im, tab, tile, im.data, im.gdata, I->grad_out, I->saved,
                              acc + (threadIdx.x >> 6) * nCP, box, box_cap);
     if (run_end) {
         float* part = reinterpret_cast<float*>(static_cast<char*>(I->ws) + align256_hd((size_t)nCP * 4));
@@ -1544,7 +1669,7 @@ __device__ __forceinline__ void batch_bwd_item(float* smem, float* acc_base, flo
 template <bool HAVES, int MAXD>
 // Work items [item_lo, item_hi) (one LDS class of instances, see
 // cpab_batch_plan), pulled from their own queue at counter.
-__global__ __launch_bounds__(BLOCK, MAXD == 2 ? 4 : 1) void k_batch_bwd(const cpab_instance_t* __restrict__ inst,
+__global__ __launch_bounds__(BLOCK, MAXD == 2 ? 4 : 3) void k_batch_bwd(const cpab_instance_t* __restrict__ inst,
                                                      const int* __restrict__ item_inst, int item_lo, int item_hi,
                                                      int ppt, float t_end, int* counter, int acc_offset,
                                                      int box_offset, int box_cap) {
@@ -2458,8 +2583,9 @@ int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_thet
     L.nP = nP;
     L.ppt = pick_ppt_bwd(t->ndim, n_theta, nP, s.g1);
     L.ty = tile_ty(t->ndim, s.g1, s.g2);
-    // 2D with saved state and dL/ddata: accumulate dL/ddata per tile in LDS
-    const int box_cap = (t->ndim == 2 && L.ty > 0 && saved && grad_data &&
+    // 2D with saved state and dL/ddata of up to 4 channels: accumulate dL/ddata
+    // per tile in LDS
+    const int box_cap = (t->ndim == 2 && L.ty > 0 && saved && grad_data && C <= 4 &&
                          lds_bwd(t->ndim, t->nC, t->nC + t->nV) + (size_t)BOX_FLOATS * 4 <= LDS_LIMIT)
                             ? BOX_FLOATS
                             : 0;
@@ -2477,15 +2603,22 @@ int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_thet
     const int tpb = bwd_tiles_per_block(t->ndim, L.ty, n_theta, L.tiles);
     const int nbt = bwd_blocks_per_theta(L.tiles, s.g1, L.ty, tpb);
     dim3 grid(nbt * n_theta);
-#define LAUNCH_DB(DD)                                                                                                     \
-    if (saved)                                                                                                             \
-        hipLaunchKernelGGL((k_transform_data_bwd<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq, grad_out,    \
-                           saved, part, box_cap, tpb);                                                                     \
-    else                                                                                                                   \
-        hipLaunchKernelGGL((k_transform_data_bwd<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq, grad_out,   \
-                           saved, part, 0, tpb);
+    // dL/ddata without the box: the merged scatter ([2, 2, 2], 6 x 2 x 49x40x35:
+    // 114 -> 85 us against an atomic per corner); without dL/ddata its registers
+    // would only cost ([3, 3, 3], 16 x 64^3: 235 -> 257 us)
+    const bool merge = grad_data && !box_cap;
+#define LAUNCH_DB3(DD, HAVES, MERGE)                                                                                  \
+    hipLaunchKernelGGL((k_transform_data_bwd<DD, HAVES, MERGE>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq,     \
+                       grad_out, saved, part, box_cap, tpb)
+#define LAUNCH_DB(DD)                                                                \
+    if (saved) {                                                                     \
+        if (merge) LAUNCH_DB3(DD, true, true); else LAUNCH_DB3(DD, true, false);     \
+    } else {                                                                         \
+        if (merge) LAUNCH_DB3(DD, false, true); else LAUNCH_DB3(DD, false, false);   \
+    }
     CPAB_DISPATCH_D(t->ndim, LAUNCH_DB)
 #undef LAUNCH_DB
+#undef LAUNCH_DB3
     if ((rc = status_from_hip())) return rc;
     return launch_reduce(t, part, n_theta, nbt, grad_theta, nullptr, stream);
 }
