@@ -284,6 +284,18 @@ int cpab_ref_forward(float* newpoints, const float* points, const float* trels, 
 int cpab_ref_backward(float* grad, const float* points, const float* As, const float* Bs, int nstepsolver,
                       const int* nc, int n_theta, int d, int ndim, int nP, int nC, int broadcast, hipStream_t stream);
 
+/* dL/dtheta [n_theta, d] of the same scheme for dL/d(end points) grad_out
+ * [n_theta, ndim, nP]: the sum of cpab_ref_backward's derivatives times
+ * grad_out (libcpab/pytorch/transformer.py:199-202), computed as the adjoint of
+ * the steps without the derivatives.  As [n_theta, nC, ndim, ndim+1] = B theta,
+ * B [nC * ndim * (ndim+1), d].  Workspace from cpab_ref_grad_workspace_bytes,
+ * which is 0 where the tessellation and the step count do not fit a block's LDS
+ * (the call then returns CPAB_ERR_LDS). */
+size_t cpab_ref_grad_workspace_bytes(int ndim, const int* nc, int n_theta, int nP, int nstepsolver);
+int cpab_ref_grad_theta(const float* points, const float* As, const float* B, int nstepsolver, const int* nc,
+                        int n_theta, int d, int ndim, int nP, int broadcast, const float* grad_out, float* grad_theta,
+                        void* workspace, size_t ws_bytes, hipStream_t stream);
+
 /* ---- use_slow: the reference's pure-torch stepping path ------------------ */
 
 /* out [n_theta, ndim, nP] = nstepsolver steps x <- Trel[cell(x)] [x; 1] of

@@ -76,6 +76,9 @@ _SIGNATURES = {
                                     _c_ptr, _c_ptr, _c_ptr]),
     "cpab_ref_backward": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                    _c_int, _c_int, _c_ptr]),
+    "cpab_ref_grad_workspace_bytes": (_c_size, [_c_int, _c_ptr, _c_int, _c_int, _c_int]),
+    "cpab_ref_grad_theta": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                     _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
 }
 
 EXPORTED = tuple(_SIGNATURES)

@@ -1840,8 +1840,9 @@ __global__ __launch_bounds__(BLOCK) void k_ref_forward(float* __restrict__ newpo
     float pt[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) pt[a] = points[(size_t)broadcast * t * nP * D + i + (size_t)a * nP];
+    const float margin = cpab_ref::lookup_margin<D>(nc);
     for (int n = 0; n < nstep; ++n) {
-        const int idx = cpab_ref::find<D>(pt, nc);
+        const int idx = cpab_ref::find<D>(pt, nc, margin);
         float np_[D];
         cpab_ref::affine<D>(np_, sT + P * idx, pt);
 #pragma unroll
@@ -1879,8 +1880,9 @@ __global__ __launch_bounds__(BLOCK) void k_ref_backward(float* __restrict__ grad
         q[a] = 0.f;
     }
     const double h = 1.0 / nstep;
+    const float margin = cpab_ref::lookup_margin<D>(nc);
     for (int s = 0; s < nstep; ++s) {
-        const int cell = cpab_ref::find<D>(p, nc);
+        const int cell = cpab_ref::find<D>(p, nc, margin);
         const float* Al = sA + P * cell;
         const float* Bl = sB + P * cell;
         cpab_ref::affine<D>(v, Al, p);
@@ -1905,6 +1907,155 @@ __global__ __launch_bounds__(BLOCK) void k_ref_backward(float* __restrict__ grad
     const size_t box = (size_t)D * nP * n_theta;
 #pragma unroll
     for (int a = 0; a < D; ++a) grad[(size_t)k * box + (size_t)D * nP * b + i + (size_t)a * nP] = q[a];
+}
+
+// dL/dtheta of the fixed-step scheme, theta_k's derivative q^k contracted with
+// grad_out g without forming any q^k.  In a step with cell map A and basis map
+// B^k of that cell, q' = q + h (B^k pm + A qm), qm = q + h/2 (B^k p + A q), so
+// with lambda carried backwards from g,
+//     mu = A^T lambda,  <g, dq^k> += <h lambda, B^k [pm; 1]> + <h^2/2 mu, B^k [p; 1]>,
+//     lambda <- lambda + h mu + h^2/2 A^T mu:
+// the step adds h lambda [pm; 1]^T + h^2/2 mu [p; 1]^T to the cell's dL/dA, and
+// dL/dtheta = B^T dL/dA once at the end.  The work per point no longer grows
+// with d, and the [d, n_theta, D, nP] derivatives are neither written nor read:
+// [3, 3] (d = 38), 8 thetas x 10000 points x 50 steps, 860 us + 18 us of products
+// and sums -> 67 us + 8 us of reduction, both sides bound by the FP64 chain of
+// the steps (with the FP32-cleared lookup; it took k_ref_forward from 42 to
+// 16 us).
+// lambda and the per-lane sums are FP64 (FP64 multiply-adds issue at the rate of
+// FP32 ones); the points p follow k_ref_backward's steps operation for
+// operation, so the cells are its cells.
+//
+// One wave per block takes 64 points at a time.  The backward sweep needs the
+// points in reverse: the forward sweep keeps every S-th (S ~ sqrt(nstep)), each
+// segment is stepped again into a buffer of S points and walked back; both live
+// in LDS, a column per lane.  A lane sums its cell's dL/dA while it stays in the
+// cell and adds it to the block's accumulator when it leaves (wave sums in a
+// fixed order).  Latency bounds it: at 8 x 10000 points there is about one wave
+// per SIMD.
+template <int D>
+__device__ __forceinline__ void ref_step(const float* A, double h, float (&p)[D], float (&pm)[D]) {
+#pragma clang fp contract(off)
+    float v[D];
+    cpab_ref::affine<D>(v, A, p);
+#pragma unroll
+    for (int a = 0; a < D; ++a) pm[a] = (float)(p[a] + h * v[a] / 2.0);
+}
+template <int D>
+__device__ __forceinline__ void ref_advance(const float* A, double h, float (&p)[D]) {
+#pragma clang fp contract(off)
+    float pm[D], vm[D];
+    ref_step<D>(A, h, p, pm);
+    cpab_ref::affine<D>(vm, A, pm);
+#pragma unroll
+    for (int a = 0; a < D; ++a) p[a] = (float)(p[a] + vm[a] * h);
+}
+
+template <int D>
+__global__ __launch_bounds__(64) void k_ref_grad_theta(const float* __restrict__ points, const float* __restrict__ As,
+                                                       const float* __restrict__ gout, int nstep, int S, int nc0,
+                                                       int nc1, int nc2, int nC, int nP, int broadcast,
+                                                       float* __restrict__ part) {
+    extern __shared__ float smem[];
+    constexpr int P = D * (D + 1);
+    const int b = blockIdx.y, lane = threadIdx.x;
+    const int nseg = (nstep + S - 1) / S;
+    float* sA = smem;
+    float* acc = sA + nC * P;
+    float* start = acc + nC * P;                            // [nseg, D, 64]
+    float* seg = start + nseg * D * 64;                     // [S, D, 64]
+    int* seg_cell = reinterpret_cast<int*>(seg + S * D * 64);  // [S, 64]
+    for (int j = lane; j < nC * P; j += 64) {
+        sA[j] = As[(size_t)b * nC * P + j];
+        acc[j] = 0.f;
+    }
+    __syncthreads();
+    const int nc[3] = {nc0, nc1, nc2};
+    const float margin = cpab_ref::lookup_margin<D>(nc);
+    const double h = 1.0 / nstep, h2 = 0.5 * h * h;
+    for (int i0 = blockIdx.x * 64; i0 < nP; i0 += gridDim.x * 64) {
+        const int i = i0 + lane;
+        const bool valid = i < nP;
+        float p[D];
+        double lam[D], G[P];
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            p[a] = valid ? points[(size_t)broadcast * b * D * nP + i + (size_t)a * nP] : 0.5f;
+            lam[a] = valid ? (double)gout[((size_t)b * D + a) * nP + i] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < P; ++k) G[k] = 0.0;
+        for (int s = 0; s < nseg; ++s) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) start[(s * D + a) * 64 + lane] = p[a];
+            if (s + 1 < nseg)
+                for (int k = 0; k < S; ++k) ref_advance<D>(sA + P * cpab_ref::find<D>(p, nc, margin), h, p);
+        }
+        int cur = -1;
+        for (int s = nseg - 1; s >= 0; --s) {
+            const int n = min(S, nstep - s * S);
+#pragma unroll
+            for (int a = 0; a < D; ++a) p[a] = start[(s * D + a) * 64 + lane];
+            for (int k = 0; k < n; ++k) {
+                const int cell = cpab_ref::find<D>(p, nc, margin);
+                seg_cell[k * 64 + lane] = cell;
+#pragma unroll
+                for (int a = 0; a < D; ++a) seg[(k * D + a) * 64 + lane] = p[a];
+                if (k + 1 < n) ref_advance<D>(sA + P * cell, h, p);
+            }
+            for (int k = n - 1; k >= 0; --k) {
+                const int cell = seg_cell[k * 64 + lane];
+                const bool moved = valid && cur >= 0 && cell != cur;
+                if (__ballot(moved)) {
+                    float Gf[P];
+#pragma unroll
+                    for (int j = 0; j < P; ++j) {
+                        Gf[j] = (float)G[j];
+                        G[j] = moved ? 0.0 : G[j];
+                    }
+                    wave_accumulate<P>(acc, moved ? cur : -1, Gf);
+                }
+                cur = cell;
+                const float* A = sA + P * cell;
+                float pm[D];
+#pragma unroll
+                for (int a = 0; a < D; ++a) p[a] = seg[(k * D + a) * 64 + lane];
+                ref_step<D>(A, h, p, pm);
+                double mu[D], nu[D];
+#pragma unroll
+                for (int c = 0; c < D; ++c) {
+                    double t = 0.0;
+#pragma unroll
+                    for (int r = 0; r < D; ++r) t = fma((double)A[r * (D + 1) + c], lam[r], t);
+                    mu[c] = t;
+                }
+#pragma unroll
+                for (int c = 0; c < D; ++c) {
+                    double t = 0.0;
+#pragma unroll
+                    for (int r = 0; r < D; ++r) t = fma((double)A[r * (D + 1) + c], mu[r], t);
+                    nu[c] = t;
+                }
+#pragma unroll
+                for (int r = 0; r < D; ++r) {
+                    const double hl = h * lam[r], hm = h2 * mu[r];
+#pragma unroll
+                    for (int a = 0; a < D; ++a)
+                        G[r * (D + 1) + a] = fma(hl, (double)pm[a], fma(hm, (double)p[a], G[r * (D + 1) + a]));
+                    G[r * (D + 1) + D] += hl + hm;
+                }
+#pragma unroll
+                for (int r = 0; r < D; ++r) lam[r] = fma(h, mu[r], fma(h2, nu[r], lam[r]));
+            }
+        }
+        float Gf[P];
+#pragma unroll
+        for (int j = 0; j < P; ++j) Gf[j] = (float)G[j];
+        wave_accumulate<P>(acc, valid ? cur : -1, Gf);
+    }
+    __syncthreads();
+    float* row = part + ((size_t)b * gridDim.x + blockIdx.x) * nC * P;
+    for (int j = lane; j < nC * P; j += 64) row[j] = acc[j];
 }
 
 // ---------------------------------------------------------------------------
@@ -2968,6 +3119,68 @@ int cpab_ref_backward(float* grad, const float* points, const float* As, const f
     CPAB_DISPATCH_D(ndim, LAUNCH_RB)
 #undef LAUNCH_RB
     return status_from_hip();
+}
+
+// Launch of k_ref_grad_theta: the kept points' spacing S, the LDS of a block
+// and the blocks per theta (64 points each, about 4096 blocks in all).  0 blocks
+// where a block's LDS would not hold the tables and the 2 sqrt(nstep) points of
+// its lanes.
+static int ref_grad_launch(int ndim, int nC, int n_theta, int nP, int nstep, int& S, size_t& lds) {
+    S = 1;
+    while ((long long)S * S < nstep) ++S;
+    const int nseg = (nstep + S - 1) / S;
+    lds = ((size_t)2 * nC * ndim * (ndim + 1) + (size_t)64 * ((size_t)(nseg + S) * ndim + S)) * 4;
+    if (lds > LDS_LIMIT || n_theta > 65535) return 0;
+    const int chunks = (nP + 63) / 64;
+    const int want = n_theta < 4096 ? 4096 / n_theta : 1;
+    return chunks < want ? chunks : want;
+}
+
+size_t cpab_ref_grad_workspace_bytes(int ndim, const int* nc, int n_theta, int nP, int nstepsolver) {
+    if (ndim < 1 || ndim > 3 || !nc || n_theta < 1 || nP < 1 || nstepsolver < 1) return 0;
+    for (int a = 0; a < ndim; ++a)
+        if (nc[a] < 1) return 0;
+    const int nC = cells_of(ndim, nc);
+    int S;
+    size_t lds;
+    const int blocks = ref_grad_launch(ndim, nC, n_theta, nP, nstepsolver, S, lds);
+    return (size_t)n_theta * blocks * nC * ndim * (ndim + 1) * 4;
+}
+
+int cpab_ref_grad_theta(const float* points, const float* As, const float* B, int nstepsolver, const int* nc,
+                        int n_theta, int d, int ndim, int nP, int broadcast, const float* grad_out, float* grad_theta,
+                        void* workspace, size_t ws_bytes, hipStream_t stream) {
+    if (ndim < 1 || ndim > 3) return CPAB_ERR_NDIM;
+    if (!points || !As || !B || !nc || !grad_out || !grad_theta || nstepsolver < 1 || n_theta < 0 || d < 1 || nP < 1)
+        return CPAB_ERR_ARG;
+    for (int a = 0; a < ndim; ++a)
+        if (nc[a] < 1) return CPAB_ERR_ARG;
+    if (n_theta == 0) return CPAB_OK;
+    const int n0 = nc[0], n1 = ndim > 1 ? nc[1] : 1, n2 = ndim > 2 ? nc[2] : 1;
+    const int nC = cells_of(ndim, nc);
+    int S;
+    size_t lds;
+    const int blocks = ref_grad_launch(ndim, nC, n_theta, nP, nstepsolver, S, lds);
+    if (blocks == 0) return CPAB_ERR_LDS;
+    if (!workspace || ws_bytes < cpab_ref_grad_workspace_bytes(ndim, nc, n_theta, nP, nstepsolver))
+        return CPAB_ERR_WORKSPACE;
+    float* part = static_cast<float*>(workspace);
+    dim3 g(blocks, n_theta);
+#define LAUNCH_RG(DD)                                                                                              \
+    hipLaunchKernelGGL((k_ref_grad_theta<DD>), g, dim3(64), lds, stream, points, As, grad_out, nstepsolver, S, n0, \
+                       n1, n2, nC, nP, broadcast ? 1 : 0, part);
+    CPAB_DISPATCH_D(ndim, LAUNCH_RG)
+#undef LAUNCH_RG
+    int rc = status_from_hip();
+    if (rc) return rc;
+    // As is in x-space: the reduction's scale from q-space is 1 for one cell per axis
+    cpab_tess_t t = {};
+    t.ndim = ndim;
+    t.nc[0] = t.nc[1] = t.nc[2] = 1;
+    t.nC = nC;
+    t.d = d;
+    t.B = B;
+    return launch_reduce(&t, part, n_theta, blocks, grad_theta, nullptr, stream);
 }
 
 int cpab_slow_forward(const float* points, const float* trels, int nstepsolver, const int* nc, int ndim, int nP,

@@ -8,7 +8,9 @@
 // cell lookup and RK2 half steps, no fused multiply-adds: contraction is off
 // in this file), so results match the reference's compiled CPU op bit for bit
 // on the same Trels.  One thread per (point, theta) in the forward and per
-// (point, theta, k) in the backward, as the work decomposes in the reference.
+// (point, theta, k) in the backward, as the work decomposes in the reference;
+// dL/dtheta itself comes from the adjoint of those steps instead
+// (k_ref_grad_theta), whose work does not grow with the number of k.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -98,11 +100,63 @@ __device__ __forceinline__ int find3(const float* pin, int nx, int ny, int nz) {
     return cell;
 }
 
+// The same cells where a point is clear of every facet: scaled coordinates in
+// FP32 decide, and the FP64 lookup above (whose remainders and quotients cost
+// ten times as much) runs only for lanes within `m` of a facet or of the
+// domain's boundary.  The scaled coordinates differ from the lookup's by at most
+// 2^-23 n per axis of n cells (one rounding of the product, one of the cell
+// width); m is 30 times the sum over the axes that a facet function adds up.
 template <int D>
-__device__ __forceinline__ int find(const float* p, const int* nc) {
+__device__ __forceinline__ float lookup_margin(const int* nc) {
+    float n = 4.f;
+#pragma unroll
+    for (int a = 0; a < D; ++a) n += (float)nc[a];
+    return 4e-6f * n;
+}
+// scaled coordinate's cell and the place in it; false within m of either face
+__device__ __forceinline__ bool clear_axis(float p, int n, float m, int& i, float& x) {
+    const float u = p * (float)n, f = floorf(u);
+    i = (int)f;
+    x = u - f;
+    return x > m && 1.f - x > m && f >= 0.f && f < (float)n;
+}
+
+__device__ __forceinline__ int find2_fast(const float* p, int nx, int ny, float m) {
+    int i, j;
+    float x, y;
+    bool ok = clear_axis(p[0], nx, m, i, x);
+    ok = clear_axis(p[1], ny, m, j, y) && ok;
+    ok = ok && fabsf(x - y) > m && fabsf(1.f - x - y) > m;
+    int cell = 4 * (i + j * nx) + (x < y ? (1.f - x < y ? 2 : 3) : (1.f - x < y ? 1 : 0));
+    if (!ok) cell = find2(p, nx, ny);
+    return cell;
+}
+
+__device__ __forceinline__ int find3_fast(const float* p, int nx, int ny, int nz, float m) {
+    int i, j, k;
+    float x, y, z;
+    bool ok = clear_axis(p[0], nx, m, i, x);
+    ok = clear_axis(p[1], ny, m, j, y) && ok;
+    ok = clear_axis(p[2], nz, m, k, z) && ok;
+    // the lookup bounds z by nz / nx
+    ok = ok && p[2] * (float)nx < (float)nz - m;
+    if ((i + j + k) & 1) {
+        const float t = x;
+        x = y;
+        y = 1.f - t;
+    }
+    const float f1 = z - x - y, f2 = x + y + z - 2.f, f3 = y - x - z, f4 = x - y - z;
+    ok = ok && fminf(fminf(fabsf(f1), fabsf(f2)), fminf(fabsf(f3), fabsf(f4))) > m;
+    int cell = 5 * (i + j * nx + k * nx * ny) + (f1 > 0.f ? 1 : f2 > 0.f ? 2 : f3 > 0.f ? 3 : f4 > 0.f ? 4 : 0);
+    if (!ok) cell = find3(p, nx, ny, nz);
+    return cell;
+}
+
+template <int D>
+__device__ __forceinline__ int find(const float* p, const int* nc, float m) {
     if constexpr (D == 1) return find1(p, nc[0]);
-    else if constexpr (D == 2) return find2(p, nc[0], nc[1]);
-    else return find3(p, nc[0], nc[1], nc[2]);
+    else if constexpr (D == 2) return find2_fast(p, nc[0], nc[1], m);
+    else return find3_fast(p, nc[0], nc[1], nc[2], m);
 }
 
 // x = A b~ (A row-major D x (D+1)), evaluated left to right like the reference

@@ -3,8 +3,8 @@
 Trels = expm(A~ / nstepsolver) per cell (libcpab/pytorch/transformer.py:146-155),
 nstepsolver steps of the cell-local Trel (libcpab/core/cpab_ops.cpp:224-260)
 and, for the gradient, the midpoint-RK2 sensitivity integration
-(libcpab/core/cpab_ops.cpp:262-372) followed by the reduction of
-libcpab/pytorch/transformer.py:199-202.  Like the reference, the analytic
+(libcpab/core/cpab_ops.cpp:262-372) with the reduction of
+libcpab/pytorch/transformer.py:199-202, as the adjoint of its steps.  Like the reference, the analytic
 backward returns no gradient w.r.t. the points.  numeric_grad=True gives the
 finite-difference gradient the reference intended
 (libcpab/pytorch/transformer.py:205-295, which does not run as written).
@@ -64,12 +64,24 @@ class NumericAnalyticGrad(torch.autograd.Function):
         p = ctx.params
         dev = H.device_tess(p, theta.device)
         n_theta, nP = theta.shape[0], points.shape[-1]
+        grad = grad.contiguous()
+        nc, nstep = H._int_arr(p.nc), int(p.nstepsolver)
+        nb = int(N.lib().cpab_ref_grad_workspace_bytes(p.ndim, nc, n_theta, nP, nstep))
+        if nb:
+            gtheta = torch.empty_like(theta)
+            ws = torch.empty(nb, device=theta.device, dtype=torch.uint8)
+            N.check(N.lib().cpab_ref_grad_theta(H._ptr(points), H._ptr(As), H._ptr(dev.B), nstep, nc, n_theta, dev.d,
+                                                p.ndim, nP, ctx.broadcast, H._ptr(grad), H._ptr(gtheta),
+                                                H._ptr(ws), nb, H._stream(theta.device)))
+            return None, gtheta, None
+        # too many cells or steps for a block's LDS (or an empty problem): every
+        # derivative on its own
         Bs = dev.B.t().contiguous()  # [d, D] = [d, nC, ndim, ndim+1]
         J = torch.empty(dev.d, n_theta, p.ndim, nP, device=theta.device, dtype=torch.float32)
         N.check(N.lib().cpab_ref_backward(H._ptr(J), H._ptr(points), H._ptr(As.contiguous()), H._ptr(Bs),
                                           int(p.nstepsolver), H._int_arr(p.nc), n_theta, dev.d, p.ndim, nP, p.nC,
                                           ctx.broadcast, H._stream(theta.device)))
-        g = J.mul_(grad.contiguous()).sum(dim=(2, 3))
+        g = J.mul_(grad).sum(dim=(2, 3))
         return None, g.t(), None
 
 
