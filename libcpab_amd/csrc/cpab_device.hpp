@@ -723,30 +723,55 @@ CPAB_HD __forceinline__ void replay(PointState<D>& st, const CellTable<D>& tab, 
 // ---------------------------------------------------------------------------
 // 1D: closed form
 // ---------------------------------------------------------------------------
-CPAB_HD __forceinline__ float phi1(float z) {  // (e^z - 1)/z
-    return (fabsf(z) < 1e-4f) ? fmaf(z, fmaf(z, 1.0f / 6.0f, 0.5f), 1.0f) : expm1f(z) / z;
+//
+// Instruction bound like the others: 2.7 chunks per wave and point on 1024-point
+// signals over 50 cells.  The library's expm1, log1p and the quotients were most
+// of them, so phi1, phi2 and the exponential come from one Taylor sum for
+// |z| <= 1 (nearly every chunk), the growth of a chunk that ends on a cell edge
+// is the velocity ratio 1 + r, and log1p(r)/r is the hardware logarithm of
+// u = 1 + r over u - 1 (the rounding of u enters both, so it cancels; measured
+// error 2.8e-7 at most over |r| = 1e-5 .. 1e3 and r > -1, 6e-8 on average).
+// us per launch, 4096 signals of 1024 points, before / after: forward 75 / 35,
+// backward 116 / 67.
+// ---------------------------------------------------------------------------
+// 1/x to ~0.5 ulp
+CPAB_HD __forceinline__ float near_rcp(float x) {
+    const float r = fast_rcp(x);
+    return fmaf(fmaf(-x, r, 1.f), r, r);
 }
-CPAB_HD __forceinline__ float phi2(float z) {  // (e^z - 1 - z)/z^2
-    if (fabsf(z) < 0.5f) {
-        float acc = 1.0f / 3628800.0f;  // 1/10!
-        acc = fmaf(acc, z, 1.0f / 362880.0f);
-        acc = fmaf(acc, z, 1.0f / 40320.0f);
-        acc = fmaf(acc, z, 1.0f / 5040.0f);
-        acc = fmaf(acc, z, 1.0f / 720.0f);
-        acc = fmaf(acc, z, 1.0f / 120.0f);
-        acc = fmaf(acc, z, 1.0f / 24.0f);
-        acc = fmaf(acc, z, 1.0f / 6.0f);
-        acc = fmaf(acc, z, 0.5f);
-        return acc;
+// e^z, p1 = (e^z - 1)/z, p2 = (e^z - 1 - z)/z^2
+CPAB_HD __forceinline__ void exp_phis(float z, float& e, float& p1, float& p2) {
+    if (fabsf(z) <= 1.f) {
+        // sum_k z^k/(k+2)!, k < 10: the next term is below 1/12! = 2.1e-9
+        constexpr float C[10] = {1.f / 2,    1.f / 6,     1.f / 24,     1.f / 120,     1.f / 720,
+                                 1.f / 5040, 1.f / 40320, 1.f / 362880, 1.f / 3628800, 1.f / 39916800};
+        float acc = C[9];
+#pragma unroll
+        for (int k = 8; k >= 0; --k) acc = fmaf(acc, z, C[k]);
+        p2 = acc;
+        p1 = fmaf(z, acc, 1.f);
+        e = fmaf(z, p1, 1.f);
+    } else {
+        const float em = expm1f(z);
+        e = expf(z);
+        p1 = em / z;
+        p2 = (em - z) / (z * z);
     }
-    return (expm1f(z) - z) / (z * z);
 }
-CPAB_HD __forceinline__ float log1p_over(float r) {  // log1p(r)/r
-    return (fabsf(r) < 1e-4f) ? fmaf(r, fmaf(r, 1.0f / 3.0f, -0.5f), 1.0f) : log1pf(r) / r;
+// log1p(r)/r for r > -1
+CPAB_HD __forceinline__ float log1p_over(float r) {
+    const float u = 1.f + r, d = u - 1.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float l = __builtin_amdgcn_logf(u);
+#else
+    const float l = log2f(u);
+#endif
+    return d == 0.f ? fmaf(r, -0.5f, 1.f) : l * 0.69314718055994531f * fast_rcp(d);
 }
 
 struct Chunk1 {
     float a, b, q0, v0, h;
+    float grow;  // e^(a h)
     int cell, facet, next;
     float q1;
 };
@@ -756,41 +781,49 @@ CPAB_HD __forceinline__ void advance1(PointState<1>& st, const CellTable<1>& tab
     const float a = tab.A[2 * c], b = tab.A[2 * c + 1];
     const float q0 = st.q[0];
     const float v0 = fmaf(a, q0, b);
-    float step = st.T;
+    float step = st.T, grow = 1.f;
     int facet = -1, next = c;
-    if (v0 != 0.f) {
-        const bool right = v0 > 0.f;
-        const int nbc = right ? c + 1 : c - 1;
-        if (nbc >= 0 && nbc < nx) {
-            const float qb = right ? (float)(c + 1) : (float)c;
-            const float dq = qb - q0;
-            const float r = a * dq / v0;
-            if (1.0f + r > 0.f) {
-                float th = (dq / v0) * log1p_over(r);
-                th = fmaxf(th, 0.f);
-                bool back = (st.zero_hops > 0 && nbc == st.came_from && th <= ZERO_HOP);
-                if (th < st.T && !back) {
-                    step = th;
-                    facet = right ? 1 : 0;
-                    next = nbc;
-                }
+    const bool right = v0 > 0.f;
+    const int nbc = right ? c + 1 : c - 1;
+    const float qb = right ? (float)(c + 1) : (float)c;
+    if (v0 != 0.f && nbc >= 0 && nbc < nx) {
+        const float dt = (qb - q0) * near_rcp(v0);
+        const float r = a * dt;
+        if (1.0f + r > 0.f) {
+            const float th = fmaxf(dt * log1p_over(r), 0.f);
+            const bool back = (st.zero_hops > 0 && nbc == st.came_from && th <= ZERO_HOP);
+            if (th < st.T && !back) {
+                step = th;
+                grow = 1.0f + r;
+                facet = right ? 1 : 0;
+                next = nbc;
             }
         }
     }
     ch.a = a; ch.b = b; ch.q0 = q0; ch.v0 = v0; ch.h = step;
     ch.cell = c; ch.facet = facet; ch.next = next;
     if (facet >= 0) {
-        ch.q1 = (facet == 1) ? (float)(c + 1) : (float)c;
+        ch.q1 = qb;
         st.T = fmaxf(st.T - step, 0.f);
         st.zero_hops = (step <= ZERO_HOP) ? st.zero_hops + 1 : 0;
         st.came_from = c;
         st.c = next;
     } else {
-        ch.q1 = fmaf(step * phi1(a * step), v0, q0);
+        float p1, p2;
+        exp_phis(a * step, grow, p1, p2);
+        ch.q1 = fmaf(step * p1, v0, q0);
         st.T = 0.f;
     }
+    ch.grow = grow;
     st.q[0] = ch.q1;
     st.iters++;
+}
+
+// The saltation factor v_next / v_prev of a crossing (1 for a continuous field;
+// formed as 1 + difference, which keeps it exact there), or its inverse for the
+// adjoint; 1 where the divisor vanishes beside the other.
+CPAB_HD __forceinline__ float saltation1(float vnum, float vden) {
+    return fabsf(vden) > 1e-6f * fabsf(vnum) && vden != 0.f ? fmaf(vnum - vden, near_rcp(vden), 1.f) : 1.f;
 }
 
 // ---------------------------------------------------------------------------
@@ -985,11 +1018,11 @@ CPAB_HD __forceinline__ void step_point(PointState<D>& st, const CellTable<D>& t
         Chunk1 ch;
         advance1(st, tab, nx, ch);
         if constexpr (WITHJ) {
-            J[0][0] *= expf(ch.a * ch.h);
+            J[0][0] *= ch.grow;
             if (ch.facet >= 0) {
                 const float vn = fmaf(tab.A[2 * ch.next], ch.q1, tab.A[2 * ch.next + 1]);
                 const float vp = fmaf(ch.a, ch.q1, ch.b);
-                if (fabsf(vp) > 1e-6f * fabsf(vn) && vp != 0.f) J[0][0] *= vn / vp;
+                J[0][0] *= saltation1(vn, vp);
             }
         }
     } else {
@@ -1180,10 +1213,11 @@ CPAB_HD __forceinline__ void chunk_grad(const Chunk<D>& ch, float (&mu)[D], floa
 }
 
 CPAB_HD __forceinline__ void chunk_grad1(const Chunk1& ch, float& mu, float (&G)[2]) {
-    const float z = -ch.a * ch.h;
-    G[0] = mu * fmaf(ch.h * ch.h, ch.b * phi2(z), ch.q0 * ch.h);
-    G[1] = mu * ch.h * phi1(z);
-    mu *= expf(z);
+    float e, p1, p2;
+    exp_phis(-ch.a * ch.h, e, p1, p2);
+    G[0] = mu * fmaf(ch.h * ch.h, ch.b * p2, ch.q0 * ch.h);
+    G[1] = mu * ch.h * p1;
+    mu *= e;
 }
 
 // ---------------------------------------------------------------------------

@@ -325,7 +325,7 @@ __device__ __forceinline__ void pass2(bool valid, const float (&q0)[D], int c0, 
                 if (ch.facet >= 0) {
                     const float vn = fmaf(tab.A[2 * ch.next], ch.q1, tab.A[2 * ch.next + 1]);
                     const float vp = fmaf(ch.a, ch.q1, ch.b);
-                    if (fabsf(vn) > 1e-6f * fabsf(vp) && vn != 0.f) mu[0] *= vp / vn;
+                    mu[0] *= saltation1(vp, vn);
                 }
             } else {
                 Chunk<D> ch;
