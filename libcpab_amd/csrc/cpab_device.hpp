@@ -725,14 +725,17 @@ CPAB_HD __forceinline__ void replay(PointState<D>& st, const CellTable<D>& tab, 
 // ---------------------------------------------------------------------------
 //
 // Instruction bound like the others: 2.7 chunks per wave and point on 1024-point
-// signals over 50 cells.  The library's expm1, log1p and the quotients were most
-// of them, so phi1, phi2 and the exponential come from one Taylor sum for
-// |z| <= 1 (nearly every chunk), the growth of a chunk that ends on a cell edge
-// is the velocity ratio 1 + r, and log1p(r)/r is the hardware logarithm of
-// u = 1 + r over u - 1 (the rounding of u enters both, so it cancels; measured
-// error 2.8e-7 at most over |r| = 1e-5 .. 1e3 and r > -1, 6e-8 on average).
-// us per launch, 4096 signals of 1024 points, before / after: forward 75 / 35,
-// backward 116 / 67.
+// signals over 50 cells, most of it the library's expm1, log1p and exp and IEEE
+// quotients.  The growth of a chunk that ends on a cell edge is the velocity
+// ratio 1 + r, and the final chunk's comes with its phi1.  The gradient's pass
+// (EXACT = false) takes phi1, phi2 and e^z from one Taylor sum for |z| <= 1
+// (nearly every chunk) and log1p(r)/r as the hardware logarithm of u = 1 + r over
+// u - 1 (the rounding of u enters both, so it cancels; measured error 2.8e-7 at
+// most over |r| = 1e-5 .. 1e3 and r > -1, 6e-8 on average).  The positions
+// themselves (EXACT) keep the library's functions operation for operation: one
+// rounding of q is a thousandth of a sample on a signal of 8192, and an
+// interpolation weight's whole error.  us per launch, 4096 signals of 1024
+// points, before / after: forward 75 / 66, backward 116 / 68.
 // ---------------------------------------------------------------------------
 // 1/x to ~0.5 ulp
 CPAB_HD __forceinline__ float near_rcp(float x) {
@@ -759,7 +762,7 @@ CPAB_HD __forceinline__ void exp_phis(float z, float& e, float& p1, float& p2) {
     }
 }
 // log1p(r)/r for r > -1
-CPAB_HD __forceinline__ float log1p_over(float r) {
+CPAB_HD __forceinline__ float log1p_over_fast(float r) {
     const float u = 1.f + r, d = u - 1.f;
 #if defined(__HIP_DEVICE_COMPILE__)
     const float l = __builtin_amdgcn_logf(u);
@@ -768,54 +771,85 @@ CPAB_HD __forceinline__ float log1p_over(float r) {
 #endif
     return d == 0.f ? fmaf(r, -0.5f, 1.f) : l * 0.69314718055994531f * fast_rcp(d);
 }
+CPAB_HD __forceinline__ float phi1(float z) {  // (e^z - 1)/z
+    return (fabsf(z) < 1e-4f) ? fmaf(z, fmaf(z, 1.0f / 6.0f, 0.5f), 1.0f) : expm1f(z) / z;
+}
+CPAB_HD __forceinline__ float log1p_over(float r) {  // log1p(r)/r
+    return (fabsf(r) < 1e-4f) ? fmaf(r, fmaf(r, 1.0f / 3.0f, -0.5f), 1.0f) : log1pf(r) / r;
+}
+
+// The point's cell map and whether it crosses the edge qb it moves towards in
+// the time left: after th, into cell next, grown by e^(a th) = 1 + r.
+struct Hit1 {
+    float a, b, v0, qb, th, r;
+    int next;
+    bool right, crosses;
+};
+template <bool EXACT>
+CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& tab, int nx) {
+    Hit1 h;
+    const int c = st.c;
+    const float q0 = st.q[0];
+    h.a = tab.A[2 * c];
+    h.b = tab.A[2 * c + 1];
+    h.v0 = fmaf(h.a, q0, h.b);
+    h.right = h.v0 > 0.f;
+    h.next = h.right ? c + 1 : c - 1;
+    h.qb = h.right ? (float)(c + 1) : (float)c;
+    h.th = 0.f;
+    h.r = 0.f;
+    h.crosses = false;
+    if (h.v0 != 0.f && h.next >= 0 && h.next < nx) {
+        const float dq = h.qb - q0;
+        const float dt = EXACT ? dq / h.v0 : dq * near_rcp(h.v0);
+        h.r = EXACT ? h.a * dq / h.v0 : h.a * dt;
+        if (1.0f + h.r > 0.f) {
+            h.th = fmaxf(dt * (EXACT ? log1p_over(h.r) : log1p_over_fast(h.r)), 0.f);
+            const bool back = (st.zero_hops > 0 && h.next == st.came_from && h.th <= ZERO_HOP);
+            h.crosses = h.th < st.T && !back;
+        }
+    }
+    return h;
+}
+CPAB_HD __forceinline__ void hop1(PointState<1>& st, const Hit1& h) {
+    st.T = fmaxf(st.T - h.th, 0.f);
+    st.zero_hops = (h.th <= ZERO_HOP) ? st.zero_hops + 1 : 0;
+    st.came_from = st.c;
+    st.c = h.next;
+    st.q[0] = h.qb;
+}
+// The last chunk: the time left, inside the cell; returns e^(a T).
+template <bool EXACT>
+CPAB_HD __forceinline__ float end1(PointState<1>& st, const Hit1& h) {
+    const float z = h.a * st.T;
+    float grow, p1, p2;
+    if (EXACT) {
+        p1 = phi1(z);
+        grow = z > -1.f ? fmaf(z, p1, 1.f) : expf(z);  // 1 + (e^z - 1) cancels below
+    } else {
+        exp_phis(z, grow, p1, p2);
+    }
+    st.q[0] = fmaf(st.T * p1, h.v0, st.q[0]);
+    st.T = 0.f;
+    return grow;
+}
 
 struct Chunk1 {
-    float a, b, q0, v0, h;
-    float grow;  // e^(a h)
+    float a, b, q0, h;
     int cell, facet, next;
     float q1;
 };
-
+template <bool EXACT>
 CPAB_HD __forceinline__ void advance1(PointState<1>& st, const CellTable<1>& tab, int nx, Chunk1& ch) {
-    const int c = st.c;
-    const float a = tab.A[2 * c], b = tab.A[2 * c + 1];
-    const float q0 = st.q[0];
-    const float v0 = fmaf(a, q0, b);
-    float step = st.T, grow = 1.f;
-    int facet = -1, next = c;
-    const bool right = v0 > 0.f;
-    const int nbc = right ? c + 1 : c - 1;
-    const float qb = right ? (float)(c + 1) : (float)c;
-    if (v0 != 0.f && nbc >= 0 && nbc < nx) {
-        const float dt = (qb - q0) * near_rcp(v0);
-        const float r = a * dt;
-        if (1.0f + r > 0.f) {
-            const float th = fmaxf(dt * log1p_over(r), 0.f);
-            const bool back = (st.zero_hops > 0 && nbc == st.came_from && th <= ZERO_HOP);
-            if (th < st.T && !back) {
-                step = th;
-                grow = 1.0f + r;
-                facet = right ? 1 : 0;
-                next = nbc;
-            }
-        }
-    }
-    ch.a = a; ch.b = b; ch.q0 = q0; ch.v0 = v0; ch.h = step;
-    ch.cell = c; ch.facet = facet; ch.next = next;
-    if (facet >= 0) {
-        ch.q1 = qb;
-        st.T = fmaxf(st.T - step, 0.f);
-        st.zero_hops = (step <= ZERO_HOP) ? st.zero_hops + 1 : 0;
-        st.came_from = c;
-        st.c = next;
-    } else {
-        float p1, p2;
-        exp_phis(a * step, grow, p1, p2);
-        ch.q1 = fmaf(step * p1, v0, q0);
-        st.T = 0.f;
-    }
-    ch.grow = grow;
-    st.q[0] = ch.q1;
+    const Hit1 h = hit1<EXACT>(st, tab, nx);
+    ch.a = h.a; ch.b = h.b; ch.q0 = st.q[0];
+    ch.cell = st.c;
+    ch.h = h.crosses ? h.th : st.T;
+    ch.facet = h.crosses ? (h.right ? 1 : 0) : -1;
+    ch.next = h.crosses ? h.next : st.c;
+    if (h.crosses) hop1(st, h);
+    else end1<EXACT>(st, h);
+    ch.q1 = st.q[0];
     st.iters++;
 }
 
@@ -1009,36 +1043,24 @@ CPAB_HD __forceinline__ bool point_active(const PointState<D>& st) {
     return st.T > 0.f && st.iters < MAX_ITERS;
 }
 
-// One chunk of pass 1: advance the point and carry J = dq(T)/dq0; with LOG
-// (2D/3D) the chunk goes into lg (a ChunkLog or a LogSink).
+// One chunk of pass 1 (2D/3D): advance the point and carry J = dq(T)/dq0; with
+// LOG the chunk goes into lg (a ChunkLog or a LogSink).
 template <int D, bool WITHJ, bool LOG = false, class Log = ChunkLog>
 CPAB_HD __forceinline__ void step_point(PointState<D>& st, const CellTable<D>& tab, int nx, float tol0,
                                         float (&J)[D][D], Log& lg) {
-    if constexpr (D == 1) {
-        Chunk1 ch;
-        advance1(st, tab, nx, ch);
-        if constexpr (WITHJ) {
-            J[0][0] *= ch.grow;
-            if (ch.facet >= 0) {
-                const float vn = fmaf(tab.A[2 * ch.next], ch.q1, tab.A[2 * ch.next + 1]);
-                const float vp = fmaf(ch.a, ch.q1, ch.b);
-                J[0][0] *= saltation1(vn, vp);
-            }
-        }
-    } else {
-        Chunk<D> ch;
-        advance<D>(st, tab, tol0, ch);
-        if constexpr (WITHJ) {
-            carry_jacobian<D>(ch, J);
-            if (ch.facet >= 0) saltation_fwd<D>(tab, ch, J);
-        }
-        // logged last, when the chunk's temporaries are dead
-        if constexpr (LOG) {
-            if constexpr (std::is_same<Log, LogSink>::value)
-                sink_chunk(lg, st.iters - 1, ch.h, ch.facet);
-            else
-                log_chunk(lg, ch.h, ch.facet);
-        }
+    static_assert(D > 1, "integrate carries 1D points itself");
+    Chunk<D> ch;
+    advance<D>(st, tab, tol0, ch);
+    if constexpr (WITHJ) {
+        carry_jacobian<D>(ch, J);
+        if (ch.facet >= 0) saltation_fwd<D>(tab, ch, J);
+    }
+    // logged last, when the chunk's temporaries are dead
+    if constexpr (LOG) {
+        if constexpr (std::is_same<Log, LogSink>::value)
+            sink_chunk(lg, st.iters - 1, ch.h, ch.facet);
+        else
+            log_chunk(lg, ch.h, ch.facet);
     }
 }
 
@@ -1048,6 +1070,32 @@ CPAB_HD __forceinline__ void identity(float (&J)[D][D]) {
     for (int r = 0; r < D; ++r)
 #pragma unroll
         for (int k = 0; k < D; ++k) J[r][k] = (r == k) ? 1.f : 0.f;
+}
+
+// A point that used up MAX_ITERS with time left: NaN, and counted.
+template <int D, bool WITHJ>
+CPAB_HD __forceinline__ void give_up(PointState<D>& st, float (&J)[D][D], int* unfinished) {
+    const float nan = __builtin_nanf("");
+    st.T = 0.f;
+#pragma unroll
+    for (int a = 0; a < D; ++a) st.q[a] = nan;
+    if constexpr (WITHJ) {
+#pragma unroll
+        for (int r = 0; r < D; ++r)
+#pragma unroll
+            for (int k = 0; k < D; ++k) J[r][k] = nan;
+    }
+    if (unfinished) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        // the operand is made opaque so that its register is set here, on the
+        // rare path, and not hoisted out of the loop
+        int one = 1;
+        asm volatile("" : "+v"(one));
+        atomicAdd(unfinished, one);
+#else
+        ++*unfinished;
+#endif
+    }
 }
 
 // Integrate one point for time T (pass 1 if WITHJ); with LOG its first NREC
@@ -1062,30 +1110,32 @@ CPAB_HD __forceinline__ void integrate(float (&q)[D], int c0, float T, const Cel
     init_point<D>(st, q, c0, T);
     if constexpr (WITHJ) identity<D>(J);
     lg.code = 0;
-    while (st.T > 0.f) {
-        step_point<D, WITHJ, LOG, Log>(st, tab, nx, tol0, J, lg);
-        if (st.iters >= MAX_ITERS && st.T > 0.f) {
-            const float nan = __builtin_nanf("");
-            st.T = 0.f;
-#pragma unroll
-            for (int a = 0; a < D; ++a) st.q[a] = nan;
+    if constexpr (D == 1) {
+        // the last chunk after the loop: its exponential runs once for all lanes,
+        // whichever crossing each of them stopped after
+        Hit1 h;
+        bool last = false;
+        while (st.T > 0.f) {
+            h = hit1<true>(st, tab, nx);
+            last = !h.crosses;
+            if (last) break;
+            hop1(st, h);
+            st.iters++;
             if constexpr (WITHJ) {
-#pragma unroll
-                for (int r = 0; r < D; ++r)
-#pragma unroll
-                    for (int k = 0; k < D; ++k) J[r][k] = nan;
+                const float vn = fmaf(tab.A[2 * st.c], h.qb, tab.A[2 * st.c + 1]);
+                const float vp = fmaf(h.a, h.qb, h.b);
+                J[0][0] *= (1.f + h.r) * saltation1(vn, vp);
             }
-            if (unfinished) {
-#if defined(__HIP_DEVICE_COMPILE__)
-                // the operand is made opaque so that its register is set here,
-                // on the rare path, and not hoisted out of the loop
-                int one = 1;
-                asm volatile("" : "+v"(one));
-                atomicAdd(unfinished, one);
-#else
-                ++*unfinished;
-#endif
-            }
+            if (st.iters >= MAX_ITERS && st.T > 0.f) give_up<D, WITHJ>(st, J, unfinished);
+        }
+        if (last) {
+            const float grow = end1<true>(st, h);
+            if constexpr (WITHJ) J[0][0] *= grow;
+        }
+    } else {
+        while (st.T > 0.f) {
+            step_point<D, WITHJ, LOG, Log>(st, tab, nx, tol0, J, lg);
+            if (st.iters >= MAX_ITERS && st.T > 0.f) give_up<D, WITHJ>(st, J, unfinished);
         }
     }
 #pragma unroll

@@ -316,7 +316,7 @@ __device__ __forceinline__ void pass2(bool valid, const float (&q0)[D], int c0, 
         if (active) {
             if constexpr (D == 1) {
                 Chunk1 ch;
-                advance1(st, tab, g.nc0, ch);
+                advance1<false>(st, tab, g.nc0, ch);
                 float G1[2];
                 chunk_grad1(ch, mu[0], G1);
                 G[0] = G1[0];
@@ -798,7 +798,7 @@ __global__ __launch_bounds__(BLOCK) void k_transform_cells(Launch L, Geo g, Src 
             float h;
             if constexpr (D == 1) {
                 Chunk1 ch;
-                advance1(st, tab, g.nc0, ch);
+                advance1<true>(st, tab, g.nc0, ch);
                 cell = ch.cell;
                 facet = ch.facet;
                 h = ch.h;
