@@ -1328,144 +1328,128 @@ __global__ __launch_bounds__(BLOCK) void k_interp_bwd(int N, int nP, Src s, Img 
     }
 }
 
-// per theta: dL/dA (x-space) = sum over tiles of the q-space partials, scaled
-// back; dL/dtheta = B^T dL/dA.  One block of nw = blockDim.x / 64 waves per
-// theta (memory-bound: many waves keep loads in flight); every sum runs in a
-// fixed order.
+// dL/dtheta of each theta from its rows of partials (q-space dL/dA): the rows
+// are summed and scaled to x-space, then B^T is applied.  Every sum runs in a
+// fixed order: wave w of nw takes rows w, w + nw, ... in two chains, the wave
+// sums are added in wave order, and likewise for B's rows.
 constexpr int RBLOCK = 1024;
-// dL/dtheta of one theta from its tile partials pp [tiles, Dt] (q-space
-// dL/dA): the block's waves sum the tiles, the wave sums are added in wave
-// order, scaled to x-space (gA, nullable, receives dL/dA), and B^T dL/dA is
-// split over the waves by rows of B and added in wave order.  sg holds
-// [nw + 1, Dt] floats.
-// Row j of the partials that reduce_theta sums (j < its row count).
+constexpr int R_COLS = 64;  // columns per block of the sliced kernels
+
+// Row j of the partials (j < the row count).
 struct AllRows {
     __device__ __forceinline__ int operator()(int j) const { return j; }
 };
 
-template <class Rows = AllRows>
-__device__ __forceinline__ void reduce_theta(float* sg, const float* __restrict__ pp, int tiles, int Dt, int ndim,
-                                             const int (&nc)[3], const float* __restrict__ B, int d,
-                                             float* __restrict__ gth, float* __restrict__ gA, Rows rows = Rows()) {
-    const int nw = blockDim.x >> 6;
-    const int P = ndim * (ndim + 1);
-    // wave w sums tiles w, w + nw, ... (two chains for overlap)
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int i = lane; i < Dt; i += 64) {
-        float s0 = 0.f, s1 = 0.f;
-        int t = w;
-        for (; t + nw < tiles; t += 2 * nw) {
-            s0 += pp[(size_t)rows(t) * Dt + i];
-            s1 += pp[(size_t)rows(t + nw) * Dt + i];
-        }
-        if (t < tiles) s0 += pp[(size_t)rows(t) * Dt + i];
-        sg[w * Dt + i] = s0 + s1;
+// this wave's share of column i
+template <class Rows>
+__device__ __forceinline__ float rows_sum(const float* __restrict__ pp, int nrows, int Dt, int i, int w, int nw,
+                                          Rows rows) {
+    float s0 = 0.f, s1 = 0.f;
+    int t = w;
+    for (; t + nw < nrows; t += 2 * nw) {
+        s0 += pp[(size_t)rows(t) * Dt + i];
+        s1 += pp[(size_t)rows(t + nw) * Dt + i];
     }
-    __syncthreads();
-    float* sA = sg + nw * Dt;
-    for (int i = threadIdx.x; i < Dt; i += blockDim.x) {
-        float s = sg[i];
-        for (int k = 1; k < nw; ++k) s += sg[k * Dt + i];
-        const int rem = i % P, r = rem / (ndim + 1), col = rem % (ndim + 1);
-        const float sc = (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
-        s *= sc;
-        sA[i] = s;
-        if (gA) gA[i] = s;
+    if (t < nrows) s0 += pp[(size_t)rows(t) * Dt + i];
+    return s0 + s1;
+}
+__device__ __forceinline__ float x_scale(int i, int ndim, const int (&nc)[3]) {
+    const int rem = i % (ndim * (ndim + 1)), r = rem / (ndim + 1), col = rem % (ndim + 1);
+    return (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
+}
+// this wave's share of (B^T sA)[k]: rows [i0, i1) of B, 16 loads in flight (the
+// last piece's missing rows count as 0 instead of being walked one by one)
+__device__ __forceinline__ float bt_sum(const float* __restrict__ B, const float* sA, int d, int k, int i0, int i1) {
+    float s = 0.f;
+    for (int i = i0; i < i1; i += 16) {
+        float b[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) b[u] = i + u < i1 ? B[(size_t)(i + u) * d + k] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            if (i + u < i1) s = fmaf(b[u], sA[i + u], s);
     }
-    __syncthreads();
-    // B^T dL/dA: wave w takes rows [i0, i1) of B, the wave partials (reusing
-    // sg[0, nw*d), d <= Dt) are added in wave order
-    const int i0 = (int)((long long)Dt * w / nw), i1 = (int)((long long)Dt * (w + 1) / nw);
-    for (int k = lane; k < d; k += 64) {
-        float s = 0.f;
-#pragma unroll 8
-        for (int i = i0; i < i1; ++i) s = fmaf(B[(size_t)i * d + k], sA[i], s);
-        sg[w * d + k] = s;
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < d; k += blockDim.x) {
-        float s = sg[k];
-        for (int w2 = 1; w2 < nw; ++w2) s += sg[w2 * d + k];
-        gth[k] = s;
-    }
+    return s;
 }
 
 // Both steps in one block per theta, for launches with enough thetas to fill
 // the chip by themselves.
 __global__ __launch_bounds__(RBLOCK) void k_reduce_theta(const float* __restrict__ part, int tiles, int Dt, int ndim,
                                                          int nc0, int nc1, int nc2, const float* __restrict__ B, int d,
-                                                         float* __restrict__ gtheta, float* __restrict__ gA) {
+                                                         float* __restrict__ gtheta) {
     extern __shared__ float sg[];  // [nw + 1, Dt]
     const int th = blockIdx.x;
     const int nc[3] = {nc0, nc1, nc2};
-    reduce_theta(sg, part + (size_t)th * tiles * Dt, tiles, Dt, ndim, nc, B, d, gtheta + (size_t)th * d,
-                 gA ? gA + (size_t)th * Dt : nullptr);
-}
-
-// Column slice blockIdx.y (columns [c0, c0 + cw)) of theta blockIdx.x's
-// dL/dA: the block's waves sum the tiles (wave w: tiles w, w + nw, ...), the
-// wave sums are added in wave order and scaled to x-space -- per column the
-// same arithmetic as reduce_theta.  The result overwrites the tile-0 row of
-// the partials (each block owns its columns and has read them all first) and
-// goes to gA when given.  Slicing the columns gives a few thetas enough
-// blocks to fill the chip.
-__global__ __launch_bounds__(RBLOCK) void k_reduce_cols(float* __restrict__ part, int tiles, int Dt, int cw, int ndim,
-                                                        int nc0, int nc1, int nc2, float* __restrict__ gA) {
-    extern __shared__ float sg[];  // [nw, cw]
-    const int th = blockIdx.x;
-    const int c0 = blockIdx.y * cw, c1 = (c0 + cw < Dt) ? c0 + cw : Dt;
-    const int nw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int P = ndim * (ndim + 1);
-    const int nc[3] = {nc0, nc1, nc2};
-    float* pp = part + (size_t)th * tiles * Dt;
-    for (int i = c0 + lane; i < c1; i += 64) {
-        float s0 = 0.f, s1 = 0.f;
-        int t = w;
-        for (; t + nw < tiles; t += 2 * nw) {
-            s0 += pp[(size_t)t * Dt + i];
-            s1 += pp[(size_t)(t + nw) * Dt + i];
-        }
-        if (t < tiles) s0 += pp[(size_t)t * Dt + i];
-        sg[w * cw + (i - c0)] = s0 + s1;
-    }
-    __syncthreads();
-    for (int i = c0 + threadIdx.x; i < c1; i += blockDim.x) {
-        float s = sg[i - c0];
-        for (int k = 1; k < nw; ++k) s += sg[k * cw + (i - c0)];
-        const int rem = i % P, r = rem / (ndim + 1), col = rem % (ndim + 1);
-        const float sc = (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
-        s *= sc;
-        pp[i] = s;
-        if (gA) gA[(size_t)th * Dt + i] = s;
-    }
-}
-
-// dL/dtheta = B^T dL/dA for theta blockIdx.x, dL/dA (x-space) in the tile-0
-// row of its partials: wave w takes rows [i0, i1) of B, the wave partials are
-// added in wave order.
-__global__ __launch_bounds__(RBLOCK) void k_reduce_bt(const float* __restrict__ part, int tiles, int Dt,
-                                                      const float* __restrict__ B, int d, float* __restrict__ gtheta) {
-    extern __shared__ float sg[];  // [Dt + nw * d]
-    const int th = blockIdx.x;
     const int nw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const float* pp = part + (size_t)th * tiles * Dt;
-    float* sA = sg;
-    float* sw = sg + Dt;
+    for (int i = lane; i < Dt; i += 64) sg[w * Dt + i] = rows_sum(pp, tiles, Dt, i, w, nw, AllRows());
+    __syncthreads();
+    float* sA = sg + nw * Dt;
+    for (int i = threadIdx.x; i < Dt; i += blockDim.x) {
+        float s = sg[i];
+        for (int k = 1; k < nw; ++k) s += sg[k * Dt + i];
+        sA[i] = s * x_scale(i, ndim, nc);
+    }
+    __syncthreads();
+    // the wave shares reuse sg[0, nw * d), d <= Dt
+    const int i0 = (int)((long long)Dt * w / nw), i1 = (int)((long long)Dt * (w + 1) / nw);
+    for (int k = lane; k < d; k += 64) sg[w * d + k] = bt_sum(B, sA, d, k, i0, i1);
+    __syncthreads();
+    for (int k = threadIdx.x; k < d; k += blockDim.x) {
+        float s = sg[k];
+        for (int w2 = 1; w2 < nw; ++w2) s += sg[w2 * d + k];
+        gtheta[(size_t)th * d + k] = s;
+    }
+}
+
+// The same in two kernels for a few thetas: columns [c0, c1) of the row sums by
+// one block, whose result overwrites row 0 of the partials (each block owns its
+// columns and has read them all first); then 64 entries of dL/dtheta by one
+// block.  Slices give a few thetas enough blocks to fill the chip.
+template <class Rows>
+__device__ __forceinline__ void reduce_cols(float* sg, float* __restrict__ pp, int nrows, int Dt, int c0, int c1,
+                                            int ndim, const int (&nc)[3], Rows rows) {
+    const int cw = c1 - c0, nw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int i = lane; i < cw; i += 64) sg[w * cw + i] = rows_sum(pp, nrows, Dt, c0 + i, w, nw, rows);
+    __syncthreads();
+    for (int i = threadIdx.x; i < cw; i += blockDim.x) {
+        float s = sg[i];
+        for (int k = 1; k < nw; ++k) s += sg[k * cw + i];
+        pp[c0 + i] = s * x_scale(c0 + i, ndim, nc);
+    }
+}
+__device__ __forceinline__ void reduce_bt(float* sg, const float* __restrict__ pp, int Dt, const float* __restrict__ B,
+                                          int d, int k0, float* __restrict__ gth) {
+    const int nw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float* sA = sg;       // [Dt]
+    float* sw = sg + Dt;  // [nw, 64]
     for (int i = threadIdx.x; i < Dt; i += blockDim.x) sA[i] = pp[i];
     __syncthreads();
     const int i0 = (int)((long long)Dt * w / nw), i1 = (int)((long long)Dt * (w + 1) / nw);
-    for (int k = lane; k < d; k += 64) {
-        float s = 0.f;
-#pragma unroll 8
-        for (int i = i0; i < i1; ++i) s = fmaf(B[(size_t)i * d + k], sA[i], s);
-        sw[w * d + k] = s;
-    }
+    const int k = k0 + lane;
+    sw[w * 64 + lane] = k < d ? bt_sum(B, sA, d, k, i0, i1) : 0.f;
     __syncthreads();
-    for (int k = threadIdx.x; k < d; k += blockDim.x) {
-        float s = sw[k];
-        for (int w2 = 1; w2 < nw; ++w2) s += sw[w2 * d + k];
-        gtheta[(size_t)th * d + k] = s;
+    if (w == 0 && k < d) {
+        float s = sw[lane];
+        for (int w2 = 1; w2 < nw; ++w2) s += sw[w2 * 64 + lane];
+        gth[k] = s;
     }
+}
+
+// grid (n_theta, slices of cw columns)
+__global__ __launch_bounds__(RBLOCK) void k_reduce_cols(float* __restrict__ part, int tiles, int Dt, int cw, int ndim,
+                                                        int nc0, int nc1, int nc2) {
+    extern __shared__ float sg[];  // [nw, cw]
+    const int nc[3] = {nc0, nc1, nc2};
+    const int c0 = blockIdx.y * cw, c1 = (c0 + cw < Dt) ? c0 + cw : Dt;
+    reduce_cols(sg, part + (size_t)blockIdx.x * tiles * Dt, tiles, Dt, c0, c1, ndim, nc, AllRows());
+}
+
+// grid (n_theta, ceil(d / 64))
+__global__ __launch_bounds__(RBLOCK) void k_reduce_bt(const float* __restrict__ part, int tiles, int Dt,
+                                                      const float* __restrict__ B, int d, float* __restrict__ gtheta) {
+    extern __shared__ float sg[];  // [Dt + nw * 64]
+    reduce_bt(sg, part + (size_t)blockIdx.x * tiles * Dt, Dt, B, d, blockIdx.y * 64, gtheta + (size_t)blockIdx.x * d);
 }
 
 // cell index of each point (libcpab/numpy/findcellidx.py semantics, FP32)
@@ -1574,24 +1558,50 @@ __global__ __launch_bounds__(BLOCK) void k_fill_zero(float* p, size_t n) {
     for (size_t i = (size_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * BLOCK) p[i] = 0.f;
 }
 
-// A_q = B theta for every instance: grid (ceil(maxDt/BLOCK), n_inst)
+// A_q = B theta for every instance: grid (ceil(maxDt/64), n_inst), 64 rows of B per
+// block.  The block reads them in pieces of 64 columns, coalesced, into LDS (odd
+// pitch); a lane of the first wave sums each row from there, in column order as
+// k_theta_to_A does.  The instances' bases are all different, so nothing is in
+// cache: a thread that walks its own row (k_theta_to_A, better where many thetas
+// share one B) asks for 64 cache lines per load, 29 us for the 200 instances of
+// a ragged batch against 12.
+constexpr int A_ROWS = 64, A_PITCH = 65;
 __global__ __launch_bounds__(BLOCK) void k_batch_A(const cpab_instance_t* __restrict__ inst) {
-    extern __shared__ float sth[];
+    __shared__ float sB[A_ROWS * A_PITCH];
     const cpab_instance_t* I = inst + blockIdx.y;
     const int nd = I->tess.ndim, d = I->tess.d;
     const int P = nd * (nd + 1);
     const int Dt = I->tess.nC * P;
-    if ((int)(blockIdx.x * BLOCK) >= Dt) return;
-    for (int k = threadIdx.x; k < d; k += BLOCK) sth[k] = I->theta[k];
-    __syncthreads();
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= Dt) return;
-    const float* b = I->tess.B + (size_t)i * d;
+    const int r0 = blockIdx.x * A_ROWS;
+    if (r0 >= Dt) return;
+    const float* __restrict__ B = I->tess.B;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     float acc = 0.f;
-    for (int k = 0; k < d; ++k) acc = fmaf(b[k], sth[k], acc);
-    const int rem = i % P, r = rem / (nd + 1), col = rem % (nd + 1);
-    const float sc = (col < nd) ? (float)I->tess.nc[r] / (float)I->tess.nc[col] : (float)I->tess.nc[r];
-    static_cast<float*>(I->ws)[i] = acc * sc;
+    for (int k0 = 0; k0 < d; k0 += 64) {
+        const int nk = d - k0 < 64 ? d - k0 : 64;
+        if (k0) __syncthreads();
+        float v[A_ROWS / WAVES];
+#pragma unroll
+        for (int e = 0; e < A_ROWS / WAVES; ++e) {
+            const int r = r0 + e * WAVES + w;
+            v[e] = r < Dt && lane < nk ? B[(size_t)r * d + k0 + lane] : 0.f;
+        }
+        const float th = lane < nk ? I->theta[k0 + lane] : 0.f;  // lane k holds theta[k0 + k]
+#pragma unroll
+        for (int e = 0; e < A_ROWS / WAVES; ++e) sB[(e * WAVES + w) * A_PITCH + lane] = v[e];
+        __syncthreads();
+        if (w == 0) {
+#pragma unroll 8
+            for (int k = 0; k < nk; ++k)
+                acc = fmaf(sB[lane * A_PITCH + k], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(th), k)), acc);
+        }
+    }
+    const int i = r0 + lane;
+    if (w == 0 && i < Dt) {
+        const int rem = i % P, r = rem / (nd + 1), col = rem % (nd + 1);
+        const float sc = (col < nd) ? (float)I->tess.nc[r] / (float)I->tess.nc[col] : (float)I->tess.nc[r];
+        static_cast<float*>(I->ws)[i] = acc * sc;
+    }
 }
 
 // MAXD: the largest ndim among the instances (2 or 3); without 3D instances
@@ -1737,17 +1747,32 @@ __device__ __forceinline__ int batch_rows(int item0, int tiles, RunRows& rr) {
     return 1 + (rr.a < tiles ? (tiles - 1 - rr.a) / GRAB + 1 : 0);
 }
 
-// per instance: dL/dtheta = B^T (sum over its items of the partials, in x-space)
-__global__ __launch_bounds__(RBLOCK) void k_batch_reduce(const cpab_instance_t* __restrict__ inst) {
-    extern __shared__ float sg[];  // [nw + 1, largest Dt of the batch]
+// dL/dtheta of every instance: grid (n_inst, ceil(maxDt / 64)), then (n_inst,
+// ceil(maxd / 64)).  Sliced as above: one block per instance left the largest
+// ones' megabytes of rows and of B to a single CU (56 us for the 200 instances of
+// a ragged batch, now 11 + 18).
+__device__ __forceinline__ float* batch_part(const cpab_instance_t* I, int Dt) {
+    return reinterpret_cast<float*>(static_cast<char*>(I->ws) + align256_hd((size_t)Dt * 4));
+}
+__global__ __launch_bounds__(RBLOCK) void k_batch_cols(const cpab_instance_t* __restrict__ inst) {
+    extern __shared__ float sg[];  // [nw, 64]
     const cpab_instance_t* I = inst + blockIdx.x;
     const int nd = I->tess.ndim;
     const int Dt = I->tess.nC * nd * (nd + 1);
-    const float* part = reinterpret_cast<const float*>(static_cast<const char*>(I->ws) + align256_hd((size_t)Dt * 4));
+    const int c0 = blockIdx.y * R_COLS, c1 = c0 + R_COLS < Dt ? c0 + R_COLS : Dt;
+    if (c0 >= Dt) return;
     const int nc[3] = {I->tess.nc[0], I->tess.nc[1], I->tess.nc[2]};
     RunRows rr;
     const int nrows = batch_rows(I->item0, I->tiles, rr);
-    reduce_theta(sg, part, nrows, Dt, nd, nc, I->tess.B, I->tess.d, I->grad_theta, nullptr, rr);
+    reduce_cols(sg, batch_part(I, Dt), nrows, Dt, c0, c1, nd, nc, rr);
+}
+__global__ __launch_bounds__(RBLOCK) void k_batch_bt(const cpab_instance_t* __restrict__ inst) {
+    extern __shared__ float sg[];  // [largest Dt of the batch + nw * 64]
+    const cpab_instance_t* I = inst + blockIdx.x;
+    const int nd = I->tess.ndim;
+    const int Dt = I->tess.nC * nd * (nd + 1);
+    if ((int)blockIdx.y * 64 >= I->tess.d) return;
+    reduce_bt(sg, batch_part(I, Dt), Dt, I->tess.B, I->tess.d, blockIdx.y * 64, I->grad_theta);
 }
 
 // ---------------------------------------------------------------------------
@@ -2313,43 +2338,42 @@ int launch_theta_to_A(const cpab_tess_t* t, const float* theta, int n_theta, flo
     return status_from_hip();
 }
 
-// dL/dtheta from the per-tile partials (overwritten): column-sliced tile sums,
-// then B^T per theta.  Deterministic: fixed summation order throughout.
-int launch_reduce(const cpab_tess_t* t, float* part, int n_theta, int tiles, float* gtheta, float* gA,
-                  hipStream_t st) {
+// dL/dtheta from the per-tile partials (overwritten).  Deterministic: fixed
+// summation order throughout.
+int launch_reduce(const cpab_tess_t* t, float* part, int n_theta, int tiles, float* gtheta, hipStream_t st) {
     const int Dt = t->nC * t->ndim * (t->ndim + 1);
     Geo g = make_geo(t);
-    // column slices of at least 64 columns, enough of them for ~1024 blocks
-    int nslice = (1024 + n_theta - 1) / n_theta;
-    const int max_slices = (Dt + 63) / 64;
-    if (nslice > max_slices) nslice = max_slices;
-    if (nslice < 1) nslice = 1;
-    if (nslice == 1 || tiles <= 64) {
-        // enough thetas, or few rows per theta: one block per theta, as many
-        // waves (up to 16) as the LDS holds [nw + 1, Dt] floats for
+    // One block per theta with enough thetas, or with few rows each; as many waves
+    // as the LDS holds [nw + 1, Dt] floats for, up to 16, but no more than 8192
+    // waves in all: past that the blocks queue and their latencies add up ([50],
+    // 4096 thetas, one row each: 37 us with 16 waves, 14 with 4).
+    if (n_theta >= 1024 || (n_theta >= 32 && tiles <= 64) || (size_t)tiles * Dt <= 8192) {
         int nw = RBLOCK / 64;
+        while (nw > 4 && (long long)n_theta * nw > 8192) nw >>= 1;
         while (nw > 1 && (size_t)(nw + 1) * Dt * sizeof(float) > LDS_LIMIT) nw >>= 1;
         if ((size_t)(nw + 1) * Dt * sizeof(float) <= LDS_LIMIT) {
             hipLaunchKernelGGL(k_reduce_theta, dim3(n_theta), dim3(nw * 64), (nw + 1) * Dt * sizeof(float), st, part,
-                               tiles, Dt, t->ndim, g.nc0, g.nc1, g.nc2, t->B, t->d, gtheta, gA);
+                               tiles, Dt, t->ndim, g.nc0, g.nc1, g.nc2, t->B, t->d, gtheta);
             return status_from_hip();
         }
     }
-    // k_reduce_cols keeps [16 waves, cw] floats in LDS: at most cols_fit columns per slice
+    // column slices of at least 64 columns, enough of them for ~1024 blocks, each
+    // with at most cols_fit columns ([16 waves, cw] floats of LDS)
+    int nslice = (1024 + n_theta - 1) / n_theta;
+    const int max_slices = (Dt + R_COLS - 1) / R_COLS;
+    if (nslice > max_slices) nslice = max_slices;
     const int nw = RBLOCK / 64;
     const int cols_fit = (int)(LDS_LIMIT / ((size_t)nw * sizeof(float)));
     if (nslice < (Dt + cols_fit - 1) / cols_fit) nslice = (Dt + cols_fit - 1) / cols_fit;
     const int cw = (Dt + nslice - 1) / nslice;
     nslice = (Dt + cw - 1) / cw;
-    // B^T: as many waves (up to 16) as the LDS holds Dt + nw * d floats for;
     // checked before the first launch
-    int nwb = RBLOCK / 64;
-    while (nwb > 1 && (size_t)(Dt + nwb * t->d) * sizeof(float) > LDS_LIMIT) nwb >>= 1;
-    if ((size_t)(Dt + nwb * t->d) * sizeof(float) > LDS_LIMIT) return CPAB_ERR_LDS;
+    const size_t lds_bt = (size_t)(Dt + nw * 64) * sizeof(float);
+    if (lds_bt > LDS_LIMIT) return CPAB_ERR_LDS;
     hipLaunchKernelGGL(k_reduce_cols, dim3(n_theta, nslice), dim3(nw * 64), (size_t)nw * cw * sizeof(float), st,
-                       part, tiles, Dt, cw, t->ndim, g.nc0, g.nc1, g.nc2, gA);
-    hipLaunchKernelGGL(k_reduce_bt, dim3(n_theta), dim3(nwb * 64), (size_t)(Dt + nwb * t->d) * sizeof(float), st,
-                       part, tiles, Dt, t->B, t->d, gtheta);
+                       part, tiles, Dt, cw, t->ndim, g.nc0, g.nc1, g.nc2);
+    hipLaunchKernelGGL(k_reduce_bt, dim3(n_theta, (t->d + 63) / 64), dim3(nw * 64), lds_bt, st, part, tiles, Dt, t->B,
+                       t->d, gtheta);
     return status_from_hip();
 }
 
@@ -2573,7 +2597,7 @@ int cpab_transform_bwd(const cpab_tess_t* t, const float* theta, int n_theta, co
     CPAB_DISPATCH_D(t->ndim, LAUNCH_TB)
 #undef LAUNCH_TB
     if ((rc = status_from_hip())) return rc;
-    return launch_reduce(t, part, n_theta, L.tiles, grad_theta, nullptr, stream);
+    return launch_reduce(t, part, n_theta, L.tiles, grad_theta, stream);
 }
 
 static int img_from(int ndim, const float* data, int C, const int* dsize, Img& im) {
@@ -2771,7 +2795,7 @@ int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_thet
 #undef LAUNCH_DB
 #undef LAUNCH_DB3
     if ((rc = status_from_hip())) return rc;
-    return launch_reduce(t, part, n_theta, nbt, grad_theta, nullptr, stream);
+    return launch_reduce(t, part, n_theta, nbt, grad_theta, stream);
 }
 
 int cpab_findcell(int ndim, const int* nc, const float* points, int nP, int* idx, hipStream_t stream) {
@@ -2943,8 +2967,7 @@ int cpab_batch_fwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
     if (rc) return rc;
     bool save = true;
     for (int i = 0; i < n_inst; ++i) save = save && host_inst[i].saved != nullptr;
-    hipLaunchKernelGGL(k_batch_A, dim3((maxDt + BLOCK - 1) / BLOCK, n_inst), dim3(BLOCK), maxd * sizeof(float), stream,
-                       dev_inst);
+    hipLaunchKernelGGL(k_batch_A, dim3((maxDt + A_ROWS - 1) / A_ROWS, n_inst), dim3(BLOCK), 0, stream, dev_inst);
     hipLaunchKernelGGL(k_counter_reset, dim3(1), dim3(64), 0, stream, counter);
     int maxnd = 1;
     for (int i = 0; i < n_inst; ++i) maxnd = host_inst[i].tess.ndim > maxnd ? host_inst[i].tess.ndim : maxnd;
@@ -2975,8 +2998,7 @@ int cpab_batch_bwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
     // with the forward's saved state, its A_q is still in every instance's
     // workspace (the backward only writes the partials after it)
     if (!have)
-        hipLaunchKernelGGL(k_batch_A, dim3((maxDt + BLOCK - 1) / BLOCK, n_inst), dim3(BLOCK), maxd * sizeof(float),
-                           stream, dev_inst);
+        hipLaunchKernelGGL(k_batch_A, dim3((maxDt + A_ROWS - 1) / A_ROWS, n_inst), dim3(BLOCK), 0, stream, dev_inst);
     hipLaunchKernelGGL(k_counter_reset, dim3(1), dim3(64), 0, stream, counter);
     // the item range of each LDS class (contiguous, as cpab_batch_plan lays
     // them out); a plan in another order runs as one class
@@ -3033,12 +3055,12 @@ int cpab_batch_bwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
     }
 #undef LAUNCH_BB
     if ((rc = status_from_hip())) return rc;
-    // as many waves (up to 16) as the LDS holds [nw + 1, maxDt] floats for
-    int nw = RBLOCK / 64;
-    while (nw > 1 && (size_t)(nw + 1) * maxDt * sizeof(float) > LDS_LIMIT) nw >>= 1;
-    if ((size_t)(nw + 1) * maxDt * sizeof(float) > LDS_LIMIT) return CPAB_ERR_LDS;
-    hipLaunchKernelGGL(k_batch_reduce, dim3(n_inst), dim3(nw * 64), (nw + 1) * maxDt * sizeof(float), stream,
-                       dev_inst);
+    const int nw = RBLOCK / 64;
+    const size_t lds_bt = (size_t)(maxDt + nw * 64) * sizeof(float);
+    if (lds_bt > LDS_LIMIT) return CPAB_ERR_LDS;
+    hipLaunchKernelGGL(k_batch_cols, dim3(n_inst, (maxDt + R_COLS - 1) / R_COLS), dim3(nw * 64),
+                       (size_t)nw * R_COLS * sizeof(float), stream, dev_inst);
+    hipLaunchKernelGGL(k_batch_bt, dim3(n_inst, (maxd + 63) / 64), dim3(nw * 64), lds_bt, stream, dev_inst);
     return status_from_hip();
 }
 
@@ -3180,7 +3202,7 @@ int cpab_ref_grad_theta(const float* points, const float* As, const float* B, in
     t.nC = nC;
     t.d = d;
     t.B = B;
-    return launch_reduce(&t, part, n_theta, blocks, grad_theta, nullptr, stream);
+    return launch_reduce(&t, part, n_theta, blocks, grad_theta, stream);
 }
 
 int cpab_slow_forward(const float* points, const float* trels, int nstepsolver, const int* nc, int ndim, int nP,
