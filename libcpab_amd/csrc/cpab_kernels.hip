@@ -132,41 +132,6 @@ __device__ __forceinline__ int div_small(int n, int d, float rd, int& rem) {
     return q;
 }
 
-// output-order index t of round r of this thread in tile `tile`, -1 if outside
-template <int D>
-__device__ __forceinline__ int tile_t(const Launch& L, const Src& s, int tile, int r) {
-    if (L.ty == 0) {
-        const int t = (tile * L.ppt + r) * BLOCK + (int)threadIdx.x;
-        return t < L.nP ? t : -1;
-    }
-    if constexpr (D == 3) {
-        const int tiles_z = (s.g2 + 7) >> 3, tiles_y = (s.g1 + 7) >> 3;
-        const int tz = tile % tiles_z, ty = (tile / tiles_z) % tiles_y, tx = tile / (tiles_z * tiles_y);
-        const int iz = tz * 8 + ((int)threadIdx.x & 7);
-        const int iy = ty * 8 + (((int)threadIdx.x >> 3) & 7);
-        const int ix = (tx * L.ppt + r) * WAVES + ((int)threadIdx.x >> 6);
-        return (ix < s.g0 && iy < s.g1 && iz < s.g2) ? (ix * s.g1 + iy) * s.g2 + iz : -1;
-    }
-    const int rows = BLOCK / L.ty;
-    const int tiles_y = (s.g1 + L.ty - 1) / L.ty;
-    const int ix = (tile / tiles_y) * (L.ppt * rows) + r * rows + (int)threadIdx.x / L.ty;
-    const int iy = (tile % tiles_y) * L.ty + (int)threadIdx.x % L.ty;
-    return (ix < s.g0 && iy < s.g1) ? ix * s.g1 + iy : -1;
-}
-
-__device__ __forceinline__ int xcd_remap(int b, int nb) {
-    // blocks are dispatched round-robin over 8 XCDs; give each XCD a contiguous
-    // range of logical tiles so one theta's tiles share an L2
-    const int xcd = b & 7, k = b >> 3;
-    const int per = nb >> 3, rem = nb & 7;
-    return xcd * per + (xcd < rem ? xcd : rem) + k;
-}
-
-template <int D>
-__device__ __forceinline__ int nc_at(const Geo& g, int a) {
-    return a == 0 ? g.nc0 : (a == 1 ? g.nc1 : g.nc2);
-}
-
 // point index p of output-order index t (last output axis fastest)
 template <int D>
 __device__ __forceinline__ int out_to_point(const Src& s, int t, int (&ix)[3]) {
@@ -184,6 +149,57 @@ __device__ __forceinline__ int out_to_point(const Src& s, int t, int (&ix)[3]) {
         ix[0] = r / s.g1;
         return ix[0] + s.g0 * (ix[1] + s.g1 * ix[2]);
     }
+}
+
+// Output-order index t and axis indexes ix of round r of this thread in tile
+// `tile`; t = -1 if outside.  The divisions are of wave-uniform values or by powers
+// of two (a per-lane division costs 25 instructions, an eighth of a 2D round).
+template <int D>
+__device__ __forceinline__ int tile_t(const Launch& L, const Src& s, int tile, int r, int (&ix)[3]) {
+    const int tid = (int)threadIdx.x;
+    if (L.ty == 0) {
+        const int t = (tile * L.ppt + r) * BLOCK + tid;
+        if (t >= L.nP) return -1;
+        out_to_point<D>(s, t, ix);
+        return t;
+    }
+    if constexpr (D == 3) {
+        const int tiles_z = (s.g2 + 7) >> 3, tiles_y = (s.g1 + 7) >> 3;
+        const int tz = tile % tiles_z, ty = (tile / tiles_z) % tiles_y, tx = tile / (tiles_z * tiles_y);
+        ix[2] = tz * 8 + (tid & 7);
+        ix[1] = ty * 8 + ((tid >> 3) & 7);
+        ix[0] = (tx * L.ppt + r) * WAVES + (tid >> 6);
+        return (ix[0] < s.g0 && ix[1] < s.g1 && ix[2] < s.g2) ? (ix[0] * s.g1 + ix[1]) * s.g2 + ix[2] : -1;
+    }
+    const int sh = L.ty == 16 ? 4 : 3;  // tile_ty
+    const int rows = BLOCK >> sh;
+    const int tiles_y = (s.g1 + L.ty - 1) >> sh;
+    const int tx = tile / tiles_y, ty = tile - tx * tiles_y;
+    ix[0] = (tx * L.ppt + r) * rows + (tid >> sh);
+    ix[1] = (ty << sh) + (tid & (L.ty - 1));
+    return (ix[0] < s.g0 && ix[1] < s.g1) ? ix[0] * s.g1 + ix[1] : -1;
+}
+template <int D>
+__device__ __forceinline__ int tile_t(const Launch& L, const Src& s, int tile, int r) {
+    if (L.ty == 0) {
+        const int t = (tile * L.ppt + r) * BLOCK + (int)threadIdx.x;
+        return t < L.nP ? t : -1;
+    }
+    int ix[3];
+    return tile_t<D>(L, s, tile, r, ix);
+}
+
+__device__ __forceinline__ int xcd_remap(int b, int nb) {
+    // blocks are dispatched round-robin over 8 XCDs; give each XCD a contiguous
+    // range of logical tiles so one theta's tiles share an L2
+    const int xcd = b & 7, k = b >> 3;
+    const int per = nb >> 3, rem = nb & 7;
+    return xcd * per + (xcd < rem ? xcd : rem) + k;
+}
+
+template <int D>
+__device__ __forceinline__ int nc_at(const Geo& g, int a) {
+    return a == 0 ? g.nc0 : (a == 1 ? g.nc1 : g.nc2);
 }
 
 // LDS layout of one theta's tables: A_q [nC*P], 1/|M|_F [nC (padded to 4)],
@@ -431,6 +447,33 @@ __device__ __forceinline__ float blend(const float (&v)[1 << D], const float (&f
 }
 
 // value of channel data dp at the corners (i0, i1, fd)
+// base[i], base uniform over the wave: in 2D and 3D, where the chunk log's 32-bit
+// row bounds keep an instance's points below 2^29, as a scalar base and a 32-bit
+// byte offset (a 64-bit address is two more instructions per access).
+template <int D>
+__device__ __forceinline__ float at(const float* base, int i) {
+    if constexpr (D == 1) return base[i];
+    asm("" : "+s"(base));
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + ((unsigned)i << 2));
+}
+template <int D>
+__device__ __forceinline__ void put(float* base, int i, float v) {
+    if constexpr (D == 1) {
+        base[i] = v;
+    } else {
+        asm("" : "+s"(base));
+        *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + ((unsigned)i << 2)) = v;
+    }
+}
+// nP, made anew in every round: the rows' base addresses are then scalar work of
+// the round.  Hoisted out of the loop they take two scalar registers each, far
+// more than there are, and come back from vector lanes at two vector instructions
+// per access.
+__device__ __forceinline__ size_t per_round(int nP) {
+    asm volatile("" : "+s"(nP));
+    return (size_t)(unsigned)nP;
+}
+
 template <int D>
 __device__ __forceinline__ float interp_value(const float* __restrict__ dp, const Img& im, const int (&i0)[3],
                                               const int (&i1)[3], const float (&fd)[3]) {
@@ -456,7 +499,7 @@ constexpr int chan_group_bwd() { return D == 2 ? 2 : 1; }
 template <int D>
 __device__ __forceinline__ void interp_channels(const float* __restrict__ data, size_t dstride, const Img& im,
                                                 const int (&i0)[3], const int (&i1)[3], const float (&fd)[3],
-                                                float* __restrict__ out, size_t ostride) {
+                                                float* __restrict__ out, int t, size_t ostride) {
     constexpr int NK = 1 << D, CG = chan_group<D>();
     int off[NK];
     corner_offsets<D>(im, i0, i1, off);
@@ -471,7 +514,7 @@ __device__ __forceinline__ void interp_channels(const float* __restrict__ data, 
             }
 #pragma unroll
         for (int k = 0; k < CG; ++k)
-            if (c0 + k < im.C) out[(size_t)(c0 + k) * ostride] = blend<D>(v[k], fd);
+            if (c0 + k < im.C) put<D>(out + (size_t)(c0 + k) * ostride, t, blend<D>(v[k], fd));
     }
 }
 
@@ -628,7 +671,7 @@ template <int D>
 __device__ __forceinline__ void interp_backward_channels(const float* __restrict__ data, float* gdata, size_t dstride,
                                                          const Img& im, const int (&i0)[3], const int (&i1)[3],
                                                          const float (&fd)[3], const float* __restrict__ gout,
-                                                         size_t gstride, float (&gk)[4], float (&dfd)[3]) {
+                                                         int t, size_t gstride, float (&gk)[4], float (&dfd)[3]) {
     constexpr int NK = 1 << D, CG = chan_group_bwd<D>();
     int off[NK];
     corner_offsets<D>(im, i0, i1, off);
@@ -638,7 +681,7 @@ __device__ __forceinline__ void interp_backward_channels(const float* __restrict
         for (int k = 0; k < CG; ++k)
             if (c0 + k < im.C) {
                 const float* dp = data + (size_t)(c0 + k) * dstride;
-                gv[k] = gout[(size_t)(c0 + k) * gstride];
+                gv[k] = at<D>(gout + (size_t)(c0 + k) * gstride, t);
 #pragma unroll
                 for (int j = 0; j < NK; ++j) v[k][j] = dp[off[j]];
             }
@@ -673,7 +716,7 @@ template <int D, bool INST = false>
 __device__ __forceinline__ void interp_backward_merged(bool valid, const float* __restrict__ data, float* gdata,
                                                        size_t dstride, const Img& im, const int (&i0)[3],
                                                        const int (&i1)[3], const float (&fd)[3],
-                                                       const float* __restrict__ gout, size_t gstride, int w,
+                                                       const float* __restrict__ gout, int t, size_t gstride, int w,
                                                        float (&dfd)[3], int inst = 0) {
     constexpr int NK = 1 << D;
     int off[NK];
@@ -687,7 +730,7 @@ __device__ __forceinline__ void interp_backward_merged(bool valid, const float* 
     }
     for (int c = 0; c < im.C; ++c) {
         const float* dp = data + (size_t)c * dstride;
-        const float g = gout[(size_t)c * gstride];
+        const float g = gout[(size_t)c * gstride + t];
         float v[NK];
 #pragma unroll
         for (int j = 0; j < NK; ++j) v[j] = dp[off[j]];
@@ -844,21 +887,21 @@ __device__ __forceinline__ void fused_fwd_tile(const Launch& L, const Geo& g, co
     // at the end of the tile: a wave-uniform sum, no per-lane state
     int wave_bad = 0;
     for (int r = 0; r < L.ppt; ++r) {
-        const int t = tile_t<D>(L, s, tile, r);
-        if (t < 0) continue;
         int ix[3];
-        out_to_point<D>(s, t, ix);
+        const int t = tile_t<D>(L, s, tile, r, ix);
+        if (t < 0) continue;
+        const size_t nP = per_round(L.nP);
         float x[D], q[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            x[a] = s.lin[goff[a] + ix[a]];
+            x[a] = at<D>(s.lin, goff[a] + ix[a]);
             q[a] = x[a] * (float)nc[a];
         }
         const int c0 = start_cell<D>(x, nc, tab, g);
         float J[D][D];
         // with saved state (2D/3D) the chunk durations go straight to their rows
         LogSink lg;
-        if constexpr (SAVE && D > 1) lg.init(sv + (size_t)(D + D * D) * L.nP, L.nP, t);
+        if constexpr (SAVE && D > 1) lg.init(sv + (D + D * D) * nP, (int)nP, t);
         integrate<D, SAVE, SAVE && (D > 1), LogSink>(q, c0, L.t_end, tab, g.nc0, g.tol0, J, lg);
         float y[D];
 #pragma unroll
@@ -866,24 +909,26 @@ __device__ __forceinline__ void fused_fwd_tile(const Launch& L, const Geo& g, co
         if constexpr (SAVE) {
             // indexed in output order t (the order threads run in) for coalesced stores
 #pragma unroll
-            for (int a = 0; a < D; ++a) sv[(size_t)a * L.nP + t] = y[a];
+            for (int a = 0; a < D; ++a) put<D>(sv + a * nP, t, y[a]);
 #pragma unroll
             for (int r2 = 0; r2 < D; ++r2)
 #pragma unroll
-                for (int k = 0; k < D; ++k) sv[(size_t)(D + r2 * D + k) * L.nP + t] = J[r2][k];
-            if constexpr (D > 1) sv[(size_t)(D + D * D + NREC) * L.nP + t] = __int_as_float(lg.code);
+                for (int k = 0; k < D; ++k) put<D>(sv + (D + r2 * D + k) * nP, t, J[r2][k]);
+            if constexpr (D > 1) put<D>(sv + (D + D * D + NREC) * nP, t, __int_as_float(lg.code));
         }
         int i0[3], i1[3];
         float fd[3];
         corners<D>(y, im, i0, i1, fd);
-        interp_channels<D>(data, dstride, im, i0, i1, fd, out + t, L.nP);
+        interp_channels<D>(data, dstride, im, i0, i1, fd, out, t, nP);
         wave_bad += __popcll(__ballot(y[0] != y[0]));
     }
     if (wave_bad && g.unfinished && __lane_id() == 0) atomicAdd(g.unfinished, wave_bad);
 }
 
+// 2D with saved state runs 6 waves per SIMD on 80 registers: 410 us against 424 at 5
+// on 84 (7 on 72 spill: 560); 3D loses to the spills (157 -> 182 at 5 on 96).
 template <int D, bool SAVE>
-__global__ __launch_bounds__(BLOCK) void k_transform_data(Launch L, Geo g, Src s, Img im, const float* __restrict__ Aq,
+__global__ __launch_bounds__(BLOCK, (D == 2 && SAVE) ? 6 : 1) void k_transform_data(Launch L, Geo g, Src s, Img im, const float* __restrict__ Aq,
                                                           float* __restrict__ out, float* __restrict__ saved) {
     extern __shared__ float smem[];
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
@@ -909,8 +954,10 @@ __device__ __forceinline__ void write_partials(float* smem_acc, float* __restric
 // adjoint of k_transform: grad_out [n_theta, D, nP] (x-space).  jac (nullable)
 // is the q-space Jacobian stored by the forward.  Writes per-tile partials of
 // dL/dA_q [n_theta, tiles, nC*P] and, if gpts != null, dL/dpoints.
+// 2D: 6 waves per SIMD on 80 registers (64 x 256^2 points without saved state: 132
+// us against 138 at 5 on 92).
 template <int D, bool HAVEJ>
-__global__ __launch_bounds__(BLOCK) void k_transform_bwd(Launch L, Geo g, Src s, const float* __restrict__ Aq,
+__global__ __launch_bounds__(BLOCK, D == 2 ? 6 : 1) void k_transform_bwd(Launch L, Geo g, Src s, const float* __restrict__ Aq,
                                                          const float* __restrict__ gout, const float* __restrict__ jac,
                                                          float* __restrict__ part, float* __restrict__ gpts) {
     extern __shared__ float smem[];
@@ -1083,7 +1130,9 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
         }
     }
     for (int r = 0; r < L.ppt; ++r) {
-        int t = tile_t<D>(L, s, tile, r);
+        int ix[3];
+        const int t = tile_t<D>(L, s, tile, r, ix);
+        const size_t nP = per_round(L.nP);
         const bool valid = t >= 0;
         float q0[D], mu[D], J[D][D], y[D];
         float dfd[3] = {0.f, 0.f, 0.f};
@@ -1099,26 +1148,24 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             for (int k = 0; k < D; ++k) J[a][k] = 0.f;
         }
         if (valid) {
-            int ix[3];
-            out_to_point<D>(s, t, ix);
             float x[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                x[a] = s.lin[goff[a] + ix[a]];
+                x[a] = at<D>(s.lin, goff[a] + ix[a]);
                 q0[a] = x[a] * (float)nc[a];
             }
             c0 = start_cell<D>(x, nc, tab, g);
             if constexpr (HAVES) {
 #pragma unroll
-                for (int a = 0; a < D; ++a) y[a] = sv[(size_t)a * L.nP + t];
+                for (int a = 0; a < D; ++a) y[a] = at<D>(sv + a * nP, t);
 #pragma unroll
                 for (int r2 = 0; r2 < D; ++r2)
 #pragma unroll
-                    for (int k = 0; k < D; ++k) J[r2][k] = sv[(size_t)(D + r2 * D + k) * L.nP + t];
+                    for (int k = 0; k < D; ++k) J[r2][k] = at<D>(sv + (D + r2 * D + k) * nP, t);
                 if constexpr (D > 1) {
 #pragma unroll
-                    for (int k = 0; k < NREC; ++k) lg.h[k] = sv[(size_t)(D + D * D + k) * L.nP + t];
-                    lg.code = __float_as_int(sv[(size_t)(D + D * D + NREC) * L.nP + t]);
+                    for (int k = 0; k < NREC; ++k) lg.h[k] = at<D>(sv + (D + D * D + k) * nP, t);
+                    lg.code = __float_as_int(at<D>(sv + (D + D * D + NREC) * nP, t));
                 }
             } else {
                 float q[D];
@@ -1132,8 +1179,8 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                 int i0[3], i1[3];
                 float fd[3], gk[4] = {0.f, 0.f, 0.f, 0.f};
                 corners<D>(y, im, i0, i1, fd);
-                interp_backward_channels<D>(data, (D != 2 || use_box) ? nullptr : gdata, dstride, im, i0, i1, fd, gout + t,
-                                            L.nP, gk, dfd);
+                interp_backward_channels<D>(data, (D != 2 || use_box) ? nullptr : gdata, dstride, im, i0, i1, fd, gout, t,
+                                            nP, gk, dfd);
                 if constexpr (D == 2) {
                     if (use_box) {
                         const int cd = code[r * BLOCK + threadIdx.x];
@@ -1150,7 +1197,7 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             int i0[3], i1[3];
             float fd[3];
             corners<D>(y, im, i0, i1, fd);
-            interp_backward_merged<D>(valid, data, gdata, dstride, im, i0, i1, fd, gout + (valid ? t : 0), L.nP, L.ty, dfd);
+            interp_backward_merged<D>(valid, data, gdata, dstride, im, i0, i1, fd, gout, valid ? t : 0, nP, L.ty, dfd);
         }
         if (valid) {
             float w[D];
@@ -1320,7 +1367,7 @@ __global__ __launch_bounds__(BLOCK) void k_interp_bwd(int N, int nP, Src s, Img 
     const size_t base = (size_t)n * im.C * dstride;
     // 2D waves are 8 x 8 tiles of one instance; others runs that may span two
     interp_backward_merged<D, D != 2>(valid, im.data + base, im.gdata ? im.gdata + base : nullptr, dstride, im, i0, i1,
-                                        fd, gout + (size_t)n * im.C * nP + t, nP, D == 2 ? 8 : 0, dfd, n);
+                                        fd, gout + (size_t)n * im.C * nP, t, nP, D == 2 ? 8 : 0, dfd, n);
     if (ggrid && valid) {
         const int sz[3] = {im.s0, im.s1, im.s2};
 #pragma unroll
