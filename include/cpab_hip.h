@@ -152,6 +152,26 @@ int cpab_transform_data_fwd(const cpab_tess_t* t, const float* theta, int n_thet
                             const int* dsize, const int* outsize, const float* lin, float t_end, float* out,
                             float* saved, void* workspace, size_t ws_bytes, hipStream_t stream);
 
+/* The transforms with A_q = B theta kept between the directions: the forward
+ * leaves it in Aq (aq_size bytes, at least n_theta * nC * ndim * (ndim+1) * 4)
+ * and needs no workspace; the backward reads it from there instead of theta, and
+ * keeps its workspace.  Otherwise as the calls without the suffix, which make A_q in
+ * each direction. */
+int cpab_transform_fwd_keep(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
+                            int per_theta_grid, const int* grid_shape, float t_end, float* out, float* jac, float* Aq,
+                            size_t aq_size, hipStream_t stream);
+int cpab_transform_bwd_kept(const cpab_tess_t* t, const float* Aq, int n_theta, const float* points, int nP,
+                            int per_theta_grid, const int* grid_shape, float t_end, const float* grad_out,
+                            const float* jac, float* grad_theta, float* grad_points, void* workspace, size_t ws_bytes,
+                            hipStream_t stream);
+int cpab_transform_data_fwd_keep(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
+                                 const int* dsize, const int* outsize, const float* lin, float t_end, float* out,
+                                 float* saved, float* Aq, size_t aq_size, hipStream_t stream);
+int cpab_transform_data_bwd_kept(const cpab_tess_t* t, const float* Aq, int n_theta, const float* data, int C,
+                                 const int* dsize, const int* outsize, const float* lin, float t_end,
+                                 const float* grad_out, const float* saved, float* grad_data, float* grad_theta,
+                                 void* workspace, size_t ws_bytes, hipStream_t stream);
+
 /* cpab_transform_data_fwd without a workspace: no counterpart in the
  * reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  A_q

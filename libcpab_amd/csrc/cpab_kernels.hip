@@ -2545,15 +2545,25 @@ int cpab_theta_to_A(const cpab_tess_t* t, const float* theta, int n_theta, float
         default: FN(3); break;    \
     }
 
-int cpab_transform_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
-                       int per_theta_grid, const int* grid_shape, float t_end, float* out, float* jac,
-                       void* workspace, size_t ws_bytes, hipStream_t stream) {
+// Where a forward puts A_q: at the head of a full workspace, in this device's
+// static scratch array (workspace NULL, ws_bytes 0), or in a buffer of its own
+// that the backward reads it from.
+enum class AqIn { Workspace, Scratch, Buffer };
+
+static size_t aq_bytes(const cpab_tess_t* t, int n_theta) {
+    return (size_t)n_theta * t->nC * t->ndim * (t->ndim + 1) * sizeof(float);
+}
+
+static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
+                    int per_theta_grid, const int* grid_shape, float t_end, float* out, float* jac,
+                    void* workspace, size_t ws_bytes, AqIn where, hipStream_t stream) {
     int rc = check_tess(t);
     if (rc) return rc;
     if (n_theta < 0 || nP < 0) return CPAB_ERR_ARG;
     if (n_theta == 0 || nP == 0) return CPAB_OK;  // arrays with no elements may be NULL
     if (!theta || !points || !out) return CPAB_ERR_ARG;
-    if (ws_bytes < cpab_workspace_bytes(t, n_theta, nP) || !workspace) return CPAB_ERR_WORKSPACE;
+    const size_t need = where == AqIn::Buffer ? aq_bytes(t, n_theta) : cpab_workspace_bytes(t, n_theta, nP);
+    if (ws_bytes < need || !workspace) return CPAB_ERR_WORKSPACE;
     const size_t lds = lds_tables(t->ndim, t->nC + t->nV);
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     float* Aq = static_cast<float*>(workspace);
@@ -2574,6 +2584,20 @@ int cpab_transform_fwd(const cpab_tess_t* t, const float* theta, int n_theta, co
     CPAB_DISPATCH_D(t->ndim, LAUNCH_TF)
 #undef LAUNCH_TF
     return status_from_hip();
+}
+
+int cpab_transform_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
+                       int per_theta_grid, const int* grid_shape, float t_end, float* out, float* jac,
+                       void* workspace, size_t ws_bytes, hipStream_t stream) {
+    return grid_fwd(t, theta, n_theta, points, nP, per_theta_grid, grid_shape, t_end, out, jac, workspace, ws_bytes,
+                    AqIn::Workspace, stream);
+}
+
+int cpab_transform_fwd_keep(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
+                            int per_theta_grid, const int* grid_shape, float t_end, float* out, float* jac, float* Aq,
+                            size_t aq_size, hipStream_t stream) {
+    return grid_fwd(t, theta, n_theta, points, nP, per_theta_grid, grid_shape, t_end, out, jac, Aq, aq_size,
+                    AqIn::Buffer, stream);
 }
 
 int cpab_transform_cells(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
@@ -2608,22 +2632,25 @@ int cpab_transform_cells(const cpab_tess_t* t, const float* theta, int n_theta, 
     return status_from_hip();
 }
 
-int cpab_transform_bwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
-                       int per_theta_grid, const int* grid_shape, float t_end, const float* grad_out, const float* jac,
-                       float* grad_theta, float* grad_points, void* workspace, size_t ws_bytes, hipStream_t stream) {
+// The grid transform's backward: A_q from kept, or (kept NULL) from theta into the
+// workspace.
+static int grid_bwd(const cpab_tess_t* t, const float* theta, const float* kept, int n_theta, const float* points,
+                    int nP, int per_theta_grid, const int* grid_shape, float t_end, const float* grad_out,
+                    const float* jac, float* grad_theta, float* grad_points, void* workspace, size_t ws_bytes,
+                    hipStream_t stream) {
     int rc = check_tess(t);
     if (rc) return rc;
     if (n_theta < 0 || nP < 0) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
     // no points: grad_theta is written with zeros; points and grad_out may be NULL
-    if (!theta || !grad_theta || (nP > 0 && (!points || !grad_out))) return CPAB_ERR_ARG;
+    if ((!theta && !kept) || !grad_theta || (nP > 0 && (!points || !grad_out))) return CPAB_ERR_ARG;
     if (ws_bytes < cpab_workspace_bytes(t, n_theta, nP) || !workspace) return CPAB_ERR_WORKSPACE;
     const size_t lds = lds_bwd(t->ndim, t->nC, t->nC + t->nV);
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     const int Dt = t->nC * t->ndim * (t->ndim + 1);
-    float* Aq = static_cast<float*>(workspace);
+    const float* Aq = kept ? kept : static_cast<const float*>(workspace);
     float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256((size_t)n_theta * Dt * 4));
-    if ((rc = launch_theta_to_A(t, theta, n_theta, Aq, stream))) return rc;
+    if (!kept && (rc = launch_theta_to_A(t, theta, n_theta, static_cast<float*>(workspace), stream))) return rc;
     Launch L;
     Src s = {};
     // 2D tiles only as far as the workspace holds their partials
@@ -2645,6 +2672,21 @@ int cpab_transform_bwd(const cpab_tess_t* t, const float* theta, int n_theta, co
 #undef LAUNCH_TB
     if ((rc = status_from_hip())) return rc;
     return launch_reduce(t, part, n_theta, L.tiles, grad_theta, stream);
+}
+
+int cpab_transform_bwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
+                       int per_theta_grid, const int* grid_shape, float t_end, const float* grad_out, const float* jac,
+                       float* grad_theta, float* grad_points, void* workspace, size_t ws_bytes, hipStream_t stream) {
+    return grid_bwd(t, theta, nullptr, n_theta, points, nP, per_theta_grid, grid_shape, t_end, grad_out, jac, grad_theta,
+                    grad_points, workspace, ws_bytes, stream);
+}
+
+int cpab_transform_bwd_kept(const cpab_tess_t* t, const float* Aq, int n_theta, const float* points, int nP,
+                            int per_theta_grid, const int* grid_shape, float t_end, const float* grad_out,
+                            const float* jac, float* grad_theta, float* grad_points, void* workspace, size_t ws_bytes,
+                            hipStream_t stream) {
+    return grid_bwd(t, nullptr, Aq, n_theta, points, nP, per_theta_grid, grid_shape, t_end, grad_out, jac, grad_theta,
+                    grad_points, workspace, ws_bytes, stream);
 }
 
 static int img_from(int ndim, const float* data, int C, const int* dsize, Img& im) {
@@ -2727,11 +2769,10 @@ size_t cpab_data_workspace_bytes(const cpab_tess_t* t, int n_theta, const int* o
     return align256((size_t)n_theta * Dt * 4) + align256((size_t)n_theta * tiles * Dt * 4);
 }
 
-// The fused forward with A_q either in the caller's workspace or (workspace
-// NULL, ws_bytes 0, from_scratch) in this device's static scratch array.
+// The fused forward with A_q where the caller wants it.
 static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
                     const int* dsize, const int* outsize, const float* lin, float t_end, float* out, float* saved,
-                    void* workspace, size_t ws_bytes, bool from_scratch, hipStream_t stream) {
+                    void* workspace, size_t ws_bytes, AqIn where, hipStream_t stream) {
     int rc = check_tess(t);
     if (rc) return rc;
     Img im;
@@ -2742,12 +2783,13 @@ static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     if (!theta || !lin || !out || n_theta < 0) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
     float* Aq;
-    if (from_scratch) {
-        const size_t Dt = (size_t)t->nC * t->ndim * (t->ndim + 1);
-        if ((size_t)n_theta * Dt * sizeof(float) > (size_t)CPAB_NOALLOC_SCRATCH_BYTES) return CPAB_ERR_SCRATCH;
+    if (where == AqIn::Scratch) {
+        if (aq_bytes(t, n_theta) > (size_t)CPAB_NOALLOC_SCRATCH_BYTES) return CPAB_ERR_SCRATCH;
         if ((rc = scratch_on_device(stream, &Aq))) return rc;
     } else {
-        if (ws_bytes < cpab_data_workspace_bytes(t, n_theta, outsize) || !workspace) return CPAB_ERR_WORKSPACE;
+        const size_t need =
+            where == AqIn::Buffer ? aq_bytes(t, n_theta) : cpab_data_workspace_bytes(t, n_theta, outsize);
+        if (ws_bytes < need || !workspace) return CPAB_ERR_WORKSPACE;
         Aq = static_cast<float*>(workspace);
     }
     Launch L;
@@ -2776,20 +2818,29 @@ static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
 int cpab_transform_data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
                             const int* dsize, const int* outsize, const float* lin, float t_end, float* out,
                             float* saved, void* workspace, size_t ws_bytes, hipStream_t stream) {
-    return data_fwd(t, theta, n_theta, data, C, dsize, outsize, lin, t_end, out, saved, workspace, ws_bytes, false,
+    return data_fwd(t, theta, n_theta, data, C, dsize, outsize, lin, t_end, out, saved, workspace, ws_bytes,
+                    AqIn::Workspace, stream);
+}
+
+int cpab_transform_data_fwd_keep(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
+                                 const int* dsize, const int* outsize, const float* lin, float t_end, float* out,
+                                 float* saved, float* Aq, size_t aq_size, hipStream_t stream) {
+    return data_fwd(t, theta, n_theta, data, C, dsize, outsize, lin, t_end, out, saved, Aq, aq_size, AqIn::Buffer,
                     stream);
 }
 
 int cpab_transform_data_fwd_noalloc(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
                                     const int* dsize, const int* outsize, const float* lin, float t_end, float* out,
                                     float* saved, hipStream_t stream) {
-    return data_fwd(t, theta, n_theta, data, C, dsize, outsize, lin, t_end, out, saved, nullptr, 0, true, stream);
+    return data_fwd(t, theta, n_theta, data, C, dsize, outsize, lin, t_end, out, saved, nullptr, 0,
+                    AqIn::Scratch, stream);
 }
 
-int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
-                            const int* dsize, const int* outsize, const float* lin, float t_end, const float* grad_out,
-                            const float* saved, float* grad_data, float* grad_theta, void* workspace, size_t ws_bytes,
-                            hipStream_t stream) {
+// The fused backward: A_q from kept, or (kept NULL) from theta into the workspace.
+static int data_bwd(const cpab_tess_t* t, const float* theta, const float* kept, int n_theta, const float* data, int C,
+                    const int* dsize, const int* outsize, const float* lin, float t_end, const float* grad_out,
+                    const float* saved, float* grad_data, float* grad_theta, void* workspace, size_t ws_bytes,
+                    hipStream_t stream) {
     int rc = check_tess(t);
     if (rc) return rc;
     Img im;
@@ -2797,7 +2848,7 @@ int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_thet
     int nP;
     if ((rc = img_from(t->ndim, data, C, dsize, im))) return rc;
     if ((rc = src_out(t->ndim, outsize, s, nP))) return rc;
-    if (!theta || !lin || !grad_out || !grad_theta || n_theta < 0) return CPAB_ERR_ARG;
+    if ((!theta && !kept) || !lin || !grad_out || !grad_theta || n_theta < 0) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
     if (ws_bytes < cpab_data_workspace_bytes(t, n_theta, outsize) || !workspace) return CPAB_ERR_WORKSPACE;
     Launch L;
@@ -2814,9 +2865,9 @@ int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_thet
     const size_t lds = lds_bwd(t->ndim, t->nC, t->nC + t->nV) + (size_t)box_cap * 4;
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     const int Dt = t->nC * t->ndim * (t->ndim + 1);
-    float* Aq = static_cast<float*>(workspace);
+    const float* Aq = kept ? kept : static_cast<const float*>(workspace);
     float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256((size_t)n_theta * Dt * 4));
-    if ((rc = launch_theta_to_A(t, theta, n_theta, Aq, stream))) return rc;
+    if (!kept && (rc = launch_theta_to_A(t, theta, n_theta, static_cast<float*>(workspace), stream))) return rc;
     im.gdata = grad_data;
     s.lin = lin;
     L.tiles = tile_count(t->ndim, nP, s.g0, s.g1, L.ppt, s.g2);
@@ -2843,6 +2894,22 @@ int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_thet
 #undef LAUNCH_DB3
     if ((rc = status_from_hip())) return rc;
     return launch_reduce(t, part, n_theta, nbt, grad_theta, stream);
+}
+
+int cpab_transform_data_bwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* data, int C,
+                            const int* dsize, const int* outsize, const float* lin, float t_end, const float* grad_out,
+                            const float* saved, float* grad_data, float* grad_theta, void* workspace, size_t ws_bytes,
+                            hipStream_t stream) {
+    return data_bwd(t, theta, nullptr, n_theta, data, C, dsize, outsize, lin, t_end, grad_out, saved, grad_data,
+                    grad_theta, workspace, ws_bytes, stream);
+}
+
+int cpab_transform_data_bwd_kept(const cpab_tess_t* t, const float* Aq, int n_theta, const float* data, int C,
+                                 const int* dsize, const int* outsize, const float* lin, float t_end,
+                                 const float* grad_out, const float* saved, float* grad_data, float* grad_theta,
+                                 void* workspace, size_t ws_bytes, hipStream_t stream) {
+    return data_bwd(t, nullptr, Aq, n_theta, data, C, dsize, outsize, lin, t_end, grad_out, saved, grad_data,
+                    grad_theta, workspace, ws_bytes, stream);
 }
 
 int cpab_findcell(int ndim, const int* nc, const float* points, int nP, int* idx, hipStream_t stream) {

@@ -8,6 +8,7 @@ the host.
 """
 import collections
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -64,6 +65,11 @@ class DeviceTess:
         ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=self.device)
         return ws, nbytes
 
+    def new_A(self, theta):
+        """Room for A = B theta of every theta; the forward fills it and the
+        backward, which saves it, reads it."""
+        return theta.new_empty((theta.shape[0], self.nC * self.ndim * (self.ndim + 1)))
+
 
 def device_tess(params, device):
     cache = getattr(params, "_device_tess", None)
@@ -97,11 +103,13 @@ def _check_unfinished(params):
 
 
 def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # the raw handle: a Stream object of torch.cuda.current_stream costs a microsecond per launch
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _require_gpu_f32(name, t):
@@ -112,11 +120,11 @@ def _require_gpu_f32(name, t):
         raise TypeError("%s must be float32, got %s" % (name, t.dtype))
 
 
+_INT3 = ctypes.c_int * 3
+
+
 def _int_arr(vals):
-    arr = (ctypes.c_int * 3)()
-    for i, v in enumerate(vals):
-        arr[i] = int(v)
-    return arr
+    return _INT3(*map(int, vals))
 
 
 # --------------------------------------------------------------------------
@@ -142,42 +150,42 @@ class TransformGrid(torch.autograd.Function):
             raise ValueError("a 3D grid needs one grid per theta")
         per_theta = int(points.dim() == 3)
         nP = points.shape[-1]
-        out = torch.empty(n_theta, ndim, nP, device=theta.device, dtype=torch.float32)
+        out = theta.new_empty((n_theta, ndim, nP))
         need = any(ctx.needs_input_grad[:2])
         jac = None
         store = getattr(params, "store_jacobian", True) if store_jac is None else store_jac
         if need and store:
-            jac = torch.empty(int(N.lib().cpab_jac_floats(ndim, n_theta, nP)), device=theta.device,
-                              dtype=torch.float32)
-        ws, nb = dev.workspace(n_theta, nP)
+            jac = theta.new_empty(N.lib().cpab_jac_floats(ndim, n_theta, nP))
+        Aq = dev.new_A(theta)
         shape = _int_arr(grid_shape) if grid_shape is not None else None
-        N.check(N.lib().cpab_transform_fwd(dev.ref, _ptr(theta), n_theta, _ptr(points), nP, per_theta, shape,
-                                           float(t_end), _ptr(out), _ptr(jac), _ptr(ws), nb, _stream(theta.device)))
+        N.check(N.lib().cpab_transform_fwd_keep(dev.ref, _ptr(theta), n_theta, _ptr(points), nP, per_theta, shape,
+                                                float(t_end), _ptr(out), _ptr(jac), _ptr(Aq), 4 * Aq.numel(),
+                                                _stream(theta.device)))
         _check_unfinished(params)
         ctx.params = params
-        ctx.t_end = t_end
+        ctx.t_end = float(t_end)
         ctx.per_theta = per_theta
         ctx.grid_shape = grid_shape
-        ctx.save_for_backward(points, theta, jac)
+        ctx.save_for_backward(points, theta, jac, Aq)
         return out
 
     @staticmethod
     @once_differentiable
     def backward(ctx, grad):
-        points, theta, jac = ctx.saved_tensors
+        points, theta, jac, Aq = ctx.saved_tensors
         dev = device_tess(ctx.params, theta.device)
         grad = grad.contiguous()
         n_theta = theta.shape[0]
         nP = points.shape[-1]
-        gtheta = torch.empty(n_theta, dev.d, device=theta.device, dtype=torch.float32)
+        gtheta = theta.new_empty((n_theta, dev.d))
         gpts = None
         if ctx.needs_input_grad[0]:
-            gpts = torch.empty(n_theta, dev.ndim, nP, device=theta.device, dtype=torch.float32)
+            gpts = theta.new_empty((n_theta, dev.ndim, nP))
         ws, nb = dev.workspace(n_theta, nP)
         shape = _int_arr(ctx.grid_shape) if ctx.grid_shape is not None else None
-        N.check(N.lib().cpab_transform_bwd(dev.ref, _ptr(theta), n_theta, _ptr(points), nP, ctx.per_theta, shape,
-                                           float(ctx.t_end), _ptr(grad), _ptr(jac), _ptr(gtheta), _ptr(gpts),
-                                           _ptr(ws), nb, _stream(theta.device)))
+        N.check(N.lib().cpab_transform_bwd_kept(dev.ref, _ptr(Aq), n_theta, _ptr(points), nP, ctx.per_theta, shape,
+                                                ctx.t_end, _ptr(grad), _ptr(jac), _ptr(gtheta), _ptr(gpts), _ptr(ws),
+                                                nb, _stream(theta.device)))
         if gpts is not None and not ctx.per_theta:
             gpts = gpts.sum(0)
         return gpts, (gtheta if ctx.needs_input_grad[1] else None), None, None, None, None
@@ -281,40 +289,45 @@ class TransformData(torch.autograd.Function):
             raise ValueError("theta must be [n_theta, %d], got %s" % (dev.d, tuple(theta.shape)))
         if data.dim() != dev.ndim + 2 or data.shape[0] != n_theta or len(outsize) != dev.ndim:
             raise ValueError("data must be [n_theta, C] + %d spatial dims" % dev.ndim)
-        nP = int(np.prod(outsize))
+        nP = math.prod(map(int, outsize))
         lin = meshgrid_axes(outsize, theta.device)
-        out = torch.empty((n_theta, C) + tuple(outsize), device=theta.device, dtype=torch.float32)
+        out = theta.new_empty((n_theta, C) + tuple(outsize))
         saved = None
         if any(ctx.needs_input_grad[:2]) and getattr(params, "store_jacobian", True):
-            saved = torch.empty(int(N.lib().cpab_saved_floats(dev.ndim, n_theta, nP)), device=theta.device,
-                                dtype=torch.float32)
-        plain = getattr(params, "launch", "batched") == "plain"
-        ws, nb = dev.workspace(1 if plain else n_theta, nP, outsize)
-        fn = N.lib().cpab_transform_data_fwd_plain if plain else N.lib().cpab_transform_data_fwd
+            saved = theta.new_empty(N.lib().cpab_saved_floats(dev.ndim, n_theta, nP))
+        Aq = None
+        if getattr(params, "launch", "batched") == "plain":
+            ws, nb = dev.workspace(1, nP, outsize)
+            fn = N.lib().cpab_transform_data_fwd_plain
+        else:
+            ws = Aq = dev.new_A(theta)
+            nb = 4 * Aq.numel()
+            fn = N.lib().cpab_transform_data_fwd_keep
         N.check(fn(dev.ref, _ptr(theta), n_theta, _ptr(data), C, _int_arr(data.shape[2:]), _int_arr(outsize),
                    _ptr(lin), float(t_end), _ptr(out), _ptr(saved), _ptr(ws), nb, _stream(theta.device)))
         _check_unfinished(params)
         ctx.params = params
         ctx.outsize = tuple(outsize)
-        ctx.t_end = t_end
-        ctx.save_for_backward(data, theta, lin, saved)
+        ctx.t_end = float(t_end)
+        ctx.save_for_backward(data, theta, lin, saved, Aq)
         return out
 
     @staticmethod
     @once_differentiable
     def backward(ctx, grad):
-        data, theta, lin, saved = ctx.saved_tensors
+        data, theta, lin, saved, Aq = ctx.saved_tensors
         dev = device_tess(ctx.params, theta.device)
         grad = grad.contiguous()
         n_theta = theta.shape[0]
         C = data.shape[1]
-        nP = int(np.prod(ctx.outsize))
+        nP = math.prod(ctx.outsize)
         gdata = torch.zeros_like(data) if ctx.needs_input_grad[0] else None
-        gtheta = torch.empty(n_theta, dev.d, device=theta.device, dtype=torch.float32)
-        plain = getattr(ctx.params, "launch", "batched") == "plain"
+        gtheta = theta.new_empty((n_theta, dev.d))
+        # a forward of launch='plain' keeps no A
+        plain = Aq is None or getattr(ctx.params, "launch", "batched") == "plain"
         ws, nb = dev.workspace(1 if plain else n_theta, nP, ctx.outsize)
-        fn = N.lib().cpab_transform_data_bwd_plain if plain else N.lib().cpab_transform_data_bwd
-        N.check(fn(dev.ref, _ptr(theta), n_theta, _ptr(data), C, _int_arr(data.shape[2:]), _int_arr(ctx.outsize),
-                   _ptr(lin), float(ctx.t_end), _ptr(grad), _ptr(saved), _ptr(gdata), _ptr(gtheta), _ptr(ws), nb,
-                   _stream(theta.device)))
+        fn = N.lib().cpab_transform_data_bwd_plain if plain else N.lib().cpab_transform_data_bwd_kept
+        N.check(fn(dev.ref, _ptr(theta if plain else Aq), n_theta, _ptr(data), C, _int_arr(data.shape[2:]),
+                   _int_arr(ctx.outsize), _ptr(lin), ctx.t_end, _ptr(grad), _ptr(saved), _ptr(gdata), _ptr(gtheta),
+                   _ptr(ws), nb, _stream(theta.device)))
         return gdata, (gtheta if ctx.needs_input_grad[1] else None), None, None, None
