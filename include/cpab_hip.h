@@ -291,6 +291,11 @@ int cpab_fill_zero(float* p, size_t n, hipStream_t stream);
  * which computes it with the Pade-13 of libcpab/pytorch/expm.py). */
 int cpab_expm_affine(const float* A, int n, int ndim, float scale, float* T, hipStream_t stream);
 
+/* As = B theta [n_theta, nC, ndim, ndim+1] and Trels = expm(A~ / nstepsolver) of
+ * every cell for the fixed-step scheme.  Replaces libcpab/pytorch/transformer.py:146-155. */
+int cpab_ref_expand(const cpab_tess_t* t, const float* theta, int n_theta, int nstepsolver, float* As, float* trels,
+                    hipStream_t stream);
+
 /* Same arguments and results as the reference's cpab_forward_op
  * (libcpab/core/cpab_ops.h:13-16, libcpab/core/cpab_ops.cpp:224-260) on device
  * pointers; nstepsolver by value, nc a host array.  Bit-exact with the

@@ -79,6 +79,7 @@ _SIGNATURES = {
     "cpab_batch_bwd_plain": (_c_int, [_c_ptr, _c_int, _c_float, _c_ptr]),
     "cpab_fill_zero": (_c_int, [_c_ptr, _c_size, _c_ptr]),
     "cpab_expm_affine": (_c_int, [_c_ptr, _c_int, _c_int, _c_float, _c_ptr, _c_ptr]),
+    "cpab_ref_expand": (_c_int, [ctypes.POINTER(CpabTess), _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr]),
     "cpab_ref_forward": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr]),
     "cpab_slow_forward": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]),
     "cpab_slow_backward": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr,

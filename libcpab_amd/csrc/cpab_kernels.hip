@@ -1827,11 +1827,9 @@ __global__ __launch_bounds__(RBLOCK) void k_batch_bt(const cpab_instance_t* __re
 // ---------------------------------------------------------------------------
 // expm(scale * A~) for n affine matrices A [D, D+1] (homogeneous last row 0),
 // FP64 scaling and squaring with a degree-12 Taylor polynomial; top D rows out.
+// T = the first D rows of expm(scale [A; 0]) in FP64; a, t: [D, D + 1]
 template <int D>
-__global__ __launch_bounds__(BLOCK) void k_expm_affine(const float* __restrict__ A, int n, float scale,
-                                                       float* __restrict__ T) {
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
+__device__ __forceinline__ void expm_affine(const float* a, double scale, float* t) {
     constexpr int E = D + 1;
     double X[E][E], R[E][E], Pw[E][E], tmp[E][E];
     double nrm = 0.0;
@@ -1839,7 +1837,7 @@ __global__ __launch_bounds__(BLOCK) void k_expm_affine(const float* __restrict__
     for (int r = 0; r < E; ++r)
 #pragma unroll
         for (int c = 0; c < E; ++c) {
-            X[r][c] = (r < D) ? (double)scale * (double)A[(size_t)i * D * E + r * E + c] : 0.0;
+            X[r][c] = (r < D) ? scale * (double)a[r * E + c] : 0.0;
             nrm += fabs(X[r][c]);
         }
     int sq = 0;
@@ -1892,7 +1890,42 @@ __global__ __launch_bounds__(BLOCK) void k_expm_affine(const float* __restrict__
 #pragma unroll
     for (int r = 0; r < D; ++r)
 #pragma unroll
-        for (int c = 0; c < E; ++c) T[(size_t)i * D * E + r * E + c] = (float)R[r][c];
+        for (int c = 0; c < E; ++c) t[r * E + c] = (float)R[r][c];
+}
+
+template <int D>
+__global__ __launch_bounds__(BLOCK) void k_expm_affine(const float* __restrict__ A, int n, float scale,
+                                                       float* __restrict__ T) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= n) return;
+    expm_affine<D>(A + (size_t)i * D * (D + 1), scale, T + (size_t)i * D * (D + 1));
+}
+
+// The fixed-step scheme's A = B theta (x-space) and Trels = expm(A~ / nstepsolver):
+// n_theta * ceil(nC / EXPAND_CELLS) blocks.  Latency bound: a few dozen FMAs per
+// entry, then one thread per cell for the series; in one launch 9 us, as a
+// product, a transposing copy and the series 15 and three times the host's work
+// ([3, 3], 8 thetas).
+constexpr int EXPAND_CELLS = 32;
+template <int D>
+__global__ __launch_bounds__(BLOCK) void k_ref_expand(const float* __restrict__ theta, const float* __restrict__ B,
+                                                      int d, int nC, double scale, float* __restrict__ As,
+                                                      float* __restrict__ trels) {
+    constexpr int P = D * (D + 1);
+    __shared__ float sA[EXPAND_CELLS * P];
+    const int nb = (nC + EXPAND_CELLS - 1) / EXPAND_CELLS, th = blockIdx.x / nb;
+    const int c0 = (blockIdx.x - th * nb) * EXPAND_CELLS, cells = min(EXPAND_CELLS, nC - c0);
+    const float* tk = theta + (size_t)th * d;
+    const size_t out = ((size_t)th * nC + c0) * P;
+    for (int i = threadIdx.x; i < cells * P; i += BLOCK) {
+        const float* b = B + ((size_t)c0 * P + i) * d;
+        float acc = 0.f;
+        for (int k = 0; k < d; ++k) acc = fmaf(b[k], tk[k], acc);
+        sA[i] = acc;
+        As[out + i] = acc;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < cells) expm_affine<D>(sA + threadIdx.x * P, scale, trels + out + threadIdx.x * P);
 }
 
 // libcpab/core/cpab_ops.cpp:224-260: grid (ceil(nP/BLOCK), batch); Trels of the
@@ -3216,6 +3249,21 @@ int cpab_expm_affine(const float* A, int n, int ndim, float scale, float* T, hip
     dim3 g((n + BLOCK - 1) / BLOCK);
 #define LAUNCH_EX(DD) hipLaunchKernelGGL((k_expm_affine<DD>), g, dim3(BLOCK), 0, stream, A, n, scale, T);
     CPAB_DISPATCH_D(ndim, LAUNCH_EX)
+#undef LAUNCH_EX
+    return status_from_hip();
+}
+
+int cpab_ref_expand(const cpab_tess_t* t, const float* theta, int n_theta, int nstepsolver, float* As, float* trels,
+                    hipStream_t stream) {
+    int rc = check_tess(t);
+    if (rc) return rc;
+    if (!theta || !As || !trels || !t->B || n_theta < 0 || nstepsolver < 1) return CPAB_ERR_ARG;
+    if (n_theta == 0) return CPAB_OK;
+    const dim3 g((unsigned)(t->nC + EXPAND_CELLS - 1) / EXPAND_CELLS * n_theta);
+    const double scale = 1.0 / nstepsolver;
+#define LAUNCH_EX(DD) \
+    hipLaunchKernelGGL((k_ref_expand<DD>), g, dim3(BLOCK), 0, stream, theta, t->B, t->d, t->nC, scale, As, trels);
+    CPAB_DISPATCH_D(t->ndim, LAUNCH_EX)
 #undef LAUNCH_EX
     return status_from_hip();
 }

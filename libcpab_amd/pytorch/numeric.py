@@ -18,27 +18,18 @@ from .. import _native as N
 from . import hip_ops as H
 
 
-def _trels(A, ndim, nstep):
-    """A [n, ndim, ndim+1] -> expm(A~/nstep)[:ndim]."""
-    A = A.contiguous()
-    T = torch.empty_like(A)
-    N.check(N.lib().cpab_expm_affine(H._ptr(A), A.shape[0], ndim, 1.0 / nstep, H._ptr(T), H._stream(A.device)))
-    return T
-
-
-def _expand(theta, dev, params):
-    As = (dev.B @ theta.t()).t().contiguous()  # [n_theta, D]
-    return As.view(theta.shape[0], params.nC, params.ndim, params.ndim + 1)
-
-
 def _forward(points, theta, params):
     dev = H.device_tess(params, theta.device)
     ndim, n_theta = params.ndim, theta.shape[0]
-    As = _expand(theta, dev, params)
-    trels = _trels(As.view(-1, ndim, ndim + 1), ndim, params.nstepsolver).view_as(As)
+    if theta.dim() != 2 or theta.shape[1] != dev.d:
+        raise RuntimeError("theta must be [n_theta, %d], got %s" % (dev.d, tuple(theta.shape)))
+    As = theta.new_empty((n_theta, params.nC, ndim, ndim + 1))
+    trels = torch.empty_like(As)
+    N.check(N.lib().cpab_ref_expand(dev.ref, H._ptr(theta), n_theta, int(params.nstepsolver), H._ptr(As),
+                                    H._ptr(trels), H._stream(theta.device)))
     broadcast = int(points.dim() == 3 and points.shape[0] == n_theta)
     nP = points.shape[-1]
-    out = torch.empty(n_theta, ndim, nP, device=theta.device, dtype=torch.float32)
+    out = theta.new_empty((n_theta, ndim, nP))
     N.check(N.lib().cpab_ref_forward(H._ptr(out), H._ptr(points), H._ptr(trels), int(params.nstepsolver),
                                      H._int_arr(params.nc), ndim, nP, n_theta, broadcast, H._stream(theta.device)))
     return out, As, broadcast

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import oracle as O
+from libcpab_amd import Cpab
 from libcpab_amd import _native as N
 from libcpab_amd.pytorch import hip_ops as H
 
@@ -93,3 +94,24 @@ def test_more_steps_than_the_lds_holds_take_the_derivatives(cuda):
         grads.append(torch.autograd.grad(T.transform_grid(pts, theta), theta, g)[0])
     # the scheme's own error at 50 steps is O(1 / steps^2); FP32 rounding over 40000
     assert (grads[0] - grads[1]).abs().max() <= 2e-2 * grads[0].abs().max()
+
+
+@pytest.mark.parametrize("nc,n", [([2], 1), ([40], 3), ([3, 3], 2), ([1, 1, 1], 2), ([2, 2, 3], 2)])
+def test_expanded_parameters_and_their_exponentials(cuda, nc, n):
+    """A = B theta and expm(A~ / nstep) of every cell, at cell counts around a block's 32, against FP64: A within the
+    rounding of its d products, the exponential within half an FP32 unit of that of the A returned."""
+    T = Cpab(nc, backend="pytorch", device="gpu", zero_boundary=len(nc) < 3)
+    dev = H.device_tess(T.params, cuda)
+    ndim, nC, d = len(nc), T.params.nC, T.get_theta_dim()
+    theta = torch.randn(n, d, generator=torch.Generator().manual_seed(1)).to(cuda)
+    As = torch.empty(n, nC, ndim, ndim + 1, device=cuda)
+    trels = torch.empty_like(As)
+    N.check(N.lib().cpab_ref_expand(dev.ref, H._ptr(theta), n, 50, H._ptr(As), H._ptr(trels), H._stream(theta.device)))
+    B, th = dev.B.double(), theta.double()
+    want = th.cpu() @ B.t().cpu()
+    size = th.abs().cpu() @ B.t().abs().cpu()
+    assert ((As.double().cpu().reshape(n, -1) - want).abs() <= (d + 1) * 2.0 ** -24 * size + 1e-30).all()
+    X = torch.zeros(n, nC, ndim + 1, ndim + 1, dtype=torch.float64)
+    X[:, :, :ndim] = As.double().cpu() / 50
+    E = torch.linalg.matrix_exp(X)[:, :, :ndim]
+    assert ((trels.double().cpu() - E).abs() <= 1.01 * 2.0 ** -24 * E.abs() + 2e-9 * X.abs().amax()).all()
