@@ -92,6 +92,7 @@ __host__ __device__ inline int tile_count(int ndim, int nP, int g0, int g1, int 
 
 // dL/ddata bins of a 2D tile: at most BIN_CELLS footprint cells (11-bit ids)
 constexpr int BIN_CELLS = 2048;
+constexpr int BOX_PPT = 2;  // points per thread of a tile with bins, at most
 
 // in-place exclusive prefix sum of v[0, n) by the whole block; v[n-1] becomes
 // the sum of the first n-1 entries
@@ -1064,13 +1065,14 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
     bool use_box = false;
     int bx0 = 0, by0 = 0, bh = 1, cells = 0;
     const int nslot = L.ppt * BLOCK;
-    int* code = reinterpret_cast<int*>(box);  // [nslot] lower corner i0 << 15 | j0, then bin | rank << 11; -1: none
-    int* bins = code + nslot;                 // [cells + 1] counts, then offsets
+    // this thread's points: lower corner i0 << 15 | j0, then bin | rank << 11; -1: none
+    int code[BOX_PPT] = {};
+    int* bins = reinterpret_cast<int*>(box);  // [cells + 1] counts, then offsets
     float2* fd2 = nullptr;                    // [nslot] corner weights (0 where a corner is clamped), bin order
     float4* gv4 = nullptr;                    // [nslot] grad_out of the channels, bin order
     if constexpr (D == 2 && HAVES) {
         // uniform over the block; corner indices must fit the 15-bit fields of code
-        if (box && gdata && nslot <= box_cap && im.s0 <= 32768 && im.s1 <= 32768) {
+        if (box && gdata && L.ppt <= BOX_PPT && im.s0 <= 32768 && im.s1 <= 32768) {
             if (threadIdx.x == 0) {
                 s_bb[0] = INT_MAX;
                 s_bb[1] = INT_MIN;
@@ -1079,15 +1081,16 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             }
             __syncthreads();
             int lo0 = INT_MAX, hi0 = INT_MIN, lo1 = INT_MAX, hi1 = INT_MIN;
-            for (int r = 0; r < L.ppt; ++r) {
-                const int t = tile_t<D>(L, s, tile, r);
-                code[r * BLOCK + threadIdx.x] = -1;
+#pragma unroll
+            for (int r = 0; r < BOX_PPT; ++r) {
+                const int t = r < L.ppt ? tile_t<D>(L, s, tile, r) : -1;
+                code[r] = -1;
                 if (t < 0) continue;
                 const float y[2] = {sv[t], sv[(size_t)L.nP + t]};
                 int i0[3], i1[3];
                 float fd[3];
                 corners<2>(y, im, i0, i1, fd);
-                code[r * BLOCK + threadIdx.x] = i0[0] << 15 | i0[1];
+                code[r] = i0[0] << 15 | i0[1];
                 lo0 = min(lo0, i0[0]);
                 hi0 = max(hi0, i1[0]);
                 lo1 = min(lo1, i0[1]);
@@ -1108,7 +1111,7 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             by0 = s_bb[2];
             bh = s_bb[3] - by0 + 1;
             cells = (s_bb[1] - bx0 + 1) * bh;
-            const long long slot0 = ((long long)nslot + cells + 1 + 3) & ~3LL;  // 16-byte aligned
+            const long long slot0 = ((long long)cells + 1 + 3) & ~3LL;  // 16-byte aligned
             use_box = bx0 != INT_MAX && im.C <= 4 && cells < BIN_CELLS && slot0 + 6LL * nslot <= box_cap;
             __syncthreads();  // s_bb is reused by the next tile of a persistent block
             if (use_box) {
@@ -1116,13 +1119,14 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                 gv4 = reinterpret_cast<float4*>(fd2 + nslot);
                 for (int i = threadIdx.x; i <= cells; i += BLOCK) bins[i] = 0;
                 __syncthreads();
-                // count the bins; each thread re-codes its own slots
-                for (int sl = threadIdx.x; sl < nslot; sl += BLOCK) {
-                    const int cd = code[sl];
+                // count the bins; each thread re-codes its own points
+#pragma unroll
+                for (int r = 0; r < BOX_PPT; ++r) {
+                    const int cd = code[r];
                     if (cd < 0) continue;
                     const int k = ((cd >> 15) - bx0) * bh + ((cd & 0x7FFF) - by0);
                     const int rank = atomicAdd(&bins[k], 1);
-                    code[sl] = k | (rank << 11);
+                    code[r] = k | (rank << 11);
                 }
                 __syncthreads();
                 block_exclusive_scan(bins, cells + 1);
@@ -1183,7 +1187,7 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                                             nP, gk, dfd);
                 if constexpr (D == 2) {
                     if (use_box) {
-                        const int cd = code[r * BLOCK + threadIdx.x];
+                        const int cd = r == 0 ? code[0] : code[1];
                         const int pos = bins[cd & 2047] + (cd >> 11);
                         // a clamped corner pair (i1 == i0) puts its whole weight on i0
                         fd2[pos] = make_float2(i1[0] != i0[0] ? fd[0] : 0.f, i1[1] != i0[1] ? fd[1] : 0.f);
@@ -2384,9 +2388,11 @@ int bwd_tiles_per_block(int ndim, int ty, int n_theta, int tiles) {
 }
 
 // LDS words for the dL/ddata bins and point slots of the fused 2D backward
-// (a 512-point tile needs 3584 + footprint cells + 1 words: up to 2047
-// cells, a 32 x 16 tile at up to ~2x magnification)
-constexpr int BOX_FLOATS = 6144;
+// (a 512-point tile needs 3072 + footprint cells + 1 words: up to 2047
+// cells, a 32 x 16 tile at up to ~2x magnification).  The points' bins stay in
+// registers: 512 words less and a block more per CU for the middle tessellations
+// ([6, 6], 40 x 100 x 90: 60.6 -> 47.7 us; 200 ragged problems 735 -> 654 us).
+constexpr int BOX_FLOATS = 5120;
 
 size_t lds_tables(int ndim, int nC) {  // nC: every cell of the facet table
     switch (ndim) {
