@@ -307,24 +307,133 @@ __device__ __forceinline__ int grad_cell(int cell, const Geo& g) {
     return cell;
 }
 
-// Pass 2 over one point per lane (wave-convergent); accumulates into acc.
-// The chunks recorded in lg by the forward are replayed (no facet search);
-// the rest are found again.
+// A point of pass 2 on its way: state, adjoint, and the chunks the forward recorded.
 template <int D>
-__device__ __forceinline__ void pass2(bool valid, const float (&q0)[D], int c0, float T, float (&mu)[D],
-                                      const CellTable<D>& tab, const Geo& g, float* acc, const ChunkLog& lg) {
-    constexpr int P = D * (D + 1);
+struct Pass2 {
     PointState<D> st;
+    float mu[D];
+    ChunkLog lg;
+    int nrec;
+    __device__ __forceinline__ bool active() const { return st.T > 0.f && st.iters < MAX_ITERS; }
+};
+template <int D>
+__device__ __forceinline__ Pass2<D> pass2_point(bool valid, const float (&q0)[D], int c0, float T,
+                                                const float (&mu)[D], const ChunkLog& lg) {
+    Pass2<D> w;
+    init_point<D>(w.st, q0, c0, valid ? T : 0.f);
 #pragma unroll
-    for (int a = 0; a < D; ++a) st.q[a] = q0[a];
-    st.T = valid ? T : 0.f;
-    st.c = c0;
-    st.came_from = -1;
-    st.zero_hops = 0;
-    st.iters = 0;
-    int nrec = lg.code & 3;
+    for (int a = 0; a < D; ++a) w.mu[a] = mu[a];
+    w.lg = lg;
+    w.nrec = lg.code & 3;
+    return w;
+}
+
+// ---------------------------------------------------------------------------
+// Points that have not ended with their first chunk wait in a stack of the wave's
+// own in LDS and go on together, a full wave of them at a time.
+//
+// A wave runs as many chunks as its longest trajectory has: 1.9 a round on
+// [4, 4] images where the mean is 1.3, 2.7 against 1.35 on [5, 7], 2.2 against
+// 1.15 on [3, 3, 3] volumes.  With the stack it is 1.4, 1.9 and 1.5.  Five eighths
+// of the capacity start a wave of deferred points; those of a round that do not fit
+// are run to their end in place (128 entries instead of 64 would save another 5% of
+// the chunks, and cost twice the LDS).  The order of a wave's chunks is a function of its points alone, so the
+// sums stay deterministic.
+// ---------------------------------------------------------------------------
+constexpr int DEFER_CAP = 64;
+constexpr int DEFER_ROUNDS = 4;  // rounds of a block from which the stack pays
+// Where it pays: 3D with saved state and without dL/ddata ([3, 3, 3], 16 x 64^3
+// points: 228 -> 213 us).  Its registers and LDS traffic cost what it gains in 2D
+// (images 667 -> 685, [8, 8] 348 -> 343, 200 ragged problems 950 -> 959 a pass) and
+// beside the merged scatter (3D with dL/ddata 328 -> 332).
+template <int D, bool HAVES, bool MERGE>
+constexpr bool stacked() { return D == 3 && HAVES && !MERGE; }
+constexpr int defer_words(int D) { return D > 1 ? 2 * D + 4 : 0; }  // per entry: q, mu, T, h, cells, counts
+
+template <int D>
+struct Deferred {
+    static constexpr int W = 2 * D + 4;
+    float2* w;  // [cap, W / 2] of this wave
+    int n, cap;
+    // base: WAVES * cap entries of LDS; cap 0: no stack
+    __device__ __forceinline__ void init(float* base, int capacity) {
+        n = 0;
+        cap = capacity;
+        w = reinterpret_cast<float2*>(base) + (threadIdx.x >> 6) * (cap * (W / 2));
+    }
+    // the lanes in mask (this one: in) go onto the stack; they fit
+    __device__ __forceinline__ void push(const Pass2<D>& p, uint64_t mask, bool in) {
+        const int i = n + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+        if (in) {
+            float v[W];
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                v[a] = p.st.q[a];
+                v[D + a] = p.mu[a];
+            }
+            v[2 * D] = p.st.T;
+            v[2 * D + 1] = p.lg.h[NREC - 1];  // the only recorded chunk that can be left
+            // the facet table in LDS holds a cell number below 2^15; past 8 the
+            // count of zero-length crossings makes no difference
+            v[2 * D + 2] = __int_as_float(p.st.c | (p.st.came_from + 1) << 16);
+            v[2 * D + 3] =
+                __int_as_float(p.st.iters | min(p.st.zero_hops, 255) << 10 | p.nrec << 18 | (p.lg.code & 0xFF) << 20);
+            float2* o = w + i * (W / 2);
+#pragma unroll
+            for (int k = 0; k < W / 2; ++k) o[k] = make_float2(v[2 * k], v[2 * k + 1]);
+        }
+        n += __popcll(mask);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // all entries, one per lane; the other lanes get points without time left
+    __device__ __forceinline__ Pass2<D> pop_all() {
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int lane = __lane_id();
+        float v[W] = {};
+        if (lane < n) {
+            const float2* o = w + lane * (W / 2);
+#pragma unroll
+            for (int k = 0; k < W / 2; ++k) {
+                const float2 u = o[k];
+                v[2 * k] = u.x;
+                v[2 * k + 1] = u.y;
+            }
+        }
+        Pass2<D> p;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            p.st.q[a] = v[a];
+            p.mu[a] = v[D + a];
+        }
+        p.st.T = v[2 * D];
+        p.lg.h[0] = 0.f;
+        p.lg.h[NREC - 1] = v[2 * D + 1];
+        const int cells = __float_as_int(v[2 * D + 2]);
+        const int counts = __float_as_int(v[2 * D + 3]);
+        p.st.c = cells & 0xFFFF;
+        p.st.came_from = (int)((unsigned)cells >> 16) - 1;
+        p.st.iters = counts & 0x3FF;
+        p.st.zero_hops = (counts >> 10) & 0xFF;
+        p.nrec = (counts >> 18) & 3;
+        p.lg.code = (counts >> 20) & 0xFF;
+        n = 0;
+        return p;
+    }
+};
+
+// Pass 2 over one point per lane (wave-convergent); accumulates into acc.
+// The chunks recorded by the forward are replayed (no facet search); the rest
+// are found again.  Points with time left after a chunk are deferred where they
+// fit.
+template <int D, bool STACK>
+__device__ __forceinline__ void pass2(Pass2<D>& w, const CellTable<D>& tab, const Geo& g, float* acc, Deferred<D>& df) {
+    constexpr int P = D * (D + 1);
+    PointState<D>& st = w.st;
     while (true) {
-        const bool active = st.T > 0.f && st.iters < MAX_ITERS;
+        const bool active = w.active();
         if (__ballot(active) == 0) break;
         int cell = -1;
         float G[P];
@@ -335,36 +444,51 @@ __device__ __forceinline__ void pass2(bool valid, const float (&q0)[D], int c0, 
                 Chunk1 ch;
                 advance1<false>(st, tab, g.nc0, ch);
                 float G1[2];
-                chunk_grad1(ch, mu[0], G1);
+                chunk_grad1(ch, w.mu[0], G1);
                 G[0] = G1[0];
                 G[1] = G1[1];
                 cell = ch.cell;
                 if (ch.facet >= 0) {
                     const float vn = fmaf(tab.A[2 * ch.next], ch.q1, tab.A[2 * ch.next + 1]);
                     const float vp = fmaf(ch.a, ch.q1, ch.b);
-                    mu[0] *= saltation1(vp, vn);
+                    w.mu[0] *= saltation1(vp, vn);
                 }
             } else {
                 Chunk<D> ch;
                 float h = 0.f;
                 int bf = -1;
-                if (st.iters < nrec) {
-                    logged_chunk(lg, st.iters, h, bf);
+                if (st.iters < w.nrec) {
+                    logged_chunk(w.lg, st.iters, h, bf);
                     // only a chunk the forward can have made is replayed (a
                     // saved state from another call is searched again instead)
-                    if (!(h >= 0.f && h <= st.T) || bf >= NF || (bf >= 0 && tab.nb[st.c * NF + bf] < 0)) nrec = 0;
+                    if (!(h >= 0.f && h <= st.T) || bf >= NF || (bf >= 0 && tab.nb[st.c * NF + bf] < 0)) w.nrec = 0;
                 }
-                if (st.iters < nrec)
+                if (st.iters < w.nrec)
                     replay<D>(st, tab, h, bf, ch);
                 else
                     advance<D>(st, tab, g.tol0, ch);
-                chunk_grad<D>(ch, mu, G);
+                chunk_grad<D>(ch, w.mu, G);
                 cell = ch.cell;
-                if (ch.facet >= 0) saltation_adj<D>(tab, ch, mu);
+                if (ch.facet >= 0) saltation_adj<D>(tab, ch, w.mu);
             }
         }
         wave_accumulate<P>(acc, grad_cell<D>(cell, g), G);
+        if constexpr (STACK) {
+            const bool left = w.active();
+            const uint64_t todo = __ballot(left);
+            if (todo && df.n + __popcll(todo) <= df.cap) {
+                df.push(w, todo, left);
+                break;
+            }
+        }
     }
+}
+
+// The next wave of pass 2: deferred points when there are enough of them or (end)
+// no others, else a round of new ones.  False: a new round (more) or none.
+template <int D>
+__device__ __forceinline__ bool take_deferred(const Deferred<D>& df, bool more, bool end) {
+    return (df.cap && df.n * 8 >= df.cap * 5) || (!more && end && df.n > 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1029,7 +1153,10 @@ __global__ __launch_bounds__(BLOCK, D == 2 ? 6 : 1) void k_transform_bwd(Launch 
                 for (int a = 0; a < D; ++a) gp[(size_t)a * L.nP + p] = mu[a] * (float)nc[a];
             }
         }
-        pass2<D>(valid, q0, c0, L.t_end, mu, tab, g, wacc, lg);
+        Pass2<D> pw = pass2_point<D>(valid, q0, c0, L.t_end, mu, lg);
+        Deferred<D> none;
+        none.init(nullptr, 0);
+        pass2<D, false>(pw, tab, g, wacc, none);
     }
     write_partials<D>(acc, part + ((size_t)th * L.tiles + tile) * nC * P, nC * P);
 }
@@ -1050,11 +1177,12 @@ __global__ __launch_bounds__(BLOCK, D == 2 ? 6 : 1) void k_transform_bwd(Launch 
 // 740 to 1506 us: the lanes that do not line up are scattered atomics.)
 //
 // MERGE: dL/ddata by merged_scatter, for the calls without the box.
-template <int D, bool HAVES, bool MERGE>
+template <int D, bool HAVES, bool MERGE, bool STACK>
 __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, const Src& s, const Img& im,
                                                const CellTable<D>& tab, int tile, const float* __restrict__ data,
                                                float* __restrict__ gdata, const float* __restrict__ gout,
-                                               const float* __restrict__ sv, float* wacc, float* box, int box_cap) {
+                                               const float* __restrict__ sv, float* wacc, float* box, int box_cap,
+                                               Deferred<D>& df, bool end) {
     const int nc[3] = {g.nc0, g.nc1, g.nc2};
     const float rnc[3] = {1.0f / (float)g.nc0, 1.0f / (float)g.nc1, 1.0f / (float)g.nc2};  // q -> x
     const int goff[3] = {0, s.g0, s.g0 + s.g1};
@@ -1133,7 +1261,8 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             }
         }
     }
-    for (int r = 0; r < L.ppt; ++r) {
+    // round r up to its second pass; false: no point of the wave
+    auto begin = [&](int r, Pass2<D>& w) __attribute__((always_inline)) {
         int ix[3];
         const int t = tile_t<D>(L, s, tile, r, ix);
         const size_t nP = per_round(L.nP);
@@ -1197,25 +1326,43 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             }
         }
         if constexpr (MERGE) {
-            if (__ballot(valid) == 0) continue;
+            if (__ballot(valid) == 0) return false;
             int i0[3], i1[3];
             float fd[3];
             corners<D>(y, im, i0, i1, fd);
             interp_backward_merged<D>(valid, data, gdata, dstride, im, i0, i1, fd, gout, valid ? t : 0, nP, L.ty, dfd);
         }
         if (valid) {
-            float w[D];
+            float gw[D];
 #pragma unroll
-            for (int a = 0; a < D; ++a) w[a] = dfd[a] * (float)(sz[a] - 1) * rnc[a];
+            for (int a = 0; a < D; ++a) gw[a] = dfd[a] * (float)(sz[a] - 1) * rnc[a];
 #pragma unroll
             for (int k = 0; k < D; ++k) {
                 float acc2 = 0.f;
 #pragma unroll
-                for (int a = 0; a < D; ++a) acc2 = fmaf(J[a][k], w[a], acc2);
+                for (int a = 0; a < D; ++a) acc2 = fmaf(J[a][k], gw[a], acc2);
                 mu[k] = acc2;
             }
         }
-        pass2<D>(valid, q0, c0, L.t_end, mu, tab, g, wacc, lg);
+        w = pass2_point<D>(valid, q0, c0, L.t_end, mu, lg);
+        return true;
+    };
+    if constexpr (STACK) {
+        for (int next = 0;;) {
+            Pass2<D> w;
+            if (take_deferred<D>(df, next < L.ppt, end))
+                w = df.pop_all();
+            else if (next >= L.ppt)
+                break;
+            else if (!begin(next++, w))
+                continue;
+            pass2<D, true>(w, tab, g, wacc, df);
+        }
+    } else {
+        for (int r = 0; r < L.ppt; ++r) {
+            Pass2<D> w;
+            if (begin(r, w)) pass2<D, false>(w, tab, g, wacc, df);
+        }
     }
     if (use_box) {
         __syncthreads();
@@ -1281,7 +1428,7 @@ template <int D, bool HAVES, bool MERGE>
 __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_data_bwd(Launch L, Geo g, Src s, Img im, const float* __restrict__ Aq,
                                                               const float* __restrict__ gout,
                                                               const float* __restrict__ saved, float* __restrict__ part,
-                                                              int box_cap, int tpb) {
+                                                              int box_cap, int tpb, int defer) {
     extern __shared__ float smem[];
     constexpr int P = D * (D + 1);
     const int nbt = bwd_blocks_per_theta(L.tiles, s.g1, L.ty, tpb);
@@ -1294,16 +1441,20 @@ __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_
     for (int i = threadIdx.x; i < WAVES * nC * P; i += BLOCK) acc[i] = 0.f;
     const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * nC * P, g);
     const size_t dstride = (size_t)im.s0 * (D > 1 ? im.s1 : 1) * (D > 2 ? im.s2 : 1);
+    float* box = acc + WAVES * nC * P;
+    Deferred<D> df;
+    df.init(box + box_cap, defer);
     for (int k = 0; k < tpb; ++k) {
         // tile row (bt / tiles_y) * tpb + k of tile column bt % tiles_y
         const int trow = (bt / tiles_y) * tpb + k;
         if (tpb > 1 && trow >= tiles_x) break;
         const int tile = tpb > 1 ? trow * tiles_y + bt % tiles_y : bt;
-        fused_bwd_tile<D, HAVES, MERGE>(L, g, s, im, tab, tile, im.data + (size_t)th * im.C * dstride,
+        fused_bwd_tile<D, HAVES, MERGE, stacked<D, HAVES, MERGE>()>(L, g, s, im, tab, tile, im.data + (size_t)th * im.C * dstride,
                                  im.gdata ? im.gdata + (size_t)th * im.C * dstride : nullptr,
                                  gout + (size_t)th * im.C * L.nP,
                                  HAVES ? saved + (size_t)th * saved_rows(D) * L.nP : nullptr,
-                                 acc + (threadIdx.x >> 6) * nC * P, box_cap ? acc + WAVES * nC * P : nullptr, box_cap);
+                                 acc + (threadIdx.x >> 6) * nC * P, box_cap ? box : nullptr, box_cap, df,
+                                 k == tpb - 1 || trow + 1 >= tiles_x);
     }
     write_partials<D>(acc, part + ((size_t)th * nbt + bt) * nC * P, nC * P);
 }
@@ -1719,8 +1870,10 @@ __device__ __forceinline__ void batch_bwd_item(float* smem, float* acc_base, flo
         for (int i = threadIdx.x; i < WAVES * nCP; i += BLOCK) acc[i] = 0.f;
     const CellTable<D> tab = restage ? stage_tables<D>(smem, static_cast<const float*>(I->ws), g) : table_view<D>(smem, g.nC + g.nV);
     if (!restage) __syncthreads();
-    fused_bwd_tile<D, HAVES, D != 2>(L, g, s, im, tab, tile, im.data, im.gdata, I->grad_out, I->saved,
-                             acc + (threadIdx.x >> 6) * nCP, box, box_cap);
+    Deferred<D> none;
+    none.init(nullptr, 0);
+    fused_bwd_tile<D, HAVES, D != 2, false>(L, g, s, im, tab, tile, im.data, im.gdata, I->grad_out, I->saved,
+                                     acc + (threadIdx.x >> 6) * nCP, box, box_cap, none, true);
     if (run_end) {
         float* part = reinterpret_cast<float*>(static_cast<char*>(I->ws) + align256_hd((size_t)nCP * 4));
         write_partials<D>(acc, part + (size_t)row * nCP, nCP);
@@ -2408,6 +2561,21 @@ size_t lds_bwd(int ndim, int nC, int nCt) { return lds_tables(ndim, nCt) + (size
 // LDS one workgroup may allocate on gfx950 (160 KB per CU, all of it per block)
 constexpr size_t LDS_LIMIT = 160 * 1024;
 
+// blocks of `bytes` dynamic LDS a CU holds (it gives LDS out in pieces of 1280
+// bytes; 256 more for the kernels' own variables)
+size_t blocks_per_cu(size_t bytes) { return LDS_LIMIT / ((bytes + 256 + 1279) / 1280 * 1280); }
+
+// Entries per wave of the 3D backward's stack beside base bytes of LDS: as many of
+// 64, 48, 32 as leave the CU its blocks (it has registers for 4), else 0.  A block
+// less costs more than the stack gives ([3, 3, 3]: 262 us with 2 blocks of 64
+// entries, 213 with 3 of 48, 228 without).
+int defer_entries(size_t base) {
+    const size_t blocks = blocks_per_cu(base), keep = blocks < 4 ? blocks : 4;
+    for (int cap = DEFER_CAP; keep && cap >= 32; cap -= 16)
+        if (blocks_per_cu(base + (size_t)defer_words(3) * cap * WAVES * 4) >= keep) return cap;
+    return 0;
+}
+
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 int status_from_hip() {
@@ -2901,7 +3069,10 @@ static int data_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
                          lds_bwd(t->ndim, t->nC, t->nC + t->nV) + (size_t)BOX_FLOATS * 4 <= LDS_LIMIT)
                             ? BOX_FLOATS
                             : 0;
-    const size_t lds = lds_bwd(t->ndim, t->nC, t->nC + t->nV) + (size_t)box_cap * 4;
+    const size_t base = lds_bwd(t->ndim, t->nC, t->nC + t->nV) + (size_t)box_cap * 4;
+    // deferred points: see stacked()
+    const int defer = (t->ndim == 3 && saved && !grad_data && L.ppt >= DEFER_ROUNDS) ? defer_entries(base) : 0;
+    const size_t lds = base + (size_t)defer_words(t->ndim) * defer * WAVES * 4;
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     const int Dt = t->nC * t->ndim * (t->ndim + 1);
     const float* Aq = kept ? kept : static_cast<const float*>(workspace);
@@ -2921,7 +3092,7 @@ static int data_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     const bool merge = grad_data && !box_cap;
 #define LAUNCH_DB3(DD, HAVES, MERGE)                                                                                  \
     hipLaunchKernelGGL((k_transform_data_bwd<DD, HAVES, MERGE>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq,     \
-                       grad_out, saved, part, box_cap, tpb)
+                       grad_out, saved, part, box_cap, tpb, defer)
 #define LAUNCH_DB(DD)                                                                \
     if (saved) {                                                                     \
         if (merge) LAUNCH_DB3(DD, true, true); else LAUNCH_DB3(DD, true, false);     \
