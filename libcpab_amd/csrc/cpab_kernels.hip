@@ -4,7 +4,7 @@
 // theta and a tile of 256*ppt points, its theta's per-cell parameters and the
 // facet table are staged in LDS; block ids are remapped so that all tiles of a
 // theta land on the same XCD and share its L2):
-//   k_theta_to_A        A = B theta, converted to q-space        (per theta)
+//   k_theta_to_A(_small)  A = B theta, converted to q-space
 //   k_transform         closed-form forward of explicit points    (transform_grid)
 //   k_transform_data    meshgrid -> closed-form -> interpolation  (transform_data)
 //   k_transform_bwd     adjoint of k_transform, dL/dA partials per tile (+ dL/dpoints)
@@ -871,10 +871,77 @@ __device__ __forceinline__ void interp_backward_merged(bool valid, const float* 
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-// A = B theta in q-space: grid (ceil(Dt/256), n_theta)
+// q-space over x-space of entry i of a theta's parameters
+__device__ __forceinline__ float x_scale(int i, int ndim, const int (&nc)[3]) {
+    const int rem = i % (ndim * (ndim + 1)), r = rem / (ndim + 1), col = rem % (ndim + 1);
+    return (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
+}
+
+// A = B theta in q-space: grid (ceil(Dt / 64), ceil(n_theta / (4 TT))).  A block
+// holds 64 rows of B in LDS, 64 columns at a time, for TT thetas in each of its
+// waves, a row per lane; an entry's products are added in the order of k.  A thread
+// that walked its own row from memory asked for 64 cache lines per load, once for
+// every theta.  us, before / after: [8, 8], 1024 thetas 280 / 28, 64 thetas 20 / 8.3;
+// [5, 5], 200 thetas 11.5 / 5.4; [50], 4096 thetas 9.8 / 5.9; [4, 4], 256 thetas
+// 6.6 / 5.4; [3, 3, 3], 16 thetas 6.1 / 4.8.
+constexpr int E_ROWS = 64, E_K = 64, E_STRIDE = E_K + 4;
+template <int TT>
 __global__ __launch_bounds__(BLOCK) void k_theta_to_A(const float* __restrict__ theta, const float* __restrict__ B,
-                                                      int d, int Dt, int ndim, int nc0, int nc1, int nc2,
+                                                      int n_theta, int d, int Dt, int ndim, int nc0, int nc1, int nc2,
                                                       float* __restrict__ Aq) {
+    __shared__ __align__(16) float sB[E_ROWS * E_STRIDE];
+    __shared__ __align__(16) float sT[WAVES * TT * E_K];
+    const int r0 = blockIdx.x * E_ROWS, row = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int t0 = blockIdx.y * (WAVES * TT);
+    float acc[TT] = {};
+    for (int k0 = 0; k0 < d; k0 += E_K) {
+        const int kn = min(E_K, d - k0);
+        if (k0 > 0) __syncthreads();
+        float bs[E_ROWS / WAVES], ts[TT];
+#pragma unroll
+        for (int i = 0; i < TT; ++i) {
+            const int t = t0 + w + WAVES * i;
+            ts[i] = row < kn && t < n_theta ? theta[(size_t)t * d + k0 + row] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < E_ROWS / WAVES; ++i) {
+            const int r = r0 + w + WAVES * i;
+            bs[i] = row < kn && r < Dt ? B[(size_t)r * d + k0 + row] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < TT; ++i) sT[(w + WAVES * i) * E_K + row] = ts[i];
+#pragma unroll
+        for (int i = 0; i < E_ROWS / WAVES; ++i) sB[(w + WAVES * i) * E_STRIDE + row] = bs[i];
+        __syncthreads();
+        const float *b = sB + row * E_STRIDE, *th = sT + w * TT * E_K;
+        int k = 0;
+#pragma unroll 4
+        for (; k + 4 <= kn; k += 4) {
+            const float4 bv = *reinterpret_cast<const float4*>(b + k);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const float4 tv = *reinterpret_cast<const float4*>(th + t * E_K + k);
+                acc[t] = fmaf(bv.w, tv.w, fmaf(bv.z, tv.z, fmaf(bv.y, tv.y, fmaf(bv.x, tv.x, acc[t]))));
+            }
+        }
+        for (; k < kn; ++k)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) acc[t] = fmaf(b[k], th[t * E_K + k], acc[t]);
+    }
+    const int i = r0 + row;
+    if (i >= Dt) return;
+    const int nc[3] = {nc0, nc1, nc2};
+    const float sc = x_scale(i, ndim, nc);
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+        if (t0 + w * TT + t < n_theta) Aq[(size_t)(t0 + w * TT + t) * Dt + i] = acc[t] * sc;
+}
+
+// The same, a thread per entry straight from memory, grid (ceil(Dt/256), n_theta):
+// for few products there is no reuse to gain and the staging's round trip shows.
+__global__ __launch_bounds__(BLOCK) void k_theta_to_A_small(const float* __restrict__ theta,
+                                                            const float* __restrict__ B, int d, int Dt, int ndim,
+                                                            int nc0, int nc1, int nc2, float* __restrict__ Aq) {
     extern __shared__ float sth[];
     const int th = blockIdx.y;
     for (int k = threadIdx.x; k < d; k += BLOCK) sth[k] = theta[(size_t)th * d + k];
@@ -884,11 +951,8 @@ __global__ __launch_bounds__(BLOCK) void k_theta_to_A(const float* __restrict__ 
     const float* b = B + (size_t)i * d;
     float acc = 0.f;
     for (int k = 0; k < d; ++k) acc = fmaf(b[k], sth[k], acc);
-    const int P = ndim * (ndim + 1);
-    const int rem = i % P, r = rem / (ndim + 1), col = rem % (ndim + 1);
     const int nc[3] = {nc0, nc1, nc2};
-    const float sc = (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
-    Aq[(size_t)th * Dt + i] = acc * sc;
+    Aq[(size_t)th * Dt + i] = acc * x_scale(i, ndim, nc);
 }
 
 template <int D, bool WITHJ>
@@ -1555,10 +1619,6 @@ __device__ __forceinline__ float rows_sum(const float* __restrict__ pp, int nrow
     if (t < nrows) s0 += pp[(size_t)rows(t) * Dt + i];
     return s0 + s1;
 }
-__device__ __forceinline__ float x_scale(int i, int ndim, const int (&nc)[3]) {
-    const int rem = i % (ndim * (ndim + 1)), r = rem / (ndim + 1), col = rem % (ndim + 1);
-    return (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
-}
 // this wave's share of (B^T sA)[k]: rows [i0, i1) of B, 16 loads in flight (the
 // last piece's missing rows count as 0 instead of being walked one by one)
 __device__ __forceinline__ float bt_sum(const float* __restrict__ B, const float* sA, int d, int k, int i0, int i1) {
@@ -1764,9 +1824,8 @@ __global__ __launch_bounds__(BLOCK) void k_fill_zero(float* p, size_t n) {
 // block.  The block reads them in pieces of 64 columns, coalesced, into LDS (odd
 // pitch); a lane of the first wave sums each row from there, in column order as
 // k_theta_to_A does.  The instances' bases are all different, so nothing is in
-// cache: a thread that walks its own row (k_theta_to_A, better where many thetas
-// share one B) asks for 64 cache lines per load, 29 us for the 200 instances of
-// a ragged batch against 12.
+// cache: a thread that walks its own row asks for 64 cache lines per load, 29 us
+// for the 200 instances of a ragged batch against 12.
 constexpr int A_ROWS = 64, A_PITCH = 65;
 __global__ __launch_bounds__(BLOCK) void k_batch_A(const cpab_instance_t* __restrict__ inst) {
     __shared__ float sB[A_ROWS * A_PITCH];
@@ -2584,11 +2643,28 @@ int status_from_hip() {
 }
 
 int launch_theta_to_A(const cpab_tess_t* t, const float* theta, int n_theta, float* Aq, hipStream_t st) {
-    const int Dt = t->nC * t->ndim * (t->ndim + 1);
-    dim3 grid((Dt + BLOCK - 1) / BLOCK, n_theta);
+    const int Dt = t->nC * t->ndim * (t->ndim + 1), rows = (Dt + E_ROWS - 1) / E_ROWS;
     Geo g = make_geo(t);
-    hipLaunchKernelGGL(k_theta_to_A, grid, dim3(BLOCK), t->d * sizeof(float), st, theta, t->B, t->d, Dt, t->ndim, g.nc0,
-                       g.nc1, g.nc2, Aq);
+    // up to 2^20 products: [3, 3], one theta 2.2 us against 3.2, 128 thetas 3.3
+    // against 3.6; [4, 4], 64 thetas (1.2 million) 4.8 against 4.7
+    if ((long long)n_theta * Dt * t->d <= 1 << 20) {
+        hipLaunchKernelGGL(k_theta_to_A_small, dim3((Dt + BLOCK - 1) / BLOCK, n_theta), dim3(BLOCK),
+                           t->d * sizeof(float), st, theta, t->B, t->d, Dt, t->ndim, g.nc0, g.nc1, g.nc2, Aq);
+        return status_from_hip();
+    }
+    // thetas per wave: as many of 1, 2, 4, 8 as leave 512 blocks
+    int tt = 1;
+    while (tt < 8 && (long long)rows * ((n_theta + 8 * tt - 1) / (8 * tt)) >= 512) tt *= 2;
+#define LAUNCH_E(TT)                                                                                             \
+    hipLaunchKernelGGL((k_theta_to_A<TT>), dim3(rows, (n_theta + WAVES * TT - 1) / (WAVES * TT)), dim3(BLOCK), 0, \
+                       st, theta, t->B, n_theta, t->d, Dt, t->ndim, g.nc0, g.nc1, g.nc2, Aq)
+    switch (tt) {
+        case 1: LAUNCH_E(1); break;
+        case 2: LAUNCH_E(2); break;
+        case 4: LAUNCH_E(4); break;
+        default: LAUNCH_E(8); break;
+    }
+#undef LAUNCH_E
     return status_from_hip();
 }
 
@@ -2601,7 +2677,12 @@ int launch_reduce(const cpab_tess_t* t, float* part, int n_theta, int tiles, flo
     // as the LDS holds [nw + 1, Dt] floats for, up to 16, but no more than 8192
     // waves in all: past that the blocks queue and their latencies add up ([50],
     // 4096 thetas, one row each: 37 us with 16 waves, 14 with 4).
-    if (n_theta >= 1024 || (n_theta >= 32 && tiles <= 64) || (size_t)tiles * Dt <= 8192) {
+    // B^T of a theta is then one CU's: with more than 2^15 entries of B that takes
+    // longer than two sliced launches ([5, 5], 32 thetas: 14.0 us against 10.1;
+    // [8, 8], 64: 61 against 23; [3, 3, 3], 40: 41 against 18; [4, 4], 256: 10.2
+    // against 12.8; [50], 4096: 14 against 39).
+    if ((size_t)Dt * t->d <= 32768 &&
+        (n_theta >= 1024 || (n_theta >= 32 && tiles <= 64) || (size_t)tiles * Dt <= 8192)) {
         int nw = RBLOCK / 64;
         while (nw > 4 && (long long)n_theta * nw > 8192) nw >>= 1;
         while (nw > 1 && (size_t)(nw + 1) * Dt * sizeof(float) > LDS_LIMIT) nw >>= 1;
