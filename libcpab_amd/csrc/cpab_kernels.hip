@@ -1525,20 +1525,27 @@ __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_
 
 // interpolation at an explicit grid [N, D, nP]; out [N, C, outsize], output order
 // The (instance n, output index t, grid index p) of this thread.  2D outputs
-// run in 16 x 16 blocks of 8 x 8 wave tiles, so the output accesses (last
-// axis fastest) and the grid accesses (first axis fastest) both come in runs
-// of 8 lanes; blocks: N * ceil(g0 / 16) * ceil(g1 / 16).  Other
-// dimensions run in output order.
-template <int D>
+// run in 16 x 16 blocks (N * ceil(g0 / 16) * ceil(g1 / 16) of them) of wave tiles
+// that are W wide along the last axis, on which the output, the upstream gradient
+// and the data's corners are contiguous, and 64 / W along the first, on which the
+// grid is: what counts is cache lines per access.  The forward reads the grid twice
+// a point and takes W = 16; the backward writes dL/dgrid too, and short runs cost
+// more in stores, so W = 8.  Neighbouring blocks halve each other's lines on both
+// sides, so they go to one XCD's L2.  64 x 256^2, 3 channels, us: W = 8 in launch
+// order 51 forward, 63.7 backward; in XCD order 49.7 and 55.5; W = 16 44.6 and 62.3.
+// (Two or four points per thread gained the forward nothing: 50.4, 54.1 at W = 8.)
+// Other dimensions run in output order.
+template <int D, int W>
 __device__ __forceinline__ bool interp_item(const Src& s, int N, int nP, int& n, int& t, int& p) {
     if constexpr (D == 2) {
         const int t0 = (s.g0 + 15) >> 4, t1 = (s.g1 + 15) >> 4;
-        const int b = blockIdx.x;
+        const int b = xcd_remap(blockIdx.x, gridDim.x);
         n = b / (t0 * t1);
         const int rem = b - n * t0 * t1;
         const int tid = threadIdx.x;
-        const int i0 = (rem / t1) * 16 + ((tid & 63) >> 3) + ((tid >> 7) << 3);
-        const int i1 = (rem % t1) * 16 + (tid & 7) + (((tid >> 6) & 1) << 3);
+        const int lane = tid & 63, w = tid >> 6;
+        const int i0 = (rem / t1) * 16 + lane / W + (W == 16 ? w * 4 : (w >> 1) * 8);
+        const int i1 = (rem % t1) * 16 + lane % W + (W == 16 ? 0 : (w & 1) * 8);
         if (n >= N || i0 >= s.g0 || i1 >= s.g1) return false;
         t = i0 * s.g1 + i1;
         p = i0 + s.g0 * i1;
@@ -1557,7 +1564,7 @@ __device__ __forceinline__ bool interp_item(const Src& s, int N, int nP, int& n,
 template <int D>
 __global__ __launch_bounds__(BLOCK) void k_interp_fwd(int N, int nP, Src s, Img im, float* __restrict__ out) {
     int n, t, p;
-    if (!interp_item<D>(s, N, nP, n, t, p)) return;
+    if (!interp_item<D, 16>(s, N, nP, n, t, p)) return;
     float y[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) y[a] = s.pts[((size_t)n * D + a) * nP + p];
@@ -1573,7 +1580,7 @@ template <int D>
 __global__ __launch_bounds__(BLOCK) void k_interp_bwd(int N, int nP, Src s, Img im, const float* __restrict__ gout,
                                                       float* __restrict__ ggrid) {
     int n = 0, t = 0, p = 0;
-    const bool valid = interp_item<D>(s, N, nP, n, t, p);
+    const bool valid = interp_item<D, 8>(s, N, nP, n, t, p);
     if (__ballot(valid) == 0) return;
     if (!valid) n = t = p = 0;
     float y[D];
