@@ -219,10 +219,47 @@ __device__ __forceinline__ CellTable<D> table_view(float* smem, int nC) {
     return t;
 }
 
+// q-space over x-space of entry i of a theta's parameters
+__device__ __forceinline__ float x_scale(int i, int ndim, const int (&nc)[3]) {
+    const int rem = i % (ndim * (ndim + 1)), r = rem / (ndim + 1), col = rem % (ndim + 1);
+    return (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
+}
+
+// A forward that makes A = B theta itself (theta not null): every block for its own
+// tables, a theta's first block into keep too.  Up to EXPAND_BLOCKS blocks and
+// EXPAND_PRODUCTS entries of B a launch of its own and the wait for it cost more
+// ([3, 3], one theta x 100^2 points, 5616 entries: 16.6 -> 14.5 us a pass, the kernel
+// 13.9 -> 18.0); beyond, the rows a block walks do ([4, 4], 256^2 points, 19200
+// entries: the kernel 19 -> 43 us).
+struct Expand {
+    const float* theta;
+    const float* B;
+    int d;
+    float* keep;
+};
+constexpr int EXPAND_BLOCKS = 256, EXPAND_PRODUCTS = 1 << 13;
+// entry i of A = B theta in q-space: the products in the order of k_theta_to_A, 16
+// loads in flight
+__device__ __forceinline__ float expand_entry(const Expand& ex, const float* theta, int i, const Geo& g) {
+    const float* b = ex.B + (size_t)i * ex.d;
+    float acc = 0.f;
+    for (int k = 0; k < ex.d; k += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = k + u < ex.d ? b[k + u] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            if (k + u < ex.d) acc = fmaf(v[u], theta[k + u], acc);
+    }
+    const int nc[3] = {g.nc0, g.nc1, g.nc2};
+    return acc * x_scale(i, g.ndim, nc);
+}
+
 // stage theta's q-space affine parameters, their inverse norms and the facet
 // table; a virtual cell gets a copy of the parameters of the simplex it uses
 template <int D>
-__device__ __forceinline__ CellTable<D> stage_tables(float* smem, const float* Aq, const Geo& g) {
+__device__ __forceinline__ CellTable<D> stage_tables(float* smem, const float* Aq, const Geo& g,
+                                                     const Expand* ex = nullptr, int th = 0, bool first = false) {
     constexpr int P = D * (D + 1);
     const int nC = g.nC;
     const int nCt = nC + g.nV;
@@ -231,9 +268,21 @@ __device__ __forceinline__ CellTable<D> stage_tables(float* smem, const float* A
     float* sInv = const_cast<float*>(t.inv_n);
     float4* sPl = const_cast<float4*>(t.pl);
     int* sNb = const_cast<int*>(t.nb);
-    for (int i = threadIdx.x; i < nC * P; i += BLOCK) sA[i] = Aq[i];
+    const bool make = ex && ex->theta;
+    if (make) {
+        const float* theta = ex->theta + (size_t)th * ex->d;
+        float* keep = ex->keep + (size_t)th * nC * P;
+        for (int i = threadIdx.x; i < nC * P; i += BLOCK) {
+            sA[i] = expand_entry(*ex, theta, i, g);
+            if (first) keep[i] = sA[i];
+        }
+        if (D == 3 && g.nV > 0) __syncthreads();
+    } else {
+        for (int i = threadIdx.x; i < nC * P; i += BLOCK) sA[i] = Aq[i];
+    }
     if constexpr (D == 3) {
-        for (int i = threadIdx.x; i < g.nV * P; i += BLOCK) sA[nC * P + i] = Aq[g.amap[i / P] * P + i % P];
+        const float* src = make ? sA : Aq;
+        for (int i = threadIdx.x; i < g.nV * P; i += BLOCK) sA[nC * P + i] = src[g.amap[i / P] * P + i % P];
     }
     if constexpr (D > 1) {
         for (int i = threadIdx.x; i < nCt * NF; i += BLOCK) {
@@ -871,12 +920,6 @@ __device__ __forceinline__ void interp_backward_merged(bool valid, const float* 
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-// q-space over x-space of entry i of a theta's parameters
-__device__ __forceinline__ float x_scale(int i, int ndim, const int (&nc)[3]) {
-    const int rem = i % (ndim * (ndim + 1)), r = rem / (ndim + 1), col = rem % (ndim + 1);
-    return (col < ndim) ? (float)nc[r] / (float)nc[col] : (float)nc[r];
-}
-
 // A = B theta in q-space: grid (ceil(Dt / 64), ceil(n_theta / (4 TT))).  A block
 // holds 64 rows of B in LDS, 64 columns at a time, for TT thetas in each of its
 // waves, a row per lane; an entry's products are added in the order of k.  A thread
@@ -956,14 +999,14 @@ __global__ __launch_bounds__(BLOCK) void k_theta_to_A_small(const float* __restr
 }
 
 template <int D, bool WITHJ>
-__global__ __launch_bounds__(BLOCK) void k_transform(Launch L, Geo g, Src s, const float* __restrict__ Aq,
+__global__ __launch_bounds__(BLOCK) void k_transform(Launch L, Geo g, Src s, Expand ex, const float* __restrict__ Aq,
                                                      float* __restrict__ out, float* __restrict__ jac) {
     extern __shared__ float smem[];
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
     const int th = lb / L.tiles, tile = lb % L.tiles;
     if (th >= L.n_theta) return;
     const int nC = g.nC;
-    const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * nC * D * (D + 1), g);
+    const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * nC * D * (D + 1), g, &ex, th, tile == 0);
     const int nc[3] = {g.nc0, g.nc1, g.nc2};
     const float rnc[3] = {1.0f / (float)g.nc0, 1.0f / (float)g.nc1, 1.0f / (float)g.nc2};  // q -> x
     const float* pts = s.pts + (s.per_theta ? (size_t)th * D * L.nP : 0);
@@ -1117,13 +1160,13 @@ __device__ __forceinline__ void fused_fwd_tile(const Launch& L, const Geo& g, co
 // 2D with saved state runs 6 waves per SIMD on 80 registers: 410 us against 424 at 5
 // on 84 (7 on 72 spill: 560); 3D loses to the spills (157 -> 182 at 5 on 96).
 template <int D, bool SAVE>
-__global__ __launch_bounds__(BLOCK, (D == 2 && SAVE) ? 6 : 1) void k_transform_data(Launch L, Geo g, Src s, Img im, const float* __restrict__ Aq,
+__global__ __launch_bounds__(BLOCK, (D == 2 && SAVE) ? 6 : 1) void k_transform_data(Launch L, Geo g, Src s, Img im, Expand ex, const float* __restrict__ Aq,
                                                           float* __restrict__ out, float* __restrict__ saved) {
     extern __shared__ float smem[];
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
     const int th = lb / L.tiles, tile = lb % L.tiles;
     if (th >= L.n_theta) return;
-    const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * g.nC * D * (D + 1), g);
+    const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * g.nC * D * (D + 1), g, &ex, th, tile == 0);
     const size_t dstride = (size_t)im.s0 * (D > 1 ? im.s1 : 1) * (D > 2 ? im.s2 : 1);
     fused_fwd_tile<D, SAVE>(L, g, s, im, tab, tile, im.data + (size_t)th * im.C * dstride,
                             out + (size_t)th * im.C * L.nP, SAVE ? saved + (size_t)th * saved_rows(D) * L.nP : nullptr);
@@ -2675,6 +2718,17 @@ int launch_theta_to_A(const cpab_tess_t* t, const float* theta, int n_theta, flo
     return status_from_hip();
 }
 
+// A_q for a forward of `blocks` blocks: made by the forward itself (returned), or by
+// a launch of its own.
+int expand_or_launch(const cpab_tess_t* t, const float* theta, int n_theta, long long blocks, float* Aq, hipStream_t st,
+                     Expand& ex) {
+    const long long Dt = (long long)t->nC * t->ndim * (t->ndim + 1);
+    ex = {nullptr, t->B, t->d, Aq};
+    if (blocks > EXPAND_BLOCKS || Dt * t->d > EXPAND_PRODUCTS) return launch_theta_to_A(t, theta, n_theta, Aq, st);
+    ex.theta = theta;
+    return CPAB_OK;
+}
+
 // dL/dtheta from the per-tile partials (overwritten).  Deterministic: fixed
 // summation order throughout.
 int launch_reduce(const cpab_tess_t* t, float* part, int n_theta, int tiles, float* gtheta, hipStream_t st) {
@@ -2862,7 +2916,6 @@ static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     const size_t lds = lds_tables(t->ndim, t->nC + t->nV);
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     float* Aq = static_cast<float*>(workspace);
-    if ((rc = launch_theta_to_A(t, theta, n_theta, Aq, stream))) return rc;
     Launch L;
     Src s = {};
     grid_launch(t, n_theta, nP, grid_shape, 0, L, s);
@@ -2871,11 +2924,13 @@ static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     s.pts = points;
     s.per_theta = per_theta_grid;
     dim3 grid(L.tiles * n_theta);
+    Expand ex;
+    if ((rc = expand_or_launch(t, theta, n_theta, (long long)L.tiles * n_theta, Aq, stream, ex))) return rc;
 #define LAUNCH_TF(DD)                                                                                                \
     if (jac)                                                                                                          \
-        hipLaunchKernelGGL((k_transform<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, Aq, out, jac);           \
+        hipLaunchKernelGGL((k_transform<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, ex, Aq, out, jac);           \
     else                                                                                                              \
-        hipLaunchKernelGGL((k_transform<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, Aq, out, jac);
+        hipLaunchKernelGGL((k_transform<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, ex, Aq, out, jac);
     CPAB_DISPATCH_D(t->ndim, LAUNCH_TF)
 #undef LAUNCH_TF
     return status_from_hip();
@@ -3094,17 +3149,18 @@ static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     L.ty = tile_ty(t->ndim, s.g1, s.g2);
     const size_t lds = lds_tables(t->ndim, t->nC + t->nV);
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
-    if ((rc = launch_theta_to_A(t, theta, n_theta, Aq, stream))) return rc;
     s.lin = lin;
     L.tiles = tile_count(t->ndim, nP, s.g0, s.g1, L.ppt, s.g2);
     L.t_end = t_end;
     Geo g = make_geo(t);
     dim3 grid(L.tiles * n_theta);
+    Expand ex;
+    if ((rc = expand_or_launch(t, theta, n_theta, (long long)L.tiles * n_theta, Aq, stream, ex))) return rc;
 #define LAUNCH_DF(DD)                                                                                                    \
     if (saved)                                                                                                            \
-        hipLaunchKernelGGL((k_transform_data<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq, out, saved);    \
+        hipLaunchKernelGGL((k_transform_data<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, im, ex, Aq, out, saved);    \
     else                                                                                                                  \
-        hipLaunchKernelGGL((k_transform_data<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq, out, saved);
+        hipLaunchKernelGGL((k_transform_data<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, im, ex, Aq, out, saved);
     CPAB_DISPATCH_D(t->ndim, LAUNCH_DF)
 #undef LAUNCH_DF
     return status_from_hip();

@@ -49,6 +49,25 @@ def test_kept_A_matches_the_calls_that_make_it_twice(cuda, nc, size, n):
     assert torch.equal(out, out2) and torch.equal(got, want)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("nc,zb", [([2], True), ([40], True), ([3, 3], True), ([2, 3], False), ([1, 2, 1], True),
+                                   ([1, 1, 1], False)])
+@pytest.mark.parametrize("n,nP", [(1, 1), (2, 300), (1, 65536), (1, 65537), (257, 20)])
+def test_the_forward_that_makes_A_leaves_the_same_bits(cuda, nc, zb, n, nP):
+    """Up to 256 blocks the forward makes A itself; cpab_theta_to_A is always a launch of its own."""
+    T = Cpab(nc, backend="pytorch", device="gpu", zero_boundary=zb)
+    L, dev = N.lib(), H.device_tess(T.params, cuda)
+    gen = torch.Generator().manual_seed(4)
+    theta = (torch.randn(n, T.params.d, generator=gen) * 0.2).to(cuda)
+    pts = (torch.rand(len(nc), nP, generator=gen) * 1.2 - 0.1).to(cuda)
+    A, want = dev.new_A(theta).fill_(float("nan")), dev.new_A(theta)
+    st, out = H._stream(theta.device), torch.empty(n, len(nc), nP, device=cuda)
+    N.check(L.cpab_transform_fwd_keep(dev.ref, theta.data_ptr(), n, pts.data_ptr(), nP, 0, None, 1.0, out.data_ptr(),
+                                      None, A.data_ptr(), 4 * A.numel(), st))
+    N.check(L.cpab_theta_to_A(dev.ref, theta.data_ptr(), n, want.data_ptr(), st))
+    assert torch.equal(A, want) and torch.isfinite(out).all()
+
+
 def test_kept_A_argument_errors():
     L, t = N.lib(), N.CpabTess()
     t.ndim, t.nc, t.nC, t.d, t.planes, t.nbr, t.B = 2, N.int3([2, 2]), 16, 10, 1, 1, 1
