@@ -67,6 +67,7 @@ struct CellTable {
     const float* inv_n;  // [nC]          1 / |Mq|_F (inf for Mq = 0)
     const float4* pl;    // [nC, NF]      (n0, n1, n2, e)
     const int* nb;       // [nC, NF]      neighbour, <0: none
+    const float2* hits = nullptr;  // 1D, nullable: [nC, 2] crossing a whole cell to the left, right: time, a dq / v0
 };
 
 template <int D>
@@ -800,6 +801,15 @@ CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& t
     h.r = 0.f;
     h.crosses = false;
     if (h.v0 != 0.f && h.next >= 0 && h.next < nx) {
+        if (EXACT && tab.hits && q0 == (h.right ? (float)c : (float)(c + 1))) {
+            // from edge to edge: the same for every point
+            const float2 f = tab.hits[2 * c + (h.right ? 1 : 0)];
+            h.th = f.x;
+            h.r = f.y;
+            const bool back = (st.zero_hops > 0 && h.next == st.came_from && h.th <= ZERO_HOP);
+            h.crosses = h.th < st.T && !back;
+            return h;
+        }
         const float dq = h.qb - q0;
         const float dt = EXACT ? dq / h.v0 : dq * near_rcp(h.v0);
         h.r = EXACT ? h.a * dq / h.v0 : h.a * dt;
@@ -810,6 +820,23 @@ CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& t
         }
     }
     return h;
+}
+// Entry of CellTable::hits: the crossing of the whole cell c to the left (dir 0) or
+// right, operation for operation that of a point that starts on the edge; a time
+// beyond any where there is none.
+CPAB_HD __forceinline__ float2 whole_cell(const CellTable<1>& tab, int c, int dir, int nx) {
+    PointState<1> st;
+    st.q[0] = dir ? (float)c : (float)(c + 1);
+    st.T = INFINITY;
+    st.c = c;
+    st.came_from = -1;
+    st.zero_hops = 0;
+    st.iters = 0;
+    const Hit1 h = hit1<true>(st, tab, nx);
+    float2 f;
+    f.x = h.crosses && h.right == (dir == 1) ? h.th : INFINITY;
+    f.y = h.r;
+    return f;
 }
 CPAB_HD __forceinline__ void hop1(PointState<1>& st, const Hit1& h) {
     st.T = fmaxf(st.T - h.th, 0.f);

@@ -42,6 +42,7 @@ struct Geo {
     int* unfinished;  // nullable: count of points that used up the chunk budget
     int nV;           // virtual cells after the nC simplices (3D outside the domain)
     const int* amap;  // [nV] simplex whose map each virtual cell uses
+    int hits;         // 1D: the tables hold the whole-cell crossings
 };
 
 
@@ -203,7 +204,8 @@ __device__ __forceinline__ int nc_at(const Geo& g, int a) {
     return a == 0 ? g.nc0 : (a == 1 ? g.nc1 : g.nc2);
 }
 
-// LDS layout of one theta's tables: A_q [nC*P], 1/|M|_F [nC (padded to 4)],
+// LDS layout of one theta's tables: A_q [nC*P], then in 1D the whole-cell crossings
+// [nC*2] float2 (up to HIT_CELLS cells), in 2D and 3D 1/|M|_F [nC (padded to 4)],
 // facet planes [nC*NF] float4, neighbours [nC*NF] int
 template <int D>
 __device__ __forceinline__ CellTable<D> table_view(float* smem, int nC) {
@@ -213,7 +215,7 @@ __device__ __forceinline__ CellTable<D> table_view(float* smem, int nC) {
     float* sInv = sA + nC * P;
     float4* sPl = reinterpret_cast<float4*>(sInv + ((nC + 3) & ~3));
     t.A = sA;
-    t.inv_n = sInv;
+    t.inv_n = D > 1 ? sInv : nullptr;
     t.pl = sPl;
     t.nb = reinterpret_cast<int*>(sPl + (D > 1 ? nC * NF : 0));
     return t;
@@ -291,6 +293,15 @@ __device__ __forceinline__ CellTable<D> stage_tables(float* smem, const float* A
         }
     }
     __syncthreads();
+    if constexpr (D == 1) {
+        if (g.hits) {
+            float2* sHit = reinterpret_cast<float2*>(sA + 2 * nC);
+            for (int i = threadIdx.x; i < 2 * nC; i += BLOCK) sHit[i] = whole_cell(t, i >> 1, i & 1, nC);
+            t.hits = sHit;
+            __syncthreads();
+        }
+        return t;
+    }
     for (int c = threadIdx.x; c < nCt; c += BLOCK) {
         float s = 0.f;
 #pragma unroll
@@ -313,9 +324,12 @@ __host__ __device__ constexpr int saved_rows(int D) { return D + D * D + (D > 1 
 // and, in 2D/3D, the chunk log.
 __host__ __device__ constexpr int jac_rows(int D) { return D * D + (D > 1 ? NREC + 1 : 0); }
 
+// Cells up to which the 1D tables have room for the whole-cell crossings.
+constexpr int HIT_CELLS = 512;
 template <int D>
 __host__ __device__ constexpr size_t table_floats(int nC) {
-    return (size_t)nC * D * (D + 1) + ((nC + 3) & ~3) + (D > 1 ? (size_t)nC * NF * 4 + (size_t)nC * NF : 0);
+    if (D == 1) return (size_t)nC * (nC <= HIT_CELLS ? 6 : 2);
+    return (size_t)nC * D * (D + 1) + ((nC + 3) & ~3) + (size_t)nC * NF * 4 + (size_t)nC * NF;
 }
 
 // Start cell of a point: the lookup, except that a 3D point outside the
@@ -1826,6 +1840,7 @@ __device__ __forceinline__ void item_args(const cpab_instance_t* I, int ppt, flo
     g.unfinished = I->tess.unfinished;
     g.nV = I->tess.nV;
     g.amap = I->tess.amap;
+    g.hits = 0;
     int m = g.nc0 > g.nc1 ? g.nc0 : g.nc1;
     m = m > g.nc2 ? m : g.nc2;
     g.tol0 = 2e-6f * (float)m;
@@ -2606,10 +2621,21 @@ Geo make_geo(const cpab_tess_t* t) {
     g.unfinished = t->unfinished;
     g.nV = t->nV;
     g.amap = t->amap;
+    g.hits = 0;
     int m = g.nc0 > g.nc1 ? g.nc0 : g.nc1;
     m = m > g.nc2 ? m : g.nc2;
     g.tol0 = 2e-6f * (float)(m > 1 ? m : 1);
     return g;
+}
+
+// 1D forwards make the table of whole-cell crossings where a thread's share of it
+// (one crossing per 64 cells) is at most one for each of its points, of which it has
+// several: a wave on signals of 1024 points over 50 cells runs 2.65 chunks a point, and
+// all but the first start on an edge.  us, before / after: 4096 of those 64.8 / 49.0,
+// 500 of 8000 points over 80 cells 61.6 / 50.2.  (The gradient's pass, whose
+// crossings are cheaper, lost by it: 65.2 -> 67.9.)
+int use_hits(const cpab_tess_t* t, int ppt) {
+    return t->ndim == 1 && t->nC <= HIT_CELLS && ppt > 1 && t->nC <= 64 * ppt;
 }
 
 // points per thread: the largest of 8, 4, 2, 1 that still gives >= 16 blocks
@@ -2921,6 +2947,7 @@ static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     grid_launch(t, n_theta, nP, grid_shape, 0, L, s);
     L.t_end = t_end;
     Geo g = make_geo(t);
+    g.hits = use_hits(t, L.ppt);
     s.pts = points;
     s.per_theta = per_theta_grid;
     dim3 grid(L.tiles * n_theta);
@@ -3153,6 +3180,7 @@ static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     L.tiles = tile_count(t->ndim, nP, s.g0, s.g1, L.ppt, s.g2);
     L.t_end = t_end;
     Geo g = make_geo(t);
+    g.hits = use_hits(t, L.ppt);
     dim3 grid(L.tiles * n_theta);
     Expand ex;
     if ((rc = expand_or_launch(t, theta, n_theta, (long long)L.tiles * n_theta, Aq, stream, ex))) return rc;
