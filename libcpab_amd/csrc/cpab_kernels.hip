@@ -635,18 +635,19 @@ __device__ __forceinline__ float blend(const float (&v)[1 << D], const float (&f
 }
 
 // value of channel data dp at the corners (i0, i1, fd)
-// base[i], base uniform over the wave: in 2D and 3D, where the chunk log's 32-bit
-// row bounds keep an instance's points below 2^29, as a scalar base and a 32-bit
-// byte offset (a 64-bit address is two more instructions per access).
-template <int D>
+// base[i], base uniform over the wave.  NARROW: as a scalar base and a 32-bit byte
+// offset (a 64-bit address is two more instructions per access), for an instance's
+// points in 2D and 3D calls with saved state, whose chunk log's 32-bit row bounds
+// keep them below 2^29.
+template <bool NARROW>
 __device__ __forceinline__ float at(const float* base, int i) {
-    if constexpr (D == 1) return base[i];
+    if constexpr (!NARROW) return base[i];
     asm("" : "+s"(base));
     return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + ((unsigned)i << 2));
 }
-template <int D>
+template <bool NARROW>
 __device__ __forceinline__ void put(float* base, int i, float v) {
-    if constexpr (D == 1) {
+    if constexpr (!NARROW) {
         base[i] = v;
     } else {
         asm("" : "+s"(base));
@@ -684,7 +685,7 @@ constexpr int chan_group_bwd() { return D == 2 ? 2 : 1; }
 // out[c * ostride] = channel c (data + c * dstride) at the corners, for every
 // channel.  The loads of a group of channels are all issued before the first
 // of them is used, so their latencies overlap instead of adding up.
-template <int D>
+template <int D, bool NARROW>
 __device__ __forceinline__ void interp_channels(const float* __restrict__ data, size_t dstride, const Img& im,
                                                 const int (&i0)[3], const int (&i1)[3], const float (&fd)[3],
                                                 float* __restrict__ out, int t, size_t ostride) {
@@ -702,7 +703,7 @@ __device__ __forceinline__ void interp_channels(const float* __restrict__ data, 
             }
 #pragma unroll
         for (int k = 0; k < CG; ++k)
-            if (c0 + k < im.C) put<D>(out + (size_t)(c0 + k) * ostride, t, blend<D>(v[k], fd));
+            if (c0 + k < im.C) put<NARROW>(out + (size_t)(c0 + k) * ostride, t, blend<D>(v[k], fd));
     }
 }
 
@@ -855,7 +856,7 @@ __device__ __forceinline__ void blend_backward(const float (&v)[1 << D], const f
 // over the channels, in channel order, and gdata (nullable) one atomic per
 // corner.  The loads of a group of channels are issued before any of them is
 // used.
-template <int D>
+template <int D, bool NARROW>
 __device__ __forceinline__ void interp_backward_channels(const float* __restrict__ data, float* gdata, size_t dstride,
                                                          const Img& im, const int (&i0)[3], const int (&i1)[3],
                                                          const float (&fd)[3], const float* __restrict__ gout,
@@ -869,7 +870,7 @@ __device__ __forceinline__ void interp_backward_channels(const float* __restrict
         for (int k = 0; k < CG; ++k)
             if (c0 + k < im.C) {
                 const float* dp = data + (size_t)(c0 + k) * dstride;
-                gv[k] = at<D>(gout + (size_t)(c0 + k) * gstride, t);
+                gv[k] = at<NARROW>(gout + (size_t)(c0 + k) * gstride, t);
 #pragma unroll
                 for (int j = 0; j < NK; ++j) v[k][j] = dp[off[j]];
             }
@@ -1125,6 +1126,7 @@ template <int D, bool SAVE>
 __device__ __forceinline__ void fused_fwd_tile(const Launch& L, const Geo& g, const Src& s, const Img& im,
                                                const CellTable<D>& tab, int tile, const float* __restrict__ data,
                                                float* __restrict__ out, float* __restrict__ sv) {
+    constexpr bool NARROW = SAVE && D > 1;
     const int nc[3] = {g.nc0, g.nc1, g.nc2};
     const float rnc[3] = {1.0f / (float)g.nc0, 1.0f / (float)g.nc1, 1.0f / (float)g.nc2};  // q -> x
     const int goff[3] = {0, s.g0, s.g0 + s.g1};
@@ -1140,7 +1142,7 @@ __device__ __forceinline__ void fused_fwd_tile(const Launch& L, const Geo& g, co
         float x[D], q[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            x[a] = at<D>(s.lin, goff[a] + ix[a]);
+            x[a] = at<NARROW>(s.lin, goff[a] + ix[a]);
             q[a] = x[a] * (float)nc[a];
         }
         const int c0 = start_cell<D>(x, nc, tab, g);
@@ -1155,17 +1157,17 @@ __device__ __forceinline__ void fused_fwd_tile(const Launch& L, const Geo& g, co
         if constexpr (SAVE) {
             // indexed in output order t (the order threads run in) for coalesced stores
 #pragma unroll
-            for (int a = 0; a < D; ++a) put<D>(sv + a * nP, t, y[a]);
+            for (int a = 0; a < D; ++a) put<NARROW>(sv + a * nP, t, y[a]);
 #pragma unroll
             for (int r2 = 0; r2 < D; ++r2)
 #pragma unroll
-                for (int k = 0; k < D; ++k) put<D>(sv + (D + r2 * D + k) * nP, t, J[r2][k]);
-            if constexpr (D > 1) put<D>(sv + (D + D * D + NREC) * nP, t, __int_as_float(lg.code));
+                for (int k = 0; k < D; ++k) put<NARROW>(sv + (D + r2 * D + k) * nP, t, J[r2][k]);
+            if constexpr (D > 1) put<NARROW>(sv + (D + D * D + NREC) * nP, t, __int_as_float(lg.code));
         }
         int i0[3], i1[3];
         float fd[3];
         corners<D>(y, im, i0, i1, fd);
-        interp_channels<D>(data, dstride, im, i0, i1, fd, out, t, nP);
+        interp_channels<D, NARROW>(data, dstride, im, i0, i1, fd, out, t, nP);
         wave_bad += __popcll(__ballot(y[0] != y[0]));
     }
     if (wave_bad && g.unfinished && __lane_id() == 0) atomicAdd(g.unfinished, wave_bad);
@@ -1304,6 +1306,7 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                                                float* __restrict__ gdata, const float* __restrict__ gout,
                                                const float* __restrict__ sv, float* wacc, float* box, int box_cap,
                                                Deferred<D>& df, bool end) {
+    constexpr bool NARROW = HAVES && D > 1;
     const int nc[3] = {g.nc0, g.nc1, g.nc2};
     const float rnc[3] = {1.0f / (float)g.nc0, 1.0f / (float)g.nc1, 1.0f / (float)g.nc2};  // q -> x
     const int goff[3] = {0, s.g0, s.g0 + s.g1};
@@ -1405,21 +1408,21 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
             float x[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                x[a] = at<D>(s.lin, goff[a] + ix[a]);
+                x[a] = at<NARROW>(s.lin, goff[a] + ix[a]);
                 q0[a] = x[a] * (float)nc[a];
             }
             c0 = start_cell<D>(x, nc, tab, g);
             if constexpr (HAVES) {
 #pragma unroll
-                for (int a = 0; a < D; ++a) y[a] = at<D>(sv + a * nP, t);
+                for (int a = 0; a < D; ++a) y[a] = at<NARROW>(sv + a * nP, t);
 #pragma unroll
                 for (int r2 = 0; r2 < D; ++r2)
 #pragma unroll
-                    for (int k = 0; k < D; ++k) J[r2][k] = at<D>(sv + (D + r2 * D + k) * nP, t);
+                    for (int k = 0; k < D; ++k) J[r2][k] = at<NARROW>(sv + (D + r2 * D + k) * nP, t);
                 if constexpr (D > 1) {
 #pragma unroll
-                    for (int k = 0; k < NREC; ++k) lg.h[k] = at<D>(sv + (D + D * D + k) * nP, t);
-                    lg.code = __float_as_int(at<D>(sv + (D + D * D + NREC) * nP, t));
+                    for (int k = 0; k < NREC; ++k) lg.h[k] = at<NARROW>(sv + (D + D * D + k) * nP, t);
+                    lg.code = __float_as_int(at<NARROW>(sv + (D + D * D + NREC) * nP, t));
                 }
             } else {
                 float q[D];
@@ -1433,7 +1436,7 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                 int i0[3], i1[3];
                 float fd[3], gk[4] = {0.f, 0.f, 0.f, 0.f};
                 corners<D>(y, im, i0, i1, fd);
-                interp_backward_channels<D>(data, (D != 2 || use_box) ? nullptr : gdata, dstride, im, i0, i1, fd, gout, t,
+                interp_backward_channels<D, NARROW>(data, (D != 2 || use_box) ? nullptr : gdata, dstride, im, i0, i1, fd, gout, t,
                                             nP, gk, dfd);
                 if constexpr (D == 2) {
                     if (use_box) {

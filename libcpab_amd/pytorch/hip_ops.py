@@ -320,7 +320,7 @@ class TransformData(torch.autograd.Function):
         grad = grad.contiguous()
         n_theta = theta.shape[0]
         C = data.shape[1]
-        nP = math.prod(ctx.outsize)
+        nP = math.prod(map(int, ctx.outsize))
         gdata = torch.zeros_like(data) if ctx.needs_input_grad[0] else None
         gtheta = theta.new_empty((n_theta, dev.d))
         # a forward of launch='plain' keeps no A
