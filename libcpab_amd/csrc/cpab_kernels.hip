@@ -1735,6 +1735,76 @@ __global__ __launch_bounds__(RBLOCK) void k_reduce_theta(const float* __restrict
 // one block, whose result overwrites row 0 of the partials (each block owns its
 // columns and has read them all first); then 64 entries of dL/dtheta by one
 // block.  Slices give a few thetas enough blocks to fill the chip.
+// Many thetas with few rows each: grid (ceil(d / 64), ceil(n_theta / (4 TT))).  A
+// block takes 64 columns of B, 64 rows at a time through LDS, for TT thetas in each
+// of its waves, a column per lane; the rows of partials are summed as they are read.
+// A block per theta read all of B for each.  us, before / after: [50], 4096 thetas
+// 14.7 / 8.2; [100], 2000 thetas 21.9 / 14.6; [8, 8], 1024 thetas of 8 rows 148 / 125.
+// With a small B and 8 rows the one-block form, whose waves share the rows, is better ([2, 2], 1100
+// thetas: 6.8 against 8.6).
+constexpr int MANY_THETAS = 1024, MANY_ROWS = 4;
+template <int TT>
+__global__ __launch_bounds__(BLOCK) void k_reduce_many(const float* __restrict__ part, int n_theta, int tiles, int Dt,
+                                                       int ndim, int nc0, int nc1, int nc2,
+                                                       const float* __restrict__ B, int d, float* __restrict__ gtheta) {
+    __shared__ __align__(16) float sB[64 * 64];
+    __shared__ __align__(16) float sG[WAVES * TT * 64];
+    const int nc[3] = {nc0, nc1, nc2};
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + lane, t0 = blockIdx.y * (WAVES * TT);
+    float acc[TT] = {};
+    for (int i0 = 0; i0 < Dt; i0 += 64) {
+        const int in = min(64, Dt - i0), i = i0 + lane;
+        float gs[TT], bs[64 / WAVES];
+#pragma unroll
+        for (int u = 0; u < 64 / WAVES; ++u) {
+            const int r = i0 + w + WAVES * u;
+            bs[u] = r < Dt && k < d ? B[(size_t)r * d + k] : 0.f;
+        }
+        const float sc = i < Dt ? x_scale(i, ndim, nc) : 0.f;
+#pragma unroll
+        for (int u = 0; u < TT; ++u) {
+            const int t = t0 + w + WAVES * u;
+            float g = 0.f;
+            if (i < Dt && t < n_theta) {
+                const float* pp = part + (size_t)t * tiles * Dt + i;
+                g = pp[0];
+                for (int r = 1; r < tiles; ++r) g += pp[(size_t)r * Dt];
+            }
+            gs[u] = g * sc;
+        }
+        if (i0 > 0) __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 64 / WAVES; ++u) sB[(w + WAVES * u) * 64 + lane] = bs[u];
+#pragma unroll
+        for (int u = 0; u < TT; ++u) sG[(w + WAVES * u) * 64 + lane] = gs[u];
+        __syncthreads();
+        const float* g = sG + w * TT * 64;
+        float p[TT] = {};
+        int j = 0;
+#pragma unroll 2
+        for (; j + 4 <= in; j += 4) {
+            float b[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) b[u] = sB[(j + u) * 64 + lane];
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const float4 v = *reinterpret_cast<const float4*>(g + t * 64 + j);
+                p[t] = fmaf(b[3], v.w, fmaf(b[2], v.z, fmaf(b[1], v.y, fmaf(b[0], v.x, p[t]))));
+            }
+        }
+        for (; j < in; ++j)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) p[t] = fmaf(sB[j * 64 + lane], g[t * 64 + j], p[t]);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[t] += p[t];
+    }
+    if (k >= d) return;
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+        if (t0 + w * TT + t < n_theta) gtheta[(size_t)(t0 + w * TT + t) * d + k] = acc[t];
+}
+
 template <class Rows>
 __device__ __forceinline__ void reduce_cols(float* sg, float* __restrict__ pp, int nrows, int Dt, int c0, int c1,
                                             int ndim, const int (&nc)[3], Rows rows) {
@@ -2763,6 +2833,24 @@ int expand_or_launch(const cpab_tess_t* t, const float* theta, int n_theta, long
 int launch_reduce(const cpab_tess_t* t, float* part, int n_theta, int tiles, float* gtheta, hipStream_t st) {
     const int Dt = t->nC * t->ndim * (t->ndim + 1);
     Geo g = make_geo(t);
+    const bool large_b = (size_t)Dt * t->d > 32768;
+    if (n_theta >= MANY_THETAS && tiles <= (large_b ? 2 * MANY_ROWS : MANY_ROWS)) {
+        const int cols = (t->d + 63) / 64;
+        // thetas per wave: as many of 1, 2, 4, 8 as leave 512 blocks
+        int tt = 1;
+        while (tt < 8 && (long long)cols * ((n_theta + 8 * tt - 1) / (8 * tt)) >= 512) tt *= 2;
+#define LAUNCH_M(TT)                                                                                               \
+    hipLaunchKernelGGL((k_reduce_many<TT>), dim3(cols, (n_theta + WAVES * TT - 1) / (WAVES * TT)), dim3(BLOCK), 0, \
+                       st, part, n_theta, tiles, Dt, t->ndim, g.nc0, g.nc1, g.nc2, t->B, t->d, gtheta)
+        switch (tt) {
+            case 1: LAUNCH_M(1); break;
+            case 2: LAUNCH_M(2); break;
+            case 4: LAUNCH_M(4); break;
+            default: LAUNCH_M(8); break;
+        }
+#undef LAUNCH_M
+        return status_from_hip();
+    }
     // One block per theta with enough thetas, or with few rows each; as many waves
     // as the LDS holds [nw + 1, Dt] floats for, up to 16, but no more than 8192
     // waves in all: past that the blocks queue and their latencies add up ([50],
@@ -2771,7 +2859,7 @@ int launch_reduce(const cpab_tess_t* t, float* part, int n_theta, int tiles, flo
     // longer than two sliced launches ([5, 5], 32 thetas: 14.0 us against 10.1;
     // [8, 8], 64: 61 against 23; [3, 3, 3], 40: 41 against 18; [4, 4], 256: 10.2
     // against 12.8; [50], 4096: 14 against 39).
-    if ((size_t)Dt * t->d <= 32768 &&
+    if (!large_b &&
         (n_theta >= 1024 || (n_theta >= 32 && tiles <= 64) || (size_t)tiles * Dt <= 8192)) {
         int nw = RBLOCK / 64;
         while (nw > 4 && (long long)n_theta * nw > 8192) nw >>= 1;
