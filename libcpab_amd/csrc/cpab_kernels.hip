@@ -11,6 +11,7 @@
 //   k_transform_data_bwd  adjoint of k_transform_data (+ dL/ddata scatter)
 //   k_interp_fwd / k_interp_bwd   linear interpolation of data at a grid
 //   k_reduce_theta      per-theta sum of the tile partials, then B^T (many thetas)
+//   k_reduce_many       the same for thousands of thetas with few rows each
 //   k_reduce_cols       column slices of that sum (few thetas), then
 //   k_reduce_bt         B^T per theta (all in a fixed order: deterministic)
 #include <hip/hip_runtime.h>
