@@ -84,12 +84,14 @@ size_t cpab_data_workspace_bytes(const cpab_tess_t* t, int n_theta, const int* o
 /* Floats in the forward's saved state for the fused backward:
  * n_theta * (ndim + ndim^2 + (ndim > 1 ? 3 : 0)) * nP -- warped points,
  * Jacobians and, in 2D/3D, the durations and crossed facets of each point's
- * first two chunks, which the backward replays without searching again. */
+ * first two chunks, which the backward replays without searching again.  From
+ * 2^29 points per theta on (2D, 3D) the calls keep no state and the answer is 0:
+ * saved is not touched and the backward integrates the points again. */
 size_t cpab_saved_floats(int ndim, int n_theta, int nP);
 
 /* Floats in cpab_transform_fwd's saved state (jac) for cpab_transform_bwd:
  * n_theta * (ndim^2 + (ndim > 1 ? 3 : 0)) * nP -- the q-space Jacobians and,
- * in 2D/3D, each point's chunk log. */
+ * in 2D/3D, each point's chunk log; 0 from 2^29 points per theta on, as above. */
 size_t cpab_jac_floats(int ndim, int n_theta, int nP);
 
 /* A_q = B theta per cell, in q-space.  Replaces the basis expansion of
@@ -235,7 +237,7 @@ typedef struct cpab_instance {
     const float* data;   /* [C, dsize...] */
     const float* lin;    /* outsize[0] + outsize[1] + outsize[2] meshgrid axis coordinates */
     float* out;          /* [C, outsize...] */
-    float* saved;        /* cpab_saved_floats(ndim, 1, nP) floats or NULL */
+    float* saved;        /* cpab_saved_floats(ndim, 1, nP) floats or NULL (kept by all instances or none) */
     const float* grad_out;
     float* grad_data;    /* NULL or zero-filled [C, dsize...] */
     float* grad_theta;   /* [d] */

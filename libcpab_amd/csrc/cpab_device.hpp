@@ -493,7 +493,9 @@ CPAB_HD __forceinline__ void log_chunk(ChunkLog& lg, float h, int facet) {
 // Sink for the forward's chunk log: durations go straight to memory (h[k] of
 // point i at base[k * stride + i], base common to the wave) as the chunks end;
 // only the facet code stays in a register.  On the device the store is a raw
-// buffer store with a 32-bit lane offset, bounded by the log rows.
+// buffer store with a 32-bit lane offset, bounded by the log rows, so a point's
+// log has to end below 4 GiB: up to LOG_POINTS points an instance.
+constexpr int LOG_POINTS = (int)((1LL << 32) / (NREC * 4)) - 1;
 struct LogSink {
     float* base;
     int stride;
@@ -508,7 +510,7 @@ struct LogSink {
         i = idx;
         code = 0;
 #if defined(__HIP_DEVICE_COMPILE__)
-        rsrc = __builtin_amdgcn_make_buffer_rsrc(b, 0, NREC * s * 4, 0x00020000);
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(b, 0, NREC * 4u * (unsigned)s, 0x00020000);
 #endif
     }
 };
@@ -518,7 +520,8 @@ CPAB_HD __forceinline__ void sink_chunk(LogSink& lg, int n, float h, int facet) 
     if (n < NREC) {
 #if defined(__HIP_DEVICE_COMPILE__)
         // the builtin's data operand is an integer: pass the bits, not the value
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h), lg.rsrc, (n * lg.stride + lg.i) * 4, 0, 0);
+        const unsigned at = ((unsigned)n * (unsigned)lg.stride + (unsigned)lg.i) * 4u;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h), lg.rsrc, at, 0, 0);
 #else
         lg.base[(size_t)n * lg.stride + lg.i] = h;
 #endif

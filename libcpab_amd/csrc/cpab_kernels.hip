@@ -638,8 +638,7 @@ __device__ __forceinline__ float blend(const float (&v)[1 << D], const float (&f
 // value of channel data dp at the corners (i0, i1, fd)
 // base[i], base uniform over the wave.  NARROW: as a scalar base and a 32-bit byte
 // offset (a 64-bit address is two more instructions per access), for an instance's
-// points in 2D and 3D calls with saved state, whose chunk log's 32-bit row bounds
-// keep them below 2^29.
+// points in 2D and 3D calls with saved state, of which there are at most LOG_POINTS.
 template <bool NARROW>
 __device__ __forceinline__ float at(const float* base, int i) {
     if constexpr (!NARROW) return base[i];
@@ -3021,6 +3020,11 @@ static size_t aq_bytes(const cpab_tess_t* t, int n_theta) {
     return (size_t)n_theta * t->nC * t->ndim * (t->ndim + 1) * sizeof(float);
 }
 
+// Saved state reaches LOG_POINTS points an instance in 2D and 3D (the chunk log and
+// the rows beside it are addressed by 32-bit byte offsets); beyond, the calls keep
+// none and the backward integrates the points again.
+static bool keeps_state(int ndim, int nP) { return ndim == 1 || nP <= LOG_POINTS; }
+
 static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const float* points, int nP,
                     int per_theta_grid, const int* grid_shape, float t_end, float* out, float* jac,
                     void* workspace, size_t ws_bytes, AqIn where, hipStream_t stream) {
@@ -3031,6 +3035,7 @@ static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     if (!theta || !points || !out) return CPAB_ERR_ARG;
     const size_t need = where == AqIn::Buffer ? aq_bytes(t, n_theta) : cpab_workspace_bytes(t, n_theta, nP);
     if (ws_bytes < need || !workspace) return CPAB_ERR_WORKSPACE;
+    if (!keeps_state(t->ndim, nP)) jac = nullptr;
     const size_t lds = lds_tables(t->ndim, t->nC + t->nV);
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     float* Aq = static_cast<float*>(workspace);
@@ -3114,6 +3119,7 @@ static int grid_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     // no points: grad_theta is written with zeros; points and grad_out may be NULL
     if ((!theta && !kept) || !grad_theta || (nP > 0 && (!points || !grad_out))) return CPAB_ERR_ARG;
     if (ws_bytes < cpab_workspace_bytes(t, n_theta, nP) || !workspace) return CPAB_ERR_WORKSPACE;
+    if (!keeps_state(t->ndim, nP)) jac = nullptr;
     const size_t lds = lds_bwd(t->ndim, t->nC, t->nC + t->nV);
     if (lds > LDS_LIMIT) return CPAB_ERR_LDS;
     const int Dt = t->nC * t->ndim * (t->ndim + 1);
@@ -3224,9 +3230,13 @@ int cpab_interpolate_bwd(int ndim, const float* data, int N, int C, const int* d
     return status_from_hip();
 }
 
-size_t cpab_saved_floats(int ndim, int n_theta, int nP) { return (size_t)n_theta * saved_rows(ndim) * nP; }
+size_t cpab_saved_floats(int ndim, int n_theta, int nP) {
+    return keeps_state(ndim, nP) ? (size_t)n_theta * saved_rows(ndim) * nP : 0;
+}
 
-size_t cpab_jac_floats(int ndim, int n_theta, int nP) { return (size_t)n_theta * jac_rows(ndim) * nP; }
+size_t cpab_jac_floats(int ndim, int n_theta, int nP) {
+    return keeps_state(ndim, nP) ? (size_t)n_theta * jac_rows(ndim) * nP : 0;
+}
 
 size_t cpab_data_workspace_bytes(const cpab_tess_t* t, int n_theta, const int* outsize) {
     if (check_tess(t) != CPAB_OK || n_theta < 0 || !outsize) return 0;
@@ -3251,6 +3261,7 @@ static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     if ((rc = src_out(t->ndim, outsize, s, nP))) return rc;
     if (!theta || !lin || !out || n_theta < 0) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
+    if (!keeps_state(t->ndim, nP)) saved = nullptr;
     float* Aq;
     if (where == AqIn::Scratch) {
         if (aq_bytes(t, n_theta) > (size_t)CPAB_NOALLOC_SCRATCH_BYTES) return CPAB_ERR_SCRATCH;
@@ -3321,6 +3332,7 @@ static int data_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     if ((rc = src_out(t->ndim, outsize, s, nP))) return rc;
     if ((!theta && !kept) || !lin || !grad_out || !grad_theta || n_theta < 0) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
+    if (!keeps_state(t->ndim, nP)) saved = nullptr;
     if (ws_bytes < cpab_data_workspace_bytes(t, n_theta, outsize) || !workspace) return CPAB_ERR_WORKSPACE;
     Launch L;
     L.n_theta = n_theta;
@@ -3554,7 +3566,8 @@ int cpab_batch_fwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
     int rc = batch_check(host_inst, n_inst, ppt, lds_tab, lds_acc, maxd, maxDt, false);
     if (rc) return rc;
     bool save = true;
-    for (int i = 0; i < n_inst; ++i) save = save && host_inst[i].saved != nullptr;
+    for (int i = 0; i < n_inst; ++i)
+        save = save && host_inst[i].saved != nullptr && keeps_state(host_inst[i].tess.ndim, host_inst[i].nP);
     hipLaunchKernelGGL(k_batch_A, dim3((maxDt + A_ROWS - 1) / A_ROWS, n_inst), dim3(BLOCK), 0, stream, dev_inst);
     hipLaunchKernelGGL(k_counter_reset, dim3(1), dim3(64), 0, stream, counter);
     int maxnd = 1;
@@ -3582,7 +3595,8 @@ int cpab_batch_bwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
     int rc = batch_check(host_inst, n_inst, ppt, lds_tab, lds_acc, maxd, maxDt, true);
     if (rc) return rc;
     bool have = true;
-    for (int i = 0; i < n_inst; ++i) have = have && host_inst[i].saved != nullptr;
+    for (int i = 0; i < n_inst; ++i)
+        have = have && host_inst[i].saved != nullptr && keeps_state(host_inst[i].tess.ndim, host_inst[i].nP);
     // with the forward's saved state, its A_q is still in every instance's
     // workspace (the backward only writes the partials after it)
     if (!have)
