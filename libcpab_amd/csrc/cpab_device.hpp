@@ -883,11 +883,11 @@ CPAB_HD __forceinline__ void advance1(PointState<1>& st, const CellTable<1>& tab
     st.iters++;
 }
 
-// The saltation factor v_next / v_prev of a crossing (1 for a continuous field;
-// formed as 1 + difference, which keeps it exact there), or its inverse for the
-// adjoint; 1 where the divisor vanishes beside the other.
+// The saltation factor v_next / v_prev of a crossing (1 for a continuous field), or
+// its inverse for the adjoint; 1 where the divisor vanishes beside the other.  A
+// quotient: the reciprocal of a subnormal velocity (theta near zero) overflows.
 CPAB_HD __forceinline__ float saltation1(float vnum, float vden) {
-    return fabsf(vden) > 1e-6f * fabsf(vnum) && vden != 0.f ? fmaf(vnum - vden, near_rcp(vden), 1.f) : 1.f;
+    return fabsf(vden) > 1e-6f * fabsf(vnum) && vden != 0.f ? vnum / vden : 1.f;
 }
 
 // ---------------------------------------------------------------------------
