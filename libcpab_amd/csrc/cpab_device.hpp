@@ -731,23 +731,14 @@ CPAB_HD __forceinline__ void replay(PointState<D>& st, const CellTable<D>& tab, 
 // Instruction bound like the others: 2.7 chunks per wave and point on 1024-point
 // signals over 50 cells, most of it the library's expm1, log1p and exp and IEEE
 // quotients.  The growth of a chunk that ends on a cell edge is the velocity
-// ratio 1 + r, and the final chunk's comes with its phi1.  The gradient's pass
-// (EXACT = false) takes phi1, phi2 and e^z from one Taylor sum for |z| <= 1
-// (nearly every chunk) and log1p(r)/r as the hardware logarithm of u = 1 + r over
-// u - 1 (the rounding of u enters both, so it cancels; measured error 2.8e-7 at
-// most over |r| = 1e-5 .. 1e3 and r > -1, 6e-8 on average).  The positions
-// themselves (EXACT) keep the library's functions operation for operation: one
-// rounding of q is a thousandth of a sample on a signal of 8192, and an
-// interpolation weight's whole error.  us per launch, 4096 signals of 1024
-// points, before / after: forward 75 / 66, backward 116 / 68.
+// ratio 1 + r.  The gradient's pass takes phi1 and phi2 from one Taylor sum for
+// |z| <= 1 (nearly every chunk; at most 9.1e-8 off, the library's quotients 1.2e-7
+// and 3.9e-7).  Hit times and positions are the forward's, bit for bit, in every
+// pass, and the exponentials the library's: e^z from the Taylor sum would be 1.9e-7
+// off at z = -1, a hit time by the hardware's logarithm and reciprocal 2.8e-7.
 // ---------------------------------------------------------------------------
-// 1/x to ~0.5 ulp
-CPAB_HD __forceinline__ float near_rcp(float x) {
-    const float r = fast_rcp(x);
-    return fmaf(fmaf(-x, r, 1.f), r, r);
-}
-// e^z, p1 = (e^z - 1)/z, p2 = (e^z - 1 - z)/z^2
-CPAB_HD __forceinline__ void exp_phis(float z, float& e, float& p1, float& p2) {
+// p1 = (e^z - 1)/z, p2 = (e^z - 1 - z)/z^2
+CPAB_HD __forceinline__ void phis(float z, float& p1, float& p2) {
     if (fabsf(z) <= 1.f) {
         // sum_k z^k/(k+2)!, k < 10: the next term is below 1/12! = 2.1e-9
         constexpr float C[10] = {1.f / 2,    1.f / 6,     1.f / 24,     1.f / 120,     1.f / 720,
@@ -757,23 +748,11 @@ CPAB_HD __forceinline__ void exp_phis(float z, float& e, float& p1, float& p2) {
         for (int k = 8; k >= 0; --k) acc = fmaf(acc, z, C[k]);
         p2 = acc;
         p1 = fmaf(z, acc, 1.f);
-        e = fmaf(z, p1, 1.f);
     } else {
         const float em = expm1f(z);
-        e = expf(z);
         p1 = em / z;
         p2 = (em - z) / (z * z);
     }
-}
-// log1p(r)/r for r > -1
-CPAB_HD __forceinline__ float log1p_over_fast(float r) {
-    const float u = 1.f + r, d = u - 1.f;
-#if defined(__HIP_DEVICE_COMPILE__)
-    const float l = __builtin_amdgcn_logf(u);
-#else
-    const float l = log2f(u);
-#endif
-    return d == 0.f ? fmaf(r, -0.5f, 1.f) : l * 0.69314718055994531f * fast_rcp(d);
 }
 CPAB_HD __forceinline__ float phi1(float z) {  // (e^z - 1)/z
     return (fabsf(z) < 1e-4f) ? fmaf(z, fmaf(z, 1.0f / 6.0f, 0.5f), 1.0f) : expm1f(z) / z;
@@ -789,7 +768,6 @@ struct Hit1 {
     int next;
     bool right, crosses;
 };
-template <bool EXACT>
 CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& tab, int nx) {
     Hit1 h;
     const int c = st.c;
@@ -804,7 +782,7 @@ CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& t
     h.r = 0.f;
     h.crosses = false;
     if (h.v0 != 0.f && h.next >= 0 && h.next < nx) {
-        if (EXACT && tab.hits && q0 == (h.right ? (float)c : (float)(c + 1))) {
+        if (tab.hits && q0 == (h.right ? (float)c : (float)(c + 1))) {
             // from edge to edge: the same for every point
             const float2 f = tab.hits[2 * c + (h.right ? 1 : 0)];
             h.th = f.x;
@@ -814,10 +792,9 @@ CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& t
             return h;
         }
         const float dq = h.qb - q0;
-        const float dt = EXACT ? dq / h.v0 : dq * near_rcp(h.v0);
-        h.r = EXACT ? h.a * dq / h.v0 : h.a * dt;
+        h.r = h.a * dq / h.v0;
         if (1.0f + h.r > 0.f) {
-            h.th = fmaxf(dt * (EXACT ? log1p_over(h.r) : log1p_over_fast(h.r)), 0.f);
+            h.th = fmaxf(dq / h.v0 * log1p_over(h.r), 0.f);
             const bool back = (st.zero_hops > 0 && h.next == st.came_from && h.th <= ZERO_HOP);
             h.crosses = h.th < st.T && !back;
         }
@@ -835,7 +812,7 @@ CPAB_HD __forceinline__ float2 whole_cell(const CellTable<1>& tab, int c, int di
     st.came_from = -1;
     st.zero_hops = 0;
     st.iters = 0;
-    const Hit1 h = hit1<true>(st, tab, nx);
+    const Hit1 h = hit1(st, tab, nx);
     float2 f;
     f.x = h.crosses && h.right == (dir == 1) ? h.th : INFINITY;
     f.y = h.r;
@@ -849,19 +826,11 @@ CPAB_HD __forceinline__ void hop1(PointState<1>& st, const Hit1& h) {
     st.q[0] = h.qb;
 }
 // The last chunk: the time left, inside the cell; returns e^(a T).
-template <bool EXACT>
 CPAB_HD __forceinline__ float end1(PointState<1>& st, const Hit1& h) {
     const float z = h.a * st.T;
-    float grow, p1, p2;
-    if (EXACT) {
-        p1 = phi1(z);
-        grow = z > -1.f ? fmaf(z, p1, 1.f) : expf(z);  // 1 + (e^z - 1) cancels below
-    } else {
-        exp_phis(z, grow, p1, p2);
-    }
-    st.q[0] = fmaf(st.T * p1, h.v0, st.q[0]);
+    st.q[0] = fmaf(st.T * phi1(z), h.v0, st.q[0]);
     st.T = 0.f;
-    return grow;
+    return expf(z);
 }
 
 struct Chunk1 {
@@ -869,16 +838,15 @@ struct Chunk1 {
     int cell, facet, next;
     float q1;
 };
-template <bool EXACT>
 CPAB_HD __forceinline__ void advance1(PointState<1>& st, const CellTable<1>& tab, int nx, Chunk1& ch) {
-    const Hit1 h = hit1<EXACT>(st, tab, nx);
+    const Hit1 h = hit1(st, tab, nx);
     ch.a = h.a; ch.b = h.b; ch.q0 = st.q[0];
     ch.cell = st.c;
     ch.h = h.crosses ? h.th : st.T;
     ch.facet = h.crosses ? (h.right ? 1 : 0) : -1;
     ch.next = h.crosses ? h.next : st.c;
     if (h.crosses) hop1(st, h);
-    else end1<EXACT>(st, h);
+    else end1(st, h);
     ch.q1 = st.q[0];
     st.iters++;
 }
@@ -1146,7 +1114,7 @@ CPAB_HD __forceinline__ void integrate(float (&q)[D], int c0, float T, const Cel
         Hit1 h;
         bool last = false;
         while (st.T > 0.f) {
-            h = hit1<true>(st, tab, nx);
+            h = hit1(st, tab, nx);
             last = !h.crosses;
             if (last) break;
             hop1(st, h);
@@ -1159,7 +1127,7 @@ CPAB_HD __forceinline__ void integrate(float (&q)[D], int c0, float T, const Cel
             if (st.iters >= MAX_ITERS && st.T > 0.f) give_up<D, WITHJ>(st, J, unfinished);
         }
         if (last) {
-            const float grow = end1<true>(st, h);
+            const float grow = end1(st, h);
             if constexpr (WITHJ) J[0][0] *= grow;
         }
     } else {
@@ -1293,11 +1261,12 @@ CPAB_HD __forceinline__ void chunk_grad(const Chunk<D>& ch, float (&mu)[D], floa
 }
 
 CPAB_HD __forceinline__ void chunk_grad1(const Chunk1& ch, float& mu, float (&G)[2]) {
-    float e, p1, p2;
-    exp_phis(-ch.a * ch.h, e, p1, p2);
+    const float z = -ch.a * ch.h;
+    float p1, p2;
+    phis(z, p1, p2);
     G[0] = mu * fmaf(ch.h * ch.h, ch.b * p2, ch.q0 * ch.h);
     G[1] = mu * ch.h * p1;
-    mu *= e;
+    mu *= expf(z);
 }
 
 // ---------------------------------------------------------------------------

@@ -506,7 +506,7 @@ __device__ __forceinline__ void pass2(Pass2<D>& w, const CellTable<D>& tab, cons
         if (active) {
             if constexpr (D == 1) {
                 Chunk1 ch;
-                advance1<false>(st, tab, g.nc0, ch);
+                advance1(st, tab, g.nc0, ch);
                 float G1[2];
                 chunk_grad1(ch, w.mu[0], G1);
                 G[0] = G1[0];
@@ -1088,7 +1088,7 @@ __global__ __launch_bounds__(BLOCK) void k_transform_cells(Launch L, Geo g, Src 
             float h;
             if constexpr (D == 1) {
                 Chunk1 ch;
-                advance1<true>(st, tab, g.nc0, ch);
+                advance1(st, tab, g.nc0, ch);
                 cell = ch.cell;
                 facet = ch.facet;
                 h = ch.h;
@@ -2701,12 +2701,12 @@ Geo make_geo(const cpab_tess_t* t) {
     return g;
 }
 
-// 1D forwards make the table of whole-cell crossings where a thread's share of it
+// 1D transforms make the table of whole-cell crossings where a thread's share of it
 // (one crossing per 64 cells) is at most one for each of its points, of which it has
 // several: a wave on signals of 1024 points over 50 cells runs 2.65 chunks a point, and
-// all but the first start on an edge.  us, before / after: 4096 of those 64.8 / 49.0,
-// 500 of 8000 points over 80 cells 61.6 / 50.2.  (The gradient's pass, whose
-// crossings are cheaper, lost by it: 65.2 -> 67.9.)
+// all but the first start on an edge.  us, without / with: 4096 of those, forward
+// 64.8 / 49.0, backward 101.6 / 86.2; 500 of 8000 points over 80 cells 61.6 / 50.2 and
+// 84.1 / 73.6.
 int use_hits(const cpab_tess_t* t, int ppt) {
     return t->ndim == 1 && t->nC <= HIT_CELLS && ppt > 1 && t->nC <= 64 * ppt;
 }
@@ -3133,6 +3133,7 @@ static int grid_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     grid_launch(t, n_theta, nP, grid_shape, (ws_bytes - head) / ((size_t)n_theta * Dt * 4), L, s);
     L.t_end = t_end;
     Geo g = make_geo(t);
+    g.hits = use_hits(t, L.ppt);
     s.pts = points;
     s.per_theta = per_theta_grid;
     dim3 grid(L.tiles * n_theta);
@@ -3359,6 +3360,7 @@ static int data_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     L.tiles = tile_count(t->ndim, nP, s.g0, s.g1, L.ppt, s.g2);
     L.t_end = t_end;
     Geo g = make_geo(t);
+    g.hits = use_hits(t, L.ppt);
     const int tpb = bwd_tiles_per_block(t->ndim, L.ty, n_theta, L.tiles);
     const int nbt = bwd_blocks_per_theta(L.tiles, s.g1, L.ty, tpb);
     dim3 grid(nbt * n_theta);
