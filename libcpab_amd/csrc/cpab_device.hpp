@@ -736,6 +736,8 @@ CPAB_HD __forceinline__ void replay(PointState<D>& st, const CellTable<D>& tab, 
 // and 3.9e-7).  Hit times and positions are the forward's, bit for bit, in every
 // pass, and the exponentials the library's: e^z from the Taylor sum would be 1.9e-7
 // off at z = -1, a hit time by the hardware's logarithm and reciprocal 2.8e-7.
+// us per launch, 4096 signals of 1024 points, before / after, with the table of
+// whole-cell crossings: forward 74 / 50, backward 115 / 86.
 // ---------------------------------------------------------------------------
 // p1 = (e^z - 1)/z, p2 = (e^z - 1 - z)/z^2
 CPAB_HD __forceinline__ void phis(float z, float& p1, float& p2) {
@@ -793,7 +795,7 @@ CPAB_HD __forceinline__ Hit1 hit1(const PointState<1>& st, const CellTable<1>& t
         }
         const float dq = h.qb - q0;
         h.r = h.a * dq / h.v0;
-        if (1.0f + h.r > 0.f) {
+        if (1.0f + h.r > 0.f && h.r < INFINITY) {  // infinite: beside a fixed point, for longer than any T
             h.th = fmaxf(dq / h.v0 * log1p_over(h.r), 0.f);
             const bool back = (st.zero_hops > 0 && h.next == st.came_from && h.th <= ZERO_HOP);
             h.crosses = h.th < st.T && !back;

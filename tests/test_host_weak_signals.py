@@ -1,11 +1,13 @@
 """1D fields of subnormal velocities, compiled for the host: points on the edges
 cross into the next cell in no time, and the Jacobian of a nearly vanishing field
 is 1."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from libcpab_amd.core.tessellation import make_tessellation
-from test_host_integrator import host_transform
+from test_host_integrator import _lib, _ptr, host_transform
 
 
 @pytest.mark.parametrize("nc", [[7], [50]])
@@ -22,3 +24,20 @@ def test_jacobian_of_vanishing_fields(nc, scale):
     assert np.isfinite(jac).all()
     if scale >= 1e-37:
         assert np.abs(jac - 1).max() <= 1e-2
+
+
+@pytest.mark.parametrize("x0", [1e-45, 1e-42, 1e-39, 1e-37])
+@pytest.mark.parametrize("slope", [0.9, 3.0, -1.5])
+def test_points_beside_a_fixed_point_stay_there(x0, slope):
+    """dq / v0 beyond the range of FP32: the edge is not reached."""
+    nc = np.array([2, 1, 1], np.int32)
+    A = np.array([slope, 0, -slope, 2 * slope], np.float32)  # a hat: 0 at both ends
+    x, out, jac = np.array([x0], np.float32), np.zeros(1, np.float32), np.zeros(1, np.float32)
+    none = np.zeros(32, np.float32)
+    _lib().host_transform(1, _ptr(nc), 2, _ptr(A), _ptr(none), _ptr(none), _ptr(x), 1, 1, 0, ctypes.c_float(1),
+                          ctypes.c_float(4e-6), _ptr(out), _ptr(jac))
+    growth = float(np.exp(np.float64(A[0])))
+    assert abs(jac[0] / growth - 1) <= 2.0 ** -22
+    # the start in cells, the velocity and the end are rounded to the smallest number's
+    # multiples
+    assert abs(float(out[0]) - float(x[0]) * growth) <= 2.0 ** -22 * x0 * growth + 4 * 2.0 ** -149 * (1 + growth)
