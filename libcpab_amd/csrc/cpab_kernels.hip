@@ -206,7 +206,7 @@ __device__ __forceinline__ int nc_at(const Geo& g, int a) {
 }
 
 // LDS layout of one theta's tables: A_q [nC*P], then in 1D the whole-cell crossings
-// [nC*2] float2 (up to HIT_CELLS cells), in 2D and 3D 1/|M|_F [nC (padded to 4)],
+// [nC*2] float2 (where Geo::hits asks for them), in 2D and 3D 1/|M|_F [nC (padded to 4)],
 // facet planes [nC*NF] float4, neighbours [nC*NF] int
 template <int D>
 __device__ __forceinline__ CellTable<D> table_view(float* smem, int nC) {
@@ -325,12 +325,16 @@ __host__ __device__ constexpr int saved_rows(int D) { return D + D * D + (D > 1 
 // and, in 2D/3D, the chunk log.
 __host__ __device__ constexpr int jac_rows(int D) { return D * D + (D > 1 ? NREC + 1 : 0); }
 
-// Cells up to which the 1D tables have room for the whole-cell crossings.
-constexpr int HIT_CELLS = 512;
+// Words of the tables, and of the whole-cell crossings after them.
 template <int D>
 __host__ __device__ constexpr size_t table_floats(int nC) {
-    if (D == 1) return (size_t)nC * (nC <= HIT_CELLS ? 6 : 2);
+    if (D == 1) return (size_t)nC * 2;
     return (size_t)nC * D * (D + 1) + ((nC + 3) & ~3) + (size_t)nC * NF * 4 + (size_t)nC * NF;
+}
+
+template <int D>
+__device__ __forceinline__ int hit_floats(const Geo& g) {
+    return D == 1 && g.hits ? 4 * g.nC : 0;
 }
 
 // Start cell of a point: the lookup, except that a 3D point outside the
@@ -1214,7 +1218,7 @@ __global__ __launch_bounds__(BLOCK, D == 2 ? 6 : 1) void k_transform_bwd(Launch 
     const int th = lb / L.tiles, tile = lb % L.tiles;
     if (th >= L.n_theta) return;
     const int nC = g.nC;
-    float* acc = smem + table_floats<D>(nC + g.nV);
+    float* acc = smem + table_floats<D>(nC + g.nV) + hit_floats<D>(g);
     for (int i = threadIdx.x; i < WAVES * nC * P; i += BLOCK) acc[i] = 0.f;
     const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * nC * P, g);
     float* wacc = acc + (threadIdx.x >> 6) * nC * P;
@@ -1561,7 +1565,7 @@ __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_
     if (th >= L.n_theta) return;
     const int tiles_y = tpb > 1 ? (s.g1 + L.ty - 1) / L.ty : 1, tiles_x = L.tiles / tiles_y;
     const int nC = g.nC;
-    float* acc = smem + table_floats<D>(nC + g.nV);
+    float* acc = smem + table_floats<D>(nC + g.nV) + hit_floats<D>(g);
     for (int i = threadIdx.x; i < WAVES * nC * P; i += BLOCK) acc[i] = 0.f;
     const CellTable<D> tab = stage_tables<D>(smem, Aq + (size_t)th * nC * P, g);
     const size_t dstride = (size_t)im.s0 * (D > 1 ? im.s1 : 1) * (D > 2 ? im.s2 : 1);
@@ -2706,10 +2710,13 @@ Geo make_geo(const cpab_tess_t* t) {
 // several: a wave on signals of 1024 points over 50 cells runs 2.65 chunks a point, and
 // all but the first start on an edge.  us, without / with: 4096 of those, forward
 // 64.8 / 49.0, backward 101.6 / 86.2; 500 of 8000 points over 80 cells 61.6 / 50.2 and
-// 84.1 / 73.6.
+// 84.1 / 73.6.  Backward over 10, 120, 256 and 500 cells: 62 / 57, 69 / 58, 205 / 153,
+// 320 / 266 (the last with a block less per CU).
+constexpr int HIT_CELLS = 512;  // 8 KB of LDS
 int use_hits(const cpab_tess_t* t, int ppt) {
     return t->ndim == 1 && t->nC <= HIT_CELLS && ppt > 1 && t->nC <= 64 * ppt;
 }
+size_t hit_bytes(const Geo& g) { return g.hits ? (size_t)g.nC * 16 : 0; }
 
 // points per thread: the largest of 8, 4, 2, 1 that still gives >= 16 blocks
 // per CU: with a few rounds of blocks per CU the last round drains the chip
@@ -3052,9 +3059,9 @@ static int grid_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     if ((rc = expand_or_launch(t, theta, n_theta, (long long)L.tiles * n_theta, Aq, stream, ex))) return rc;
 #define LAUNCH_TF(DD)                                                                                                \
     if (jac)                                                                                                          \
-        hipLaunchKernelGGL((k_transform<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, ex, Aq, out, jac);           \
+        hipLaunchKernelGGL((k_transform<DD, true>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, ex, Aq, out, jac);           \
     else                                                                                                              \
-        hipLaunchKernelGGL((k_transform<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, ex, Aq, out, jac);
+        hipLaunchKernelGGL((k_transform<DD, false>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, ex, Aq, out, jac);
     CPAB_DISPATCH_D(t->ndim, LAUNCH_TF)
 #undef LAUNCH_TF
     return status_from_hip();
@@ -3139,10 +3146,10 @@ static int grid_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     dim3 grid(L.tiles * n_theta);
 #define LAUNCH_TB(DD)                                                                                                   \
     if (jac)                                                                                                             \
-        hipLaunchKernelGGL((k_transform_bwd<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, Aq, grad_out, jac, part, \
+        hipLaunchKernelGGL((k_transform_bwd<DD, true>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, Aq, grad_out, jac, part, \
                            grad_points);                                                                                 \
     else                                                                                                                 \
-        hipLaunchKernelGGL((k_transform_bwd<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, Aq, grad_out, jac,     \
+        hipLaunchKernelGGL((k_transform_bwd<DD, false>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, Aq, grad_out, jac,     \
                            part, grad_points);
     CPAB_DISPATCH_D(t->ndim, LAUNCH_TB)
 #undef LAUNCH_TB
@@ -3290,9 +3297,9 @@ static int data_fwd(const cpab_tess_t* t, const float* theta, int n_theta, const
     if ((rc = expand_or_launch(t, theta, n_theta, (long long)L.tiles * n_theta, Aq, stream, ex))) return rc;
 #define LAUNCH_DF(DD)                                                                                                    \
     if (saved)                                                                                                            \
-        hipLaunchKernelGGL((k_transform_data<DD, true>), grid, dim3(BLOCK), lds, stream, L, g, s, im, ex, Aq, out, saved);    \
+        hipLaunchKernelGGL((k_transform_data<DD, true>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, im, ex, Aq, out, saved);    \
     else                                                                                                                  \
-        hipLaunchKernelGGL((k_transform_data<DD, false>), grid, dim3(BLOCK), lds, stream, L, g, s, im, ex, Aq, out, saved);
+        hipLaunchKernelGGL((k_transform_data<DD, false>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, im, ex, Aq, out, saved);
     CPAB_DISPATCH_D(t->ndim, LAUNCH_DF)
 #undef LAUNCH_DF
     return status_from_hip();
@@ -3369,7 +3376,7 @@ static int data_bwd(const cpab_tess_t* t, const float* theta, const float* kept,
     // would only cost ([3, 3, 3], 16 x 64^3: 235 -> 257 us)
     const bool merge = grad_data && !box_cap;
 #define LAUNCH_DB3(DD, HAVES, MERGE)                                                                                  \
-    hipLaunchKernelGGL((k_transform_data_bwd<DD, HAVES, MERGE>), grid, dim3(BLOCK), lds, stream, L, g, s, im, Aq,     \
+    hipLaunchKernelGGL((k_transform_data_bwd<DD, HAVES, MERGE>), grid, dim3(BLOCK), lds + hit_bytes(g), stream, L, g, s, im, Aq,     \
                        grad_out, saved, part, box_cap, tpb, defer)
 #define LAUNCH_DB(DD)                                                                \
     if (saved) {                                                                     \
