@@ -3721,7 +3721,8 @@ int cpab_ref_expand(const cpab_tess_t* t, const float* theta, int n_theta, int n
                     hipStream_t stream) {
     int rc = check_tess(t);
     if (rc) return rc;
-    if (!theta || !As || !trels || !t->B || n_theta < 0 || nstepsolver < 1) return CPAB_ERR_ARG;
+    // a basis without columns (one 1D cell, zero boundary): arrays with no elements may be NULL
+    if ((t->d > 0 && (!theta || !t->B)) || !As || !trels || n_theta < 0 || nstepsolver < 1) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
     const dim3 g((unsigned)(t->nC + EXPAND_CELLS - 1) / EXPAND_CELLS * n_theta);
     const double scale = 1.0 / nstepsolver;
