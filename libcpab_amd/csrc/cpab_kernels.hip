@@ -2436,9 +2436,10 @@ __global__ __launch_bounds__(64) void k_ref_grad_theta(const float* __restrict__
     const int nc[3] = {nc0, nc1, nc2};
     const float margin = cpab_ref::lookup_margin<D>(nc);
     const double h = 1.0 / nstep, h2 = 0.5 * h * h;
-    for (int i0 = blockIdx.x * 64; i0 < nP; i0 += gridDim.x * 64) {
-        const int i = i0 + lane;
-        const bool valid = i < nP;
+    // unsigned: the last step past nP may go beyond 2^31
+    for (unsigned i0 = blockIdx.x * 64; i0 < (unsigned)nP; i0 += gridDim.x * 64) {
+        const unsigned i = i0 + lane;
+        const bool valid = i < (unsigned)nP;
         float p[D];
         double lam[D], G[P];
 #pragma unroll
@@ -3780,7 +3781,7 @@ static int ref_grad_launch(int ndim, int nC, int n_theta, int nP, int nstep, int
     const int nseg = (nstep + S - 1) / S;
     lds = ((size_t)2 * nC * ndim * (ndim + 1) + (size_t)64 * ((size_t)(nseg + S) * ndim + S)) * 4;
     if (lds > LDS_LIMIT || n_theta > 65535) return 0;
-    const int chunks = (nP + 63) / 64;
+    const int chunks = (int)(((long long)nP + 63) / 64);
     const int want = n_theta < 4096 ? 4096 / n_theta : 1;
     return chunks < want ? chunks : want;
 }
