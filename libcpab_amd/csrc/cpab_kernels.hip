@@ -2183,9 +2183,8 @@ __global__ __launch_bounds__(RBLOCK) void k_batch_bt(const cpab_instance_t* __re
 // ---------------------------------------------------------------------------
 // method='numeric': the reference's fixed-step scheme
 // ---------------------------------------------------------------------------
-// expm(scale * A~) for n affine matrices A [D, D+1] (homogeneous last row 0),
-// FP64 scaling and squaring with a degree-12 Taylor polynomial; top D rows out.
-// T = the first D rows of expm(scale [A; 0]) in FP64; a, t: [D, D + 1]
+// t = the first D rows of expm(scale [a; 0]) (a, t: [D, D + 1]): FP64 scaling and
+// squaring with a degree-12 Taylor polynomial
 template <int D>
 __device__ __forceinline__ void expm_affine(const float* a, double scale, float* t) {
     constexpr int E = D + 1;
@@ -2251,8 +2250,9 @@ __device__ __forceinline__ void expm_affine(const float* a, double scale, float*
         for (int c = 0; c < E; ++c) t[r * E + c] = (float)R[r][c];
 }
 
+// expm(scale * A~) for n affine matrices A [D, D+1] (homogeneous last row 0), a thread each
 template <int D>
-__global__ __launch_bounds__(BLOCK) void k_expm_affine(const float* __restrict__ A, int n, float scale,
+__global__ __launch_bounds__(BLOCK) void k_expm_affine(const float* __restrict__ A, int n, double scale,
                                                        float* __restrict__ T) {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
@@ -3707,15 +3707,34 @@ int cpab_fill_zero(float* p, size_t n, hipStream_t stream) {
     return status_from_hip();
 }
 
-int cpab_expm_affine(const float* A, int n, int ndim, float scale, float* T, hipStream_t stream) {
-    if (ndim < 1 || ndim > 3) return CPAB_ERR_NDIM;
-    if (!A || !T || n < 0) return CPAB_ERR_ARG;
-    if (n == 0) return CPAB_OK;
+static int launch_expm(const float* A, int n, int ndim, double scale, float* T, hipStream_t stream) {
     dim3 g((n + BLOCK - 1) / BLOCK);
 #define LAUNCH_EX(DD) hipLaunchKernelGGL((k_expm_affine<DD>), g, dim3(BLOCK), 0, stream, A, n, scale, T);
     CPAB_DISPATCH_D(ndim, LAUNCH_EX)
 #undef LAUNCH_EX
     return status_from_hip();
+}
+
+int cpab_expm_affine(const float* A, int n, int ndim, float scale, float* T, hipStream_t stream) {
+    if (ndim < 1 || ndim > 3) return CPAB_ERR_NDIM;
+    if (!A || !T || n < 0) return CPAB_ERR_ARG;
+    if (n == 0) return CPAB_OK;
+    return launch_expm(A, n, ndim, scale, T, stream);
+}
+
+// The single launch of k_ref_expand, else a product and the exponentials by
+// themselves (the same sums and series, so the same bits).  It saves a launch, but a
+// thread walks its row of B alone and a block's first waves do all the exponentials.
+// us, one / two launches: [3, 3], 8 thetas (7344 entries of B) 9.1 / 8.7, of which
+// the host's second launch takes more; [2, 2, 2], one theta (12960) 13.8 / 10.6;
+// [8, 8], one (390144) 29.0 / 12.4; [4, 4, 4], two (864000) 63 / 16.  By blocks:
+// [2, 2], 256 thetas 8.0 / 8.3, 512 thetas 11.6 / 8.5; [1, 1, 1], 1000 thetas
+// 32.2 / 11.8; in 1D, whose exponentials are short, [50], 512 thetas (1024 blocks)
+// 6.5 / 6.9, 1000 thetas 11.8 / 7.0.
+static bool expand_in_one(const cpab_tess_t* t, int n_theta) {
+    const long long entries = (long long)t->nC * t->ndim * (t->ndim + 1) * t->d;
+    const long long blocks = (long long)((t->nC + EXPAND_CELLS - 1) / EXPAND_CELLS) * n_theta;
+    return entries <= 1 << 13 && blocks <= (t->ndim == 1 ? 1024 : 256);
 }
 
 int cpab_ref_expand(const cpab_tess_t* t, const float* theta, int n_theta, int nstepsolver, float* As, float* trels,
@@ -3725,8 +3744,15 @@ int cpab_ref_expand(const cpab_tess_t* t, const float* theta, int n_theta, int n
     // a basis without columns (one 1D cell, zero boundary): arrays with no elements may be NULL
     if ((t->d > 0 && (!theta || !t->B)) || !As || !trels || n_theta < 0 || nstepsolver < 1) return CPAB_ERR_ARG;
     if (n_theta == 0) return CPAB_OK;
-    const dim3 g((unsigned)(t->nC + EXPAND_CELLS - 1) / EXPAND_CELLS * n_theta);
     const double scale = 1.0 / nstepsolver;
+    if (!expand_in_one(t, n_theta)) {
+        // in x-space: the scale to q-space is 1 for one cell per axis
+        cpab_tess_t x = *t;
+        x.nc[0] = x.nc[1] = x.nc[2] = 1;
+        if ((rc = launch_theta_to_A(&x, theta, n_theta, As, stream))) return rc;
+        return launch_expm(As, t->nC * n_theta, t->ndim, scale, trels, stream);
+    }
+    const dim3 g((unsigned)(t->nC + EXPAND_CELLS - 1) / EXPAND_CELLS * n_theta);
 #define LAUNCH_EX(DD) \
     hipLaunchKernelGGL((k_ref_expand<DD>), g, dim3(BLOCK), 0, stream, theta, t->B, t->d, t->nC, scale, As, trels);
     CPAB_DISPATCH_D(t->ndim, LAUNCH_EX)
