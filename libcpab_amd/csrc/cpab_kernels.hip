@@ -94,7 +94,7 @@ __host__ __device__ inline int tile_count(int ndim, int nP, int g0, int g1, int 
 
 // dL/ddata bins of a 2D tile: at most BIN_CELLS footprint cells (11-bit ids)
 constexpr int BIN_CELLS = 2048;
-constexpr int BOX_PPT = 2;  // points per thread of a tile with bins, at most
+constexpr int BOX_PPT = 3;  // points per thread of a tile with bins, at most
 
 // in-place exclusive prefix sum of v[0, n) by the whole block; v[n-1] becomes
 // the sum of the first n-1 entries
@@ -1444,7 +1444,7 @@ __device__ __forceinline__ void fused_bwd_tile(const Launch& L, const Geo& g, co
                                             nP, gk, dfd);
                 if constexpr (D == 2) {
                     if (use_box) {
-                        const int cd = r == 0 ? code[0] : code[1];
+                        const int cd = r == 0 ? code[0] : (r == 1 ? code[1] : code[2]);
                         const int pos = bins[cd & 2047] + (cd >> 11);
                         // a clamped corner pair (i1 == i0) puts its whole weight on i0
                         fd2[pos] = make_float2(i1[0] != i0[0] ? fd[0] : 0.f, i1[1] != i0[1] ? fd[1] : 0.f);
@@ -2761,7 +2761,12 @@ int bwd_tiles_per_block(int ndim, int ty, int n_theta, int tiles) {
 // cells, a 32 x 16 tile at up to ~2x magnification).  The points' bins stay in
 // registers: 512 words less and a block more per CU for the middle tessellations
 // ([6, 6], 40 x 100 x 90: 60.6 -> 47.7 us; 200 ragged problems 735 -> 654 us).
+// A batch with 768-point tiles (three points a thread: 4608 words and the cells) takes
+// bins where a tile covers up to 767 samples, as one of 48 x 16 does below 0.95x: 64
+// problems of 3 x 128 x 128 from 64 x 64 or 85 x 85 samples 146 and 148 us, 438 and 361
+// with an atomic per corner.
 constexpr int BOX_FLOATS = 5120;
+int box_floats(int ppt) { return ppt == 3 ? 5376 : BOX_FLOATS; }
 
 size_t lds_tables(int ndim, int nC) {  // nC: every cell of the facet table
     switch (ndim) {
@@ -3502,10 +3507,10 @@ size_t cpab_batch_workspace_bytes(const cpab_tess_t* t, const int* outsize, int 
 // LDS class of an instance in the batched backward: its tables and
 // per-wave accumulators next to a full dL/ddata box fit 4 (class 0), 3 (1)
 // or 2 or fewer (2) blocks per CU
-static int batch_class(const cpab_instance_t& I) {
+static int batch_class(const cpab_instance_t& I, int ppt) {
     const int nd = I.tess.ndim;
     const size_t need = align256(lds_tables(nd, I.tess.nC + I.tess.nV)) +
-                        (size_t)WAVES * I.tess.nC * nd * (nd + 1) * 4 + (size_t)BOX_FLOATS * 4 + 256;
+                        (size_t)WAVES * I.tess.nC * nd * (nd + 1) * 4 + (size_t)box_floats(ppt) * 4 + 256;
     return need <= LDS_LIMIT / 4 ? 0 : (need <= LDS_LIMIT / 3 ? 1 : 2);
 }
 
@@ -3527,7 +3532,7 @@ int cpab_batch_plan(cpab_instance_t* inst, int n_inst, int ppt, int* item_inst, 
     for (int cls = 0; cls < BATCH_CLASSES; ++cls)
         for (int i = 0; i < n_inst; ++i) {
             cpab_instance_t& I = inst[i];
-            if (batch_class(I) != cls) continue;
+            if (batch_class(I, ppt) != cls) continue;
             const int nd = I.tess.ndim;
             const int tiles =
                 tile_count(nd, I.nP, I.outsize[0], nd > 1 ? I.outsize[1] : 1, ppt, nd > 2 ? I.outsize[2] : 1);
@@ -3622,7 +3627,7 @@ int cpab_batch_bwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
     }
     for (int i = 0; i < n_inst; ++i) {
         const cpab_instance_t& I = host_inst[i];
-        const int c = batch_class(I);
+        const int c = batch_class(I, ppt);
         lo[c] = I.item0 < lo[c] ? I.item0 : lo[c];
         hi[c] = I.item0 + I.tiles > hi[c] ? I.item0 + I.tiles : hi[c];
         cnt[c] += I.tiles;
@@ -3640,7 +3645,7 @@ int cpab_batch_bwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
         int maxnd = 1;
         for (int i = 0; i < n_inst; ++i) {
             const cpab_instance_t& I = host_inst[i];
-            if (split && batch_class(I) != c) continue;
+            if (split && batch_class(I, ppt) != c) continue;
             const int nd = I.tess.ndim;
             maxnd = nd > maxnd ? nd : maxnd;
             const size_t tb = lds_tables(nd, I.tess.nC + I.tess.nV);
@@ -3652,7 +3657,7 @@ int cpab_batch_bwd(const cpab_instance_t* host_inst, const cpab_instance_t* dev_
         ltab = align256(ltab);
         const int acc_off = (int)(ltab / 4);
         // LDS box for dL/ddata when some 2D instance has a tiled grid and wants it
-        const int box_cap = (have && want_box && ltab + lacc + (size_t)BOX_FLOATS * 4 <= LDS_LIMIT) ? BOX_FLOATS : 0;
+        const int box_cap = (have && want_box && ltab + lacc + (size_t)box_floats(ppt) * 4 <= LDS_LIMIT) ? box_floats(ppt) : 0;
         const int box_off = (int)((ltab + lacc) / 4);
         const size_t lds = ltab + lacc + (size_t)box_cap * 4;
         int* q = counter + 16 * c;
