@@ -229,18 +229,23 @@ __device__ __forceinline__ float x_scale(int i, int ndim, const int (&nc)[3]) {
 }
 
 // A forward that makes A = B theta itself (theta not null): every block for its own
-// tables, a theta's first block into keep too.  Up to EXPAND_BLOCKS blocks and
-// EXPAND_PRODUCTS entries of B a launch of its own and the wait for it cost more
-// ([3, 3], one theta x 100^2 points, 5616 entries: 16.6 -> 14.5 us a pass, the kernel
-// 13.9 -> 18.0); beyond, the rows a block walks do ([4, 4], 256^2 points, 19200
-// entries: the kernel 19 -> 43 us).
+// tables, a theta's first block into keep too.  That saves a launch (2.7 us of a host
+// that calls one forward after another) and the wait for it, and costs the walk along
+// the rows of B, which grows with them and shows in full where the host does not bound
+// the calls (graph replays).  us a forward of one theta, made inside / by a launch,
+// replayed and called from Python: [20], 300 points (760 entries of B) 5.7 / 5.8 and
+// 15.3 / 18.0; [30] (1740) 6.3 / 6.3; [35] (2380) 7.0 / 6.2; [50] (4900) 8.7 / 6.6;
+// [3, 2], 32 x 32 points (3168) 12.3 / 12.3; [3, 3], 100 x 100 (7344) 14.6 / 12.8 and
+// 15.1 / 17.4; [4, 3] (13248) 19.5 / 13.0 and 19.9 / 18.6; [4, 4], 256 x 256 (23808)
+// 34 / 16.  So up to 2^13 entries, 2^11 in 1D, and for a block per CU.
 struct Expand {
     const float* theta;
     const float* B;
     int d;
     float* keep;
 };
-constexpr int EXPAND_BLOCKS = 256, EXPAND_PRODUCTS = 1 << 13;
+constexpr int EXPAND_BLOCKS = 256;
+constexpr int expand_entries(int ndim) { return ndim == 1 ? 1 << 11 : 1 << 13; }
 // entry i of A = B theta in q-space: the products in the order of k_theta_to_A, 16
 // loads in flight
 __device__ __forceinline__ float expand_entry(const Expand& ex, const float* theta, int i, const Geo& g) {
@@ -2836,7 +2841,7 @@ int expand_or_launch(const cpab_tess_t* t, const float* theta, int n_theta, long
                      Expand& ex) {
     const long long Dt = (long long)t->nC * t->ndim * (t->ndim + 1);
     ex = {nullptr, t->B, t->d, Aq};
-    if (blocks > EXPAND_BLOCKS || Dt * t->d > EXPAND_PRODUCTS) return launch_theta_to_A(t, theta, n_theta, Aq, st);
+    if (blocks > EXPAND_BLOCKS || Dt * t->d > expand_entries(t->ndim)) return launch_theta_to_A(t, theta, n_theta, Aq, st);
     ex.theta = theta;
     return CPAB_OK;
 }
