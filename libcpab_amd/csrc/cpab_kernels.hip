@@ -644,7 +644,6 @@ __device__ __forceinline__ float blend(const float (&v)[1 << D], const float (&f
     }
 }
 
-// value of channel data dp at the corners (i0, i1, fd)
 // base[i], base uniform over the wave.  NARROW: as a scalar base and a 32-bit byte
 // offset (a 64-bit address is two more instructions per access), for an instance's
 // points in 2D and 3D calls with saved state, of which there are at most LOG_POINTS.
@@ -672,6 +671,7 @@ __device__ __forceinline__ size_t per_round(int nP) {
     return (size_t)(unsigned)nP;
 }
 
+// value of channel data dp at the corners (i0, i1, fd)
 template <int D>
 __device__ __forceinline__ float interp_value(const float* __restrict__ dp, const Img& im, const int (&i0)[3],
                                               const int (&i1)[3], const float (&fd)[3]) {
@@ -1592,7 +1592,6 @@ __global__ __launch_bounds__(BLOCK, (D == 3 && HAVES) ? 4 : 1) void k_transform_
     write_partials<D>(acc, part + ((size_t)th * nbt + bt) * nC * P, nC * P);
 }
 
-// interpolation at an explicit grid [N, D, nP]; out [N, C, outsize], output order
 // The (instance n, output index t, grid index p) of this thread.  2D outputs
 // run in 16 x 16 blocks (N * ceil(g0 / 16) * ceil(g1 / 16) of them) of wave tiles
 // that are W wide along the last axis, on which the output, the upstream gradient
@@ -1630,6 +1629,7 @@ __device__ __forceinline__ bool interp_item(const Src& s, int N, int nP, int& n,
     }
 }
 
+// interpolation at an explicit grid [N, D, nP]; out [N, C, outsize], output order
 template <int D>
 __global__ __launch_bounds__(BLOCK) void k_interp_fwd(int N, int nP, Src s, Img im, float* __restrict__ out) {
     int n, t, p;
@@ -1740,10 +1740,6 @@ __global__ __launch_bounds__(RBLOCK) void k_reduce_theta(const float* __restrict
     }
 }
 
-// The same in two kernels for a few thetas: columns [c0, c1) of the row sums by
-// one block, whose result overwrites row 0 of the partials (each block owns its
-// columns and has read them all first); then 64 entries of dL/dtheta by one
-// block.  Slices give a few thetas enough blocks to fill the chip.
 // Many thetas with few rows each: grid (ceil(d / 64), ceil(n_theta / (4 TT))).  A
 // block takes 64 columns of B, 64 rows at a time through LDS, for TT thetas in each
 // of its waves, a column per lane; the rows of partials are summed as they are read.
@@ -1814,6 +1810,10 @@ __global__ __launch_bounds__(BLOCK) void k_reduce_many(const float* __restrict__
         if (t0 + w * TT + t < n_theta) gtheta[(size_t)(t0 + w * TT + t) * d + k] = acc[t];
 }
 
+// Both steps in two kernels for a few thetas: columns [c0, c1) of the row sums by
+// one block, whose result overwrites row 0 of the partials (each block owns its
+// columns and has read them all first); then 64 entries of dL/dtheta by one
+// block.  Slices give a few thetas enough blocks to fill the chip.
 template <class Rows>
 __device__ __forceinline__ void reduce_cols(float* sg, float* __restrict__ pp, int nrows, int Dt, int c0, int c1,
                                             int ndim, const int (&nc)[3], Rows rows) {
@@ -2386,7 +2386,7 @@ __global__ __launch_bounds__(BLOCK) void k_ref_backward(float* __restrict__ grad
 // the step adds h lambda [pm; 1]^T + h^2/2 mu [p; 1]^T to the cell's dL/dA, and
 // dL/dtheta = B^T dL/dA once at the end.  The work per point no longer grows
 // with d, and the [d, n_theta, D, nP] derivatives are neither written nor read:
-// [3, 3] (d = 38), 8 thetas x 10000 points x 50 steps, 860 us + 18 us of products
+// [3, 3] (d = 34), 8 thetas x 10000 points x 50 steps, 860 us + 18 us of products
 // and sums -> 67 us + 8 us of reduction, both sides bound by the FP64 chain of
 // the steps (with the FP32-cleared lookup; it took k_ref_forward from 42 to
 // 16 us).
@@ -2813,7 +2813,7 @@ int launch_theta_to_A(const cpab_tess_t* t, const float* theta, int n_theta, flo
     const int Dt = t->nC * t->ndim * (t->ndim + 1), rows = (Dt + E_ROWS - 1) / E_ROWS;
     Geo g = make_geo(t);
     // up to 2^20 products: [3, 3], one theta 2.2 us against 3.2, 128 thetas 3.3
-    // against 3.6; [4, 4], 64 thetas (1.2 million) 4.8 against 4.7
+    // against 3.6; [4, 4], 64 thetas (1.5 million) 4.8 against 4.7
     if ((long long)n_theta * Dt * t->d <= 1 << 20) {
         hipLaunchKernelGGL(k_theta_to_A_small, dim3((Dt + BLOCK - 1) / BLOCK, n_theta), dim3(BLOCK),
                            t->d * sizeof(float), st, theta, t->B, t->d, Dt, t->ndim, g.nc0, g.nc1, g.nc2, Aq);
